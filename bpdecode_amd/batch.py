@@ -149,6 +149,7 @@ def index_tensor(values: Sequence[int], device: torch.device) -> torch.Tensor:
 
 _DENSE_CODES = {torch.float32: _lib.DTYPE_F32, torch.float16: _lib.DTYPE_F16,
                 torch.bfloat16: _lib.DTYPE_BF16, torch.float64: _lib.DTYPE_F64}
+_SOFT_CODES = {k: v for k, v in _DENSE_CODES.items() if k != torch.float64}
 _TOKEN_CODES = {torch.int32: _lib.INDEX_I32, torch.int64: _lib.INDEX_I64_LOW32}
 _COMMIT_FUSED_ROWS = 4096  # the one-block commit kernel takes queued writes up to this many rows
 
@@ -427,6 +428,19 @@ class ConstraintBatch:
         """In place: ``logits += alpha * lookahead[state]`` (and mask)."""
         if self.fsa.lookahead is None:
             raise ValueError("fsa has no lookahead table; build with dense + with_lookahead")
+        code = _SOFT_CODES.get(logits.dtype)
+        la = self.fsa.lookahead
+        if (self._fast and code is not None and self._fast_logits(logits, len(seq_ids))
+                and la.dtype == torch.float32 and la.is_contiguous() and la.shape[1] == self._V):
+            B = len(seq_ids)
+            slots, pend, n = self._slots_fused(seq_ids, True)
+            check(lib().bpd_soft_apply_queued(
+                logits.data_ptr(), code, B, self._V, logits.stride(0) if B > 1 else self._V, la.data_ptr(),
+                int(la.shape[0]), self._pool_ptr, slots, pend, n, float(alpha), None,
+                _lib.stream_of(self.device)))
+            if n:
+                self._launched()
+            return logits
         slots = self._slots(seq_ids)
         ops.soft_apply_(logits, self.fsa.lookahead, self._state, slots, alpha)
         return logits

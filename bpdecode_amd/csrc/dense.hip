@@ -23,50 +23,20 @@
 #include <algorithm>
 
 #include "bpd_common.hpp"
+#include "rows.hpp"
 
 namespace bpd {
 namespace {
 
-constexpr int kXcds = 8;
 constexpr int kFillWaves = 4;                 // waves per block: one row, 4 chunks
 constexpr int kFillThreads = 64 * kFillWaves;
 constexpr int kFillGroups = 32;               // 64-column groups per chunk (one wave)
 constexpr int64_t kChunkCols = int64_t(kFillGroups) * 64;
 
-// Block index -> logical block, numbered so that consecutive logical blocks
-// run on one XCD (workgroups are dealt round-robin to the 8 XCDs).
-// gridDim.x is a multiple of kXcds.
-__device__ __forceinline__ uint32_t logical_block() {
-  const uint32_t nb = gridDim.x;
-  const uint32_t hw = blockIdx.x;
-  return (hw % kXcds) * (nb / kXcds) + hw / kXcds;
-}
-
 template <int E> struct Elem;
 template <> struct Elem<2> { using T = uint16_t; };
 template <> struct Elem<4> { using T = uint32_t; };
 template <> struct Elem<8> { using T = uint64_t; };
-
-// Wave-uniform state of row r: the pool entry at its slot, or the value of a
-// queued write to that slot (`pending` = num_pending slots, then as many
-// values; slots are distinct).
-__device__ __forceinline__ int32_t wave_row_state(const int32_t* states, const int64_t* slots,
-                                                  const int64_t* pending, int32_t num_pending,
-                                                  uint32_t r, int lane) {
-  const int64_t slot = slots ? slots[r] : int64_t(r);
-  int32_t s = __builtin_amdgcn_readfirstlane(states[slot]);
-  for (int32_t base = 0; base < num_pending; base += 64) {
-    const int32_t i = base + lane;
-    const bool hit = i < num_pending && pending[i] == slot;
-    const uint64_t m = __ballot(hit);
-    if (m) {
-      const int src = __builtin_ctzll(m);
-      const int32_t v = hit ? int32_t(pending[num_pending + i]) : 0;
-      s = __builtin_amdgcn_readlane(v, src);
-    }
-  }
-  return s;
-}
 
 // Dense mask, write-only.  A wave owns one row and a chunk of 2048 columns
 // (32 groups of 64); for each group the 64 verdicts of its columns decide
@@ -370,13 +340,9 @@ int launch_fill(void* logits, int dtype, int64_t rows, int64_t vocab, int64_t ld
   BPD_REQUIRE(rows >= 0 && vocab >= 0 && ld >= vocab, "bad logits shape rows=%lld vocab=%lld ld=%lld",
               (long long)rows, (long long)vocab, (long long)ld);
   BPD_REQUIRE(num_states > 0, "empty grammar table");
-  BPD_REQUIRE(num_pending >= 0 && num_pending <= BPD_MAX_FUSED_PENDING,
-              "at most %d queued pool writes per launch (got %lld)", BPD_MAX_FUSED_PENDING,
-              (long long)num_pending);
-  BPD_REQUIRE(num_pending == 0 || (pending && slots), "queued writes need a slot map");
+  if (int rc = check_pending(pending, num_pending, slots, rows)) return rc;
   uint64_t fill = 0;
   if (int rc = fill_bits64(dtype, neg_inf, &fill)) return rc;
-  BPD_REQUIRE(rows > 0 || num_pending == 0, "queued writes need at least one row");
   if (rows == 0) return BPD_OK;
   BPD_REQUIRE(logits && table && states, "null pointer argument");
   BPD_REQUIRE(reinterpret_cast<uintptr_t>(logits) % E == 0, "logits are not aligned to their element size");

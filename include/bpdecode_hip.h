@@ -446,6 +446,11 @@ int bpd_soft_build_lookahead(const int32_t* tok_next, int32_t num_states, int64_
 int bpd_soft_apply(void* logits, int dtype, int64_t rows, int64_t vocab, int64_t ld,
                    const float* lookahead, int32_t num_states, const int32_t* states,
                    const int64_t* slots, float alpha, int32_t* err, void* stream);
+/* The same with queued pool writes (`pending`, as bpd_dense_apply_mask). */
+int bpd_soft_apply_queued(void* logits, int dtype, int64_t rows, int64_t vocab, int64_t ld,
+                          const float* lookahead, int32_t num_states, int32_t* states,
+                          const int64_t* slots, const int64_t* pending, int64_t num_pending,
+                          float alpha, int32_t* err, void* stream);
 
 int bpd_host_soft_build_lookahead(const int32_t* tok_next, int32_t num_states, int64_t vocab,
                                   const uint8_t* accept, const uint8_t* live, int32_t eos_id,

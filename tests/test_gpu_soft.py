@@ -69,6 +69,61 @@ def test_apply_soft(dev, dtype, alpha):
         assert np.all(np.abs(g[fin] - want[fin]) <= 1e-2 * np.abs(want[fin]) + 1e-2)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,vocab,pad", [(1, 1, 0), (3, 7, 0), (5, 4095, 1), (2, 2049, 3), (9, 8192, 0),
+                                            (300, 8193, 5), (300, 16384, 0), (67, 40_001, 8)])
+def test_apply_soft_row_shapes(dev, dtype, rows, vocab, pad):
+    """Rows of any stride, start alignment and length around the block's
+    4096- and 8192-element spans, on the one- and the two-group grid: the
+    same words as the library's host entry point.  float16: the device fuses
+    the multiply, the add and the conversion (one rounding, where the host
+    rounds to float first), so the words are those of the float64 value."""
+    g = torch.Generator().manual_seed(rows * 31 + vocab)
+    S = 5
+    la = torch.randn(S, vocab, generator=g) * 4
+    la[torch.rand(S, vocab, generator=g) < 0.8] = -torch.inf
+    st = torch.randint(-2, S + 1, (rows,), generator=g, dtype=torch.int32)  # S: out of range, masked
+    wide = (torch.randn(rows, vocab + pad, generator=g) * 3).to(dtype)
+    got = wide.to(dev)
+    off = min(1, pad)
+    ops.soft_apply_(got[:, off:off + vocab], la.to(dev), st.to(dev), alpha=0.75)
+    want = wide.clone()
+    ops.soft_apply_(want[:, off:off + vocab], la, st.where(st < S, -1), alpha=0.75)
+    if dtype == torch.float16:
+        bias = la.double()[st.clamp(0, S - 1).long()].numpy()
+        v = wide[:, off:off + vocab].double().numpy() + 0.75 * bias
+        keep = np.isfinite(want[:, off:off + vocab].float().numpy())
+        want[:, off:off + vocab] = torch.from_numpy(np.where(keep, v, -np.inf).astype(np.float16))
+    assert torch.equal(got.cpu().view(torch.uint8), want.view(torch.uint8))
+
+
+def test_apply_soft_carries_queued_writes(dev):
+    """add / evict / reset before apply_soft: the mask launch applies them,
+    and the pool holds them for the next commit."""
+    fsa = FsaTensors.build("a[012]+|b0", TOY_VOCAB).with_lookahead(3).to(dev)
+    batch = ConstraintBatch(fsa, capacity=8, device=dev)
+    for i in range(6):
+        batch.add(i)
+    tok = TOY_VOCAB.token_bytes.index(b"a")
+    batch.commit(list(range(6)), torch.full((6,), tok, dtype=torch.int64, device=dev))
+    batch.evict(1)
+    batch.evict(4)
+    batch.add(7)
+    batch.reset(2)
+    ids = [7, 0, 2, 3, 5]
+    after = int(fsa.tok_next[fsa.start, tok])
+    states = [fsa.start, after, fsa.start, after, after]
+    x = torch.randn(5, TOY_VOCAB.size)
+    got = x.to(dev)
+    batch.apply_soft(ids, got, 0.5)
+    want = x.clone()
+    ops.apply_soft_(want, fsa.to("cpu"), torch.tensor(states, dtype=torch.int32), 0.5)
+    assert torch.equal(got.cpu(), want)
+    assert [batch.state_of(i) for i in ids] == states
+    nxt = batch.commit(ids, torch.full((5,), tok, dtype=torch.int64, device=dev)).tolist()
+    assert nxt == [int(fsa.tok_next[s, tok]) if s >= 0 else -1 for s in states]
+
+
 # ------------------------------------------------------- prior-weighted --
 # The toy vocabulary with three more tokens: V = 20, a multiple of 4, so the
 # vectorised kernels apply (V = 17 takes the scalar ones).
