@@ -24,6 +24,7 @@
 
 #include "bpd_common.hpp"
 #include "rows.hpp"
+#include "walk.hpp"
 
 namespace bpd {
 namespace {
@@ -104,6 +105,7 @@ __global__ __launch_bounds__(kFillThreads) void dense_fill_kernel(
 // torch advanced indexing does.  False when the id is out of range.
 __device__ __forceinline__ int32_t row_state(const int32_t* __restrict__ states,
                                              const int64_t* __restrict__ slots, int64_t r) {
+  if (!states) return int32_t(r);  // every state's row
   return states[slots ? slots[r] : r];
 }
 
@@ -226,29 +228,120 @@ __global__ void dense_scatter_kernel(int32_t* __restrict__ states, const int64_t
   states[slots ? slots[b] : b] = next[b];
 }
 
-// One thread per token; each wave64 packs its 64 verdicts with a ballot into
-// two consecutive uint32 words (LSB-first), written by lane 0.
-__global__ __launch_bounds__(256) void dense_bits_kernel(
+// Packed allow bits of the rows' table rows, grid (ceil(vocab / 4096), rows).
+// Bound by the read of the int32 rows, so each lane has four 16-byte loads in
+// flight (a row starts at any 4-byte boundary).  A lane's four verdicts are a
+// nibble of its word; the eight lanes of a word are combined by DPP
+// exchanges, and lane u of the eight writes the word of load u (LSB-first).
+// 71 rows of V = 151,936: 22.4 us with one load per thread, 8.2 now.
+constexpr int kBitsThreads = 256;
+constexpr int kBitsLoads = 4;
+constexpr int64_t kBitsTokens = int64_t(kBitsThreads) * 4 * kBitsLoads;
+typedef int32_t I4u __attribute__((ext_vector_type(4), aligned(4)));
+
+template <int Ctrl>
+__device__ __forceinline__ uint32_t or_lane(uint32_t v) {
+  return v | uint32_t(__builtin_amdgcn_update_dpp(0, int(v), Ctrl, 0xF, 0xF, false));
+}
+
+__global__ __launch_bounds__(kBitsThreads) void dense_bits_kernel(
     const int32_t* __restrict__ tok_next, int32_t num_states, int64_t vocab,
     const int32_t* __restrict__ states, const int64_t* __restrict__ slots, int64_t rows,
     uint32_t* __restrict__ bits, int64_t words, int32_t* __restrict__ err) {
   const int64_t r = blockIdx.y;
-  if (r >= rows) return;
-  const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  const int sub = threadIdx.x & 7;
+  const int64_t t0 = int64_t(blockIdx.x) * kBitsTokens + threadIdx.x * 4;
   const int32_t s = row_state(states, slots, r);
   const bool live_row = s >= 0 && s < num_states;
-  if (s >= num_states && err && t == 0) atomicOr(err, BPD_FLAG_STATE_RANGE);
-  const bool allowed = live_row && t < vocab && tok_next[int64_t(s) * vocab + t] != -1;
-  const uint64_t m = __ballot(allowed);
-  if ((threadIdx.x & 63) == 0) {
-    const int64_t w0 = t >> 5;
-    if (w0 < words) bits[r * words + w0] = uint32_t(m);
-    if (w0 + 1 < words) bits[r * words + w0 + 1] = uint32_t(m >> 32);
+  if (s >= num_states && err && t0 == 0) atomicOr(err, BPD_FLAG_STATE_RANGE);
+  const int32_t* row = tok_next + (live_row ? int64_t(s) * vocab : 0);
+  I4u v[kBitsLoads];
+#pragma unroll
+  for (int u = 0; u < kBitsLoads; ++u) {
+    const int64_t t = t0 + int64_t(u) * kBitsThreads * 4;
+    v[u] = I4u{-1, -1, -1, -1};
+    if (live_row && t + 4 <= vocab) {
+      v[u] = *reinterpret_cast<const I4u*>(row + t);
+    } else if (live_row) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (t + q < vocab) v[u][q] = row[t + q];
+    }
+  }
+  uint32_t mine = 0;
+#pragma unroll
+  for (int u = 0; u < kBitsLoads; ++u) {
+    uint32_t w = 0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) w |= v[u][q] != -1 ? 1u << q : 0u;
+    w <<= 4 * sub;
+    w = or_lane<0xB1>(w);   // lane ^ 1
+    w = or_lane<0x4E>(w);   // lane ^ 2
+    w = or_lane<0x141>(w);  // the other four of the eight
+    if (sub == u) mine = w;
+  }
+  const int64_t at = (t0 - 4 * sub) / 32 + int64_t(sub) * (kBitsThreads / 8);
+  if (sub < kBitsLoads && at < words) bits[r * words + at] = mine;
+}
+
+// tok_next builder over the staged walk table (walk.hpp), grid (tokens, rows /
+// rows_per_block): a thread holds one token's symbols and walks them from the
+// block's rows, four at a time; each row's results go out as one coalesced
+// store per wave.  Bound by the walk's instructions and LDS reads.  71 states
+// x 151,936 tokens: 68.2 us with one thread per (row, token) reading symbols
+// and table from memory, 21.1 us now (19 without the stores).
+__global__ __launch_bounds__(1024) void build_walk_kernel(
+    const int32_t* __restrict__ trans, int32_t S, int32_t M, int32_t dead,
+    const uint8_t* __restrict__ accept, const uint8_t* __restrict__ live,
+    const int32_t* __restrict__ offsets, const uint8_t* __restrict__ syms, int64_t vocab,
+    int32_t eos_id, const int32_t* __restrict__ row_states, int32_t num_rows, int32_t rows_per_block,
+    int32_t* __restrict__ out) {
+  extern __shared__ __align__(16) uint16_t walk_tab[];
+  const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  const bool on = t < vocab;
+  int32_t b = 0, e = 0;
+  if (on && t != eos_id) {
+    b = offsets[t];
+    e = offsets[t + 1];
+  }
+  const WalkToken tok = load_walk_token(syms, b, e - b, offsets[vocab], M);
+  stage_walk_table(walk_tab, trans, S, M, dead, live);
+  __syncthreads();
+  const uint32_t W = uint32_t(M) + 3, fail = uint32_t(S) * W;
+  const int32_t r0 = int32_t(blockIdx.y) * rows_per_block;
+  const int32_t r1 = r0 + rows_per_block < num_rows ? r0 + rows_per_block : num_rows;
+  const bool has_eos = __any(t == eos_id) != 0;  // only this wave needs the accepting flags
+  int32_t* o = out + int64_t(r0) * vocab + t;
+  for (int32_t r = r0; r < r1; r += kWalkRows) {
+    uint32_t cur[kWalkRows];
+    int32_t st[kWalkRows];
+#pragma unroll
+    for (int q = 0; q < kWalkRows; ++q) {
+      st[q] = r + q;
+      if (row_states) st[q] = r + q < r1 ? row_states[r + q] : -1;
+      cur[q] = uint32_t(st[q]) < uint32_t(S) ? uint32_t(st[q]) * W : fail;
+    }
+    walk_rows(walk_tab, M, fail, tok, cur);
+    int32_t res[kWalkRows];
+#pragma unroll
+    for (int q = 0; q < kWalkRows; ++q) {
+      const uint32_t v = walk_tab[cur[q] + M + 2];
+      res[q] = v == kWalkNone ? -1 : int32_t(v);
+    }
+    if (has_eos) {
+#pragma unroll
+      for (int q = 0; q < kWalkRows; ++q)
+        if (t == eos_id) res[q] = uint32_t(st[q]) < uint32_t(S) && accept[st[q]] ? st[q] : -1;
+    }
+#pragma unroll
+    for (int q = 0; q < kWalkRows; ++q)
+      if (on && r + q < r1) o[int64_t(q) * vocab] = res[q];
+    o += int64_t(kWalkRows) * vocab;
   }
 }
 
-// tok_next builder: one thread per (row, token); walks the token's symbol
-// classes through the dense symbol-class table.
+// The builder for tables too large to stage: one thread per (row, token),
+// symbols and table read through the caches.
 __global__ __launch_bounds__(256) void build_tok_next_kernel(
     const int32_t* __restrict__ trans, int32_t num_states, int32_t num_symbols, int32_t dead,
     const uint8_t* __restrict__ accept, const uint8_t* __restrict__ live,
@@ -283,6 +376,16 @@ __global__ __launch_bounds__(256) void build_tok_next_kernel(
     res = (ok && live[cur]) ? cur : -1;
   }
   out[int64_t(r) * vocab + t] = res;
+}
+
+// int32 symbol ids to bytes, and *bad |= 1 where one lies outside [0, 255].
+__global__ __launch_bounds__(256) void narrow_symbols_kernel(const int32_t* __restrict__ sym, int64_t n,
+                                                             uint8_t* __restrict__ out,
+                                                             int32_t* __restrict__ bad) {
+  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  const int32_t v = i < n ? sym[i] : 0;
+  if (i < n) out[i] = uint8_t(v);
+  if (__any(v < 0 || v > 255) && (threadIdx.x & 63) == 0) atomicOr(bad, 1);
 }
 
 // Reachability (the live set of a DFA): live[s] = 1 iff an accepting state
@@ -442,10 +545,28 @@ extern "C" int bpd_dense_compute_mask(const int32_t* tok_next, int32_t num_state
   if (rows == 0 || words == 0) return BPD_OK;
   BPD_REQUIRE(rows < 65536, "at most 65535 rows");
   BPD_REQUIRE(tok_next && states && bits, "null pointer argument");
-  const dim3 grid = dim3(unsigned((vocab + 255) / 256), unsigned(rows));
-  dense_bits_kernel<<<grid, 256, 0, as_stream(stream)>>>(tok_next, num_states, vocab, states,
+  const dim3 grid = dim3(unsigned((vocab + kBitsTokens - 1) / kBitsTokens), unsigned(rows));
+  dense_bits_kernel<<<grid, kBitsThreads, 0, as_stream(stream)>>>(tok_next, num_states, vocab, states,
                                                           slots, rows, bits, words, err);
   BPD_LAUNCHED();
+  return BPD_OK;
+}
+
+extern "C" int bpd_dense_table_bits(const int32_t* tok_next, int32_t num_states, int64_t vocab, uint32_t* bits,
+                                    void* stream) {
+  BPD_REQUIRE(num_states > 0 && vocab >= 0, "bad shape");
+  const int64_t words = (vocab + 31) / 32;
+  if (words == 0) return BPD_OK;
+  BPD_REQUIRE(tok_next && bits, "null pointer argument");
+  hipStream_t st = as_stream(stream);
+  // the grid's second dimension takes 65535 rows
+  for (int32_t s0 = 0; s0 < num_states; s0 += 65535) {
+    const int32_t n = num_states - s0 < 65535 ? num_states - s0 : 65535;
+    const dim3 grid = dim3(unsigned((vocab + kBitsTokens - 1) / kBitsTokens), unsigned(n));
+    dense_bits_kernel<<<grid, kBitsThreads, 0, st>>>(tok_next + int64_t(s0) * vocab, n, vocab, nullptr, nullptr, n,
+                                            bits + int64_t(s0) * words, words, nullptr);
+    BPD_LAUNCHED();
+  }
   return BPD_OK;
 }
 
@@ -458,10 +579,39 @@ extern "C" int bpd_build_tok_next(const int32_t* trans, int32_t num_states, int3
   BPD_REQUIRE(dead >= 0 && dead < num_states, "dead state out of range");
   if (vocab == 0 || num_rows == 0) return BPD_OK;
   BPD_REQUIRE(num_rows < 65536, "at most 65535 table rows per launch");
+  // A staged table up to 16 KB leaves a CU its four blocks of 512 threads
+  // (71 states: 21.6 us; 256 threads 23.6, 1024 22.9); a larger one is shared
+  // by a block of 1024 threads (two on a CU).
+  if (walk_table_fits(num_states, num_symbols, 79 * 1024)) {
+    const size_t lds = walk_table_bytes(num_states, num_symbols);
+    const int threads = lds <= 16 * 1024 ? 512 : 1024;
+    const int64_t tiles = (vocab + threads - 1) / threads;
+    // as many waves as the chip holds (8192), so that each staging serves as
+    // many rows as that allows (half as many: 23.9 us, twice as many: 26.5)
+    int64_t split = (8192 * 64 + tiles * threads - 1) / (tiles * threads);
+    const int64_t groups = (num_rows + kWalkRows - 1) / kWalkRows;
+    if (split > groups) split = groups;
+    const int64_t per = (groups + split - 1) / split * kWalkRows;
+    const dim3 grid = dim3(unsigned(tiles), unsigned((num_rows + per - 1) / per));
+    build_walk_kernel<<<grid, threads, lds, as_stream(stream)>>>(
+        trans, num_states, num_symbols, dead, accept, live, tok_offsets, tok_symbols, vocab, eos_id,
+        row_states, num_rows, int32_t(per), out);
+    BPD_LAUNCHED();
+    return BPD_OK;
+  }
   const dim3 grid = dim3(unsigned((vocab + 255) / 256), unsigned(num_rows));
   build_tok_next_kernel<<<grid, 256, 0, as_stream(stream)>>>(
       trans, num_states, num_symbols, dead, accept, live, tok_offsets, tok_symbols, vocab,
       eos_id, row_states, num_rows, out);
+  BPD_LAUNCHED();
+  return BPD_OK;
+}
+
+extern "C" int bpd_narrow_symbols(const int32_t* symbols, int64_t n, uint8_t* out, int32_t* bad, void* stream) {
+  BPD_REQUIRE(n >= 0 && n < (int64_t(1) << 31), "bad symbol count");
+  if (n == 0) return BPD_OK;
+  BPD_REQUIRE(symbols && out && bad, "null pointer argument");
+  narrow_symbols_kernel<<<unsigned((n + 255) / 256), 256, 0, as_stream(stream)>>>(symbols, n, out, bad);
   BPD_LAUNCHED();
   return BPD_OK;
 }

@@ -256,13 +256,18 @@ class FsaTensors:
         the walking kernel (every state's row; no [states, vocab] int32
         table).  A host bundle without tok_next is densified first."""
         if self.allow_bits is None:
-            st = torch.arange(self.num_states, dtype=torch.int32, device=self.device)
-            if self.tok_next is None and self.device.type == "cuda":
+            on_dev = self.device.type == "cuda"
+            if self.tok_next is None and on_dev:
+                st = torch.arange(self.num_states, dtype=torch.int32, device=self.device)
                 self.allow_bits = fsa_compute_mask(self, st)
             else:
                 base = self.densify()
                 self.tok_next = base.tok_next
-                self.allow_bits = dense_compute_mask(base.tok_next, st)
+                if on_dev and base.tok_next.device == self.device:
+                    self.allow_bits = dense_table_bits(base.tok_next)
+                else:
+                    st = torch.arange(self.num_states, dtype=torch.int32, device=self.device)
+                    self.allow_bits = dense_compute_mask(base.tok_next, st)
         return self.allow_bits
 
     def allow_bits_or_none(self) -> torch.Tensor | None:
@@ -349,6 +354,16 @@ def _unit_stride_rows(logits: torch.Tensor) -> tuple[torch.Tensor, bool]:
 
 def _symbols_u8(fsa: FsaTensors) -> torch.Tensor:
     sym = fsa.symbols
+    if sym.device.type == "cuda" and sym.dtype == torch.int32 and sym.numel():
+        # one pass narrows and checks; one read-back instead of a minimum's
+        # and a maximum's
+        sym = sym.contiguous()
+        out = torch.empty(sym.numel(), dtype=torch.uint8, device=sym.device)
+        bad = torch.zeros(1, dtype=torch.int32, device=sym.device)
+        check(lib().bpd_narrow_symbols(ptr(sym), sym.numel(), ptr(out), ptr(bad), _lib.stream_of(sym.device)))
+        if int(bad):
+            raise RuntimeError("symbol-class ids must lie in [0, 255]")
+        return out
     if sym.numel() and (int(sym.min()) < 0 or int(sym.max()) > 255):
         raise RuntimeError("symbol-class ids must lie in [0, 255]")
     return sym.to(torch.uint8).contiguous() if sym.numel() else torch.zeros(1, dtype=torch.uint8, device=sym.device)
@@ -566,6 +581,15 @@ def dense_compute_mask(tok_next, states, slots=None, err=None):
                                            _lib.stream_of(dev)))
     else:
         check(lib().bpd_host_dense_compute_mask(ptr(tn), S, V, ptr(st), ptr(sl), B, ptr(out)))
+    return out
+
+
+def dense_table_bits(tok_next: torch.Tensor) -> torch.Tensor:
+    """The packed allow bits of every row of a device table."""
+    tn = _i32(tok_next)
+    S, V = tn.shape
+    out = torch.empty((S, (V + 31) // 32), dtype=torch.int32, device=tn.device)
+    check(lib().bpd_dense_table_bits(ptr(tn), S, V, ptr(out), _lib.stream_of(tn.device)))
     return out
 
 

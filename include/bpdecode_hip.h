@@ -135,6 +135,16 @@ int bpd_build_tok_next(const int32_t* trans, int32_t num_states, int32_t num_sym
                        int64_t vocab, int32_t eos_id, const int32_t* row_states,
                        int32_t num_rows, int32_t* out, void* stream);
 
+/* bpd_dense_table_bits: the packed allow bits [num_states, ceil(vocab/32)] of
+ * every row of tok_next (bpd_dense_compute_mask over all states). */
+int bpd_dense_table_bits(const int32_t* tok_next, int32_t num_states, int64_t vocab, uint32_t* bits,
+                         void* stream);
+
+/* bpd_narrow_symbols: the symbol classes of bpd_build_tok_next from int32
+ * ids; *bad (zeroed by the caller, device memory) becomes non-zero when an id
+ * lies outside [0, 255]. */
+int bpd_narrow_symbols(const int32_t* symbols, int64_t n, uint8_t* out, int32_t* bad, void* stream);
+
 /* bpd_build_reachability: live[s] = 1 iff an accepting state is reachable
  * from s through trans ([num_states * num_symbols], targets outside
  * [0, num_states) ignored); device pointers, at most 65536 states.  The

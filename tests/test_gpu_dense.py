@@ -414,3 +414,57 @@ def test_device_built_bundles_equal_host_built(dev, serving_vocab):
     d2 = FsaTensors.build(dfa, serving_vocab, device=dev)
     assert h2.tok_next is None and d2.tok_next is None
     assert torch.equal(d2.live.cpu(), h2.live) and torch.equal(d2.trans.cpu(), h2.trans)
+
+
+def random_bundle(S: int, M: int, V: int, seed: int, max_len: int = 40) -> FsaTensors:
+    """A bundle of arbitrary tables: targets outside the table, symbol ids at
+    and above M, empty tokens, tokens longer than 16 symbols, EOS inside the
+    vocabulary and a live set that need not be closed (``dead`` live in half
+    of them)."""
+    g = np.random.default_rng(seed)
+    trans = g.integers(-2, S + 2, size=S * M).astype(np.int32)
+    keep = g.random(S * M) < 0.9
+    trans[keep] = g.integers(0, S, size=int(keep.sum()))
+    dead = int(g.integers(0, S))
+    live = (g.random(S) < 0.7).astype(np.uint8)
+    live[dead] = seed % 2
+    lens = g.integers(0, max_len + 1, size=V)
+    lens[g.random(V) < 0.7] //= 8
+    off = np.zeros(V + 1, dtype=np.int32)
+    np.cumsum(lens, out=off[1:])
+    sym = g.integers(0, M, size=int(off[-1]))
+    bad = g.random(sym.size) < 0.01
+    sym[bad] = np.minimum(M + g.integers(0, 4, size=int(bad.sum())), 255)
+    t = torch.from_numpy
+    return FsaTensors(trans=t(trans), accept=t((g.random(S) < 0.3).astype(np.uint8)), live=t(live), num_symbols=M,
+                      dead=dead, offsets=t(off), symbols=t(sym.astype(np.int32)), eos_id=int(g.integers(0, V)))
+
+
+@pytest.mark.parametrize("S,M,V", [(1, 1, 1), (1, 1, 700), (5, 3, 63), (71, 30, 5001), (72, 110, 513), (73, 110, 1025),
+                                   (300, 24, 1023), (820, 45, 2049), (900, 60, 700), (40, 253, 511), (40, 254, 511)])
+@pytest.mark.parametrize("seed", [1, 2])
+def test_table_builder_shapes(dev, S, M, V, seed):
+    """The staged walk at its limits (tables of 512- and 1024-thread blocks,
+    the largest staged one, one state or symbol more than fits), the rows
+    argument with states outside the table, and the allow bits: the words of
+    the library's host builder."""
+    _log(f"case table builder S={S} M={M} V={V} seed={seed}")
+    host = random_bundle(S, M, V, seed)
+    want = ops.build_token_transitions(host)
+    fd = host.to(dev)
+    got = ops.build_token_transitions(fd)
+    assert torch.equal(got.cpu(), want)
+    rows = torch.tensor([S - 1, 0, -1, S, S + 9, S // 2, 0], dtype=torch.int32)
+    sub = ops.build_token_transitions(fd, rows=rows.to(dev)).cpu()
+    for i, r in enumerate(rows.tolist()):
+        assert torch.equal(sub[i], want[r] if 0 <= r < S else torch.full((V,), -1, dtype=torch.int32)), (i, r)
+    bits = fd.densify().ensure_allow_bits().cpu().numpy().view(np.uint32)
+    assert np.array_equal(bits, OD.compute_mask_bits(want.numpy(), np.arange(S)))
+
+
+def test_table_builder_refuses_wide_symbols(dev):
+    for bad in (256, -1):
+        fsa = random_bundle(4, 3, 50, 1)
+        fsa.symbols[7] = bad
+        with pytest.raises(RuntimeError, match="symbol-class ids"):
+            ops.build_token_transitions(fsa.to(dev))
