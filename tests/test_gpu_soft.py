@@ -8,6 +8,7 @@ import pytest
 import torch
 
 from bpdecode_amd import ops, synth
+from bpdecode_amd._lib import check, lib, stream_of
 from bpdecode_amd.batch import ConstraintBatch
 from bpdecode_amd.ops import FsaTensors
 from bpdecode_amd.tokenizer import Vocabulary
@@ -42,6 +43,30 @@ def test_build_lookahead_email_serving(dev):
     want = OS.build_lookahead(fsa.tok_next.cpu().numpy(), fsa.live.cpu().numpy(),
                               fsa.accept.cpu().numpy(), fsa.eos_id, 4)
     assert close(la, want)
+
+
+@pytest.mark.parametrize("S,V", [(1, 1), (2, 4097), (63, 4095), (65, 1000), (512, 4097), (513, 4097)])
+@pytest.mark.parametrize("k", [1, 2, 4])
+def test_build_lookahead_state_counts(dev, S, V, k):
+    """Rounds from (state, next) counts up to 512 states, from the table
+    above; chunk edges, entries outside the table, states without tokens."""
+    g = np.random.default_rng(S + k)
+    tn = g.integers(0, S, size=(S, V)).astype(np.int32)
+    tn[g.random((S, V)) < 0.9] = -1
+    tn[g.random((S, V)) < 0.01] = S + 3  # outside the table: rejected
+    tn[S // 2] = -1
+    live, accept = (g.random(S) < 0.8).astype(np.uint8), (g.random(S) < 0.3).astype(np.uint8)
+    eos = V - 1
+    out = torch.empty((S, V), dtype=torch.float32, device=dev)
+    need = int(lib().bpd_soft_workspace_bytes(0, S, k))
+    ws = torch.empty(need, dtype=torch.uint8, device=dev)
+    d = [torch.from_numpy(a).to(dev) for a in (tn, accept, live)]
+    want = OS.build_lookahead(np.where(tn < S, tn, -1), live, accept, eos, k)
+    for size in (need, 8 * S):  # the two vectors alone: the table-reading rounds
+        out.fill_(7.0)
+        check(lib().bpd_soft_build_lookahead(d[0].data_ptr(), S, V, d[1].data_ptr(), d[2].data_ptr(), eos, k,
+                                             out.data_ptr(), ws.data_ptr(), size, stream_of(dev)))
+        assert close(out.cpu().double().numpy(), want)
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
