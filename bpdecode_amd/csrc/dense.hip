@@ -305,7 +305,7 @@ __global__ __launch_bounds__(1024) void build_walk_kernel(
     e = offsets[t + 1];
   }
   const WalkToken tok = load_walk_token(syms, b, e - b, offsets[vocab], M);
-  stage_walk_table(walk_tab, trans, S, M, dead, live);
+  stage_walk_table<true>(walk_tab, trans, S, M, dead, live);
   __syncthreads();
   const uint32_t W = uint32_t(M) + 3, fail = uint32_t(S) * W;
   const int32_t r0 = int32_t(blockIdx.y) * rows_per_block;

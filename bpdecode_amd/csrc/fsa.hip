@@ -2,17 +2,18 @@
 // on the fly (no [states, vocab] tok_next table): the device form of the
 // reference's non-dense operators for grammars too large to densify.
 //
-// One block covers kFsaRows rows and kFsaThreads * kFsaTok tokens.  The
-// transition table and the live flags are staged in LDS when they fit; each
-// token's first 16 symbol classes are loaded once into registers and walked
-// from every row state of the block.  Verdicts become fill stores (logits)
-// or wave64 ballots (packed bits).
+// A token's first 16 symbol classes are loaded once into registers and walked
+// from every row state of the block.  Verdicts become fill stores (logits) or
+// wave64 ballots (packed bits).  Tables that fit are walked in the absorbing
+// LDS form of walk.hpp (fsa_walk_kernel), larger ones through L2
+// (fsa_mask_kernel, kFsaRows rows and kFsaThreads * kFsaTok tokens a block).
 
 #include <atomic>
 #include <cstdlib>
 #include <cstring>
 
 #include "bpd_common.hpp"
+#include "walk.hpp"
 
 namespace bpd {
 namespace {
@@ -20,10 +21,8 @@ namespace {
 constexpr int kFsaThreads = 256;
 constexpr int kFsaTok = 4;     // tokens per thread, kFsaThreads apart
 constexpr int kFsaRows = 8;    // rows per block
-// The table is staged in LDS only when small: every block stages its own
-// copy, which for large tables costs more than reading them through L2
-// (a 75 KB uint16 copy per block measured 3x slower than L2 reads).
-constexpr size_t kFsaMaxLds = 16 * 1024;
+constexpr size_t kWalkMaxLds = 79 * 1024;  // staged walk tables: two blocks on a CU
+constexpr int kWalkBlockRows = 256;        // most rows of one block
 constexpr int32_t kNoRow = INT32_MIN;
 constexpr int kFsaAdvThreads = 256;
 // The fused commit (one block: gather, queued pool writes, walk, scatter)
@@ -87,26 +86,95 @@ __device__ __forceinline__ bool walk_token(const FsaView& f, const int32_t* __re
   return lv[cur] != 0;
 }
 
-// Mask (Bits = false: fill the rejected logits, element size E) or packed
-// allow bits (Bits = true).  grid (ceil(V / (kFsaThreads kFsaTok)), ceil(rows / kFsaRows)).
-template <int E, bool Bits, bool InLds>
+// Mask over the staged walk table: a thread holds one token and walks it from
+// the block's rows (row_lo + rows_per_block of them), four at a time.  Bound
+// by the walk's instructions and LDS reads.  The row states are read once per
+// block, into LDS, beside the table.
+// 826 states, V = 151,936, packed bits: 256 rows 150 us through L2, 67 here;
+// 826 rows 412 and 163; 71 states, 256 rows: 230 and 52.
+template <int E, bool Bits>
+__global__ __launch_bounds__(1024) void fsa_walk_kernel(
+    FsaView f, const int32_t* __restrict__ states, const int64_t* __restrict__ slots, int64_t rows,
+    int32_t rows_per_block, uint8_t* __restrict__ logits, int64_t ld_bytes, uint32_t fill,
+    uint32_t* __restrict__ bits, int64_t words, int32_t* __restrict__ err) {
+  extern __shared__ __align__(16) uint16_t walk_tab[];
+  __shared__ int32_t rs[kWalkBlockRows];
+  const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  const bool on = t < f.V;
+  const bool is_eos = t == f.eos;
+  const int64_t r0 = int64_t(blockIdx.y) * rows_per_block;
+  const int32_t n = int32_t(rows - r0 < rows_per_block ? rows - r0 : rows_per_block);
+  for (int32_t i = threadIdx.x; i < rows_per_block; i += blockDim.x) {
+    int32_t s = -1;
+    if (i < n) {
+      s = states[slots ? slots[r0 + i] : r0 + i];
+      if (s >= f.S) {
+        if (err) atomicOr(err, BPD_FLAG_STATE_RANGE);
+        s = -1;  // the whole row is masked
+      }
+    }
+    rs[i] = s;
+  }
+  int32_t b = 0, e = 0;
+  if (on && !is_eos) {
+    b = f.off[t];
+    e = f.off[t + 1];
+  }
+  const WalkToken tok = load_walk_token(f.sym, b, e - b, f.off[f.V], f.NS);
+  stage_walk_table<false>(walk_tab, f.trans, f.S, f.NS, f.dead, f.live);
+  __syncthreads();
+  const uint32_t W = uint32_t(f.NS) + 3, fail = uint32_t(f.S) * W;
+  const bool has_eos = __any(is_eos) != 0;
+  for (int32_t i = 0; i < n; i += kWalkRows) {
+    uint32_t cur[kWalkRows];
+    int32_t st[kWalkRows];
+#pragma unroll
+    for (int q = 0; q < kWalkRows; ++q) {
+      st[q] = __builtin_amdgcn_readfirstlane(rs[i + q]);  // rows_per_block is a multiple of kWalkRows
+      cur[q] = st[q] >= 0 ? uint32_t(st[q]) * W : fail;
+    }
+    walk_rows(walk_tab, f.NS, fail, tok, cur);
+    bool ok[kWalkRows];
+#pragma unroll
+    for (int q = 0; q < kWalkRows; ++q) ok[q] = on && walk_tab[cur[q] + f.NS + 2] != kWalkNone;
+    if (has_eos) {
+#pragma unroll
+      for (int q = 0; q < kWalkRows; ++q)
+        if (is_eos) ok[q] = st[q] >= 0 && f.accept[st[q]] != 0;
+    }
+#pragma unroll
+    for (int q = 0; q < kWalkRows; ++q) {
+      if (i + q >= n) break;
+      if (Bits) {
+        const uint64_t m = __ballot(ok[q]);
+        const int64_t tw = t - (threadIdx.x & 63);  // first token of the wave, a multiple of 64
+        if ((threadIdx.x & 63) == 0 && tw < f.V) {
+          uint32_t* out = bits + (r0 + i + q) * words + (tw >> 5);
+          out[0] = uint32_t(m);
+          if ((tw >> 5) + 1 < words) out[1] = uint32_t(m >> 32);
+        }
+      } else if (on && !ok[q]) {
+        uint8_t* p = logits + (r0 + i + q) * ld_bytes + t * E;
+        if (E == 2)
+          *reinterpret_cast<uint16_t*>(p) = uint16_t(fill);
+        else
+          *reinterpret_cast<uint32_t*>(p) = fill;
+      }
+    }
+  }
+}
+
+// The mask for tables too large to stage (Bits = false: fill the rejected
+// logits, element size E) or packed allow bits (Bits = true).  grid (ceil(V / (kFsaThreads kFsaTok)), ceil(rows / kFsaRows)).
+template <int E, bool Bits>
 __global__ __launch_bounds__(kFsaThreads) void fsa_mask_kernel(
     FsaView f, const int32_t* __restrict__ states, const int64_t* __restrict__ slots, int64_t rows,
     uint8_t* __restrict__ logits, int64_t ld_bytes, uint32_t fill, uint32_t* __restrict__ bits,
     int64_t words, int32_t* __restrict__ err) {
-  extern __shared__ __align__(16) int32_t lds[];
   __shared__ int32_t rs[kFsaRows];
   const int tid = threadIdx.x;
   const int32_t* tr = f.trans;
   const uint8_t* lv = f.live;
-  if (InLds) {
-    const int64_t n = int64_t(f.S) * f.NS;
-    for (int64_t i = tid; i < n; i += kFsaThreads) lds[i] = f.trans[i];
-    uint8_t* l8 = reinterpret_cast<uint8_t*>(lds + n);
-    for (int32_t i = tid; i < f.S; i += kFsaThreads) l8[i] = f.live[i];
-    tr = lds;
-    lv = l8;
-  }
   const int64_t r0 = int64_t(blockIdx.y) * kFsaRows;
   if (tid < kFsaRows) {
     const int64_t r = r0 + tid;
@@ -400,31 +468,44 @@ FsaView view_of(const BpdFsaTable& t) {
                  t.tok_offsets, t.tok_symbols, t.vocab, t.eos_id, t.trans16, t.tok_records};
 }
 
-size_t fsa_lds_bytes(const BpdFsaTable& t) {
-  return size_t(t.num_states) * size_t(t.num_symbols) * 4 + size_t(t.num_states);
-}
-
 template <int E, bool Bits>
 int launch_fsa_mask(const BpdFsaTable& t, const int32_t* states, const int64_t* slots, int64_t rows,
                     void* logits, int64_t ld_bytes, uint32_t fill, uint32_t* bits, int64_t words,
                     int32_t* err, hipStream_t s) {
-  const size_t lds = fsa_lds_bytes(t);
-  bool in_lds = lds <= kFsaMaxLds;
+  // Staging a large table takes a launch of a few rows about 12 us whatever
+  // they are, the walk through L2 8 us for one row, 9 for two and 12-20 for
+  // three (826 states); up to 16 KB the staged walk is the faster one from the
+  // first row on (71 states: 7 us against 14).
+  const size_t lds = walk_table_bytes(t.num_states, t.num_symbols);
+  const bool large = lds > 16 * 1024;
+  bool staged = walk_table_fits(t.num_states, t.num_symbols, kWalkMaxLds) && (!large || rows > 2);
   // BPD_FSA_TABLE=global forces the global-memory form (tests cover both
   // forms on small grammars with it)
   if (const char* e = std::getenv("BPD_FSA_TABLE"))
-    if (std::strcmp(e, "global") == 0) in_lds = false;
-  const int64_t gx = (t.vocab + kFsaThreads * kFsaTok - 1) / (kFsaThreads * kFsaTok);
-  const int64_t gy = (rows + kFsaRows - 1) / kFsaRows;
-  BPD_REQUIRE(gy < 65536, "at most %d rows per launch", 65535 * kFsaRows);
-  const dim3 grid = dim3(unsigned(gx), unsigned(gy));
+    if (std::strcmp(e, "global") == 0) staged = false;
+  BPD_REQUIRE((rows + kFsaRows - 1) / kFsaRows < 65536, "at most %d rows per launch", 65535 * kFsaRows);
   uint8_t* lg = static_cast<uint8_t*>(logits);
-  if (in_lds)
-    fsa_mask_kernel<E, Bits, true><<<grid, kFsaThreads, lds, s>>>(view_of(t), states, slots, rows, lg,
-                                                                   ld_bytes, fill, bits, words, err);
-  else
-    fsa_mask_kernel<E, Bits, false><<<grid, kFsaThreads, 0, s>>>(view_of(t), states, slots, rows, lg,
-                                                                  ld_bytes, fill, bits, words, err);
+  if (staged) {
+    const int threads = large ? 1024 : 512;
+    const int64_t tiles = (t.vocab + threads - 1) / threads;
+    // as many waves as the chip holds, so that a staged table serves as many
+    // rows as that allows, and 16 rows at least for a large one (32 rows of
+    // 826 states: 24 us against 30 with 8)
+    int64_t split = (8192 * 64 + tiles * threads - 1) / (tiles * threads);
+    const int64_t groups = (rows + kWalkRows - 1) / kWalkRows;
+    if (split > groups) split = groups;
+    int64_t per = (groups + split - 1) / split * kWalkRows;
+    if (large && per < 16) per = 16;
+    if (per > kWalkBlockRows) per = kWalkBlockRows;
+    const dim3 grid = dim3(unsigned(tiles), unsigned((rows + per - 1) / per));
+    fsa_walk_kernel<E, Bits><<<grid, threads, lds, s>>>(view_of(t), states, slots, rows, int32_t(per), lg,
+                                                         ld_bytes, fill, bits, words, err);
+  } else {
+    const int64_t gx = (t.vocab + kFsaThreads * kFsaTok - 1) / (kFsaThreads * kFsaTok);
+    const dim3 grid = dim3(unsigned(gx), unsigned((rows + kFsaRows - 1) / kFsaRows));
+    fsa_mask_kernel<E, Bits><<<grid, kFsaThreads, 0, s>>>(view_of(t), states, slots, rows, lg, ld_bytes, fill,
+                                                           bits, words, err);
+  }
   BPD_LAUNCHED();
   return BPD_OK;
 }

@@ -28,17 +28,20 @@ inline bool walk_table_fits(int64_t S, int64_t M, size_t max_bytes) {
 inline size_t walk_table_bytes(int64_t S, int64_t M) { return size_t((S + 1) * (M + 3)) * 2; }
 
 // Stages the table; every thread of the block takes part, and a barrier must
-// follow.  A step into `dead` ends the walk with `dead`'s own liveness, as
-// does a walk that starts there.  Loads go out eight entries at a time: one
+// follow.  DeadEnds: a step into `dead` ends the walk with `dead`'s own
+// liveness, as does a walk that starts there (the dense builder's rule);
+// otherwise a step into `dead` fails and a walk that starts there goes on.
+// Loads go out eight entries at a time: one
 // entry per iteration made the staging a chain of memory round trips (the
 // dense builder's 2,400 entries per block took 10 of its 38 us).
+template <bool DeadEnds>
 __device__ __forceinline__ void stage_walk_table(uint16_t* T, const int32_t* __restrict__ trans, int32_t S,
                                                  int32_t M, int32_t dead, const uint8_t* __restrict__ live) {
   constexpr int kBatch = 8;
   const uint32_t W = uint32_t(M) + 3, n = uint32_t(S + 1) * W, nt = blockDim.x;
   const uint32_t magic = uint32_t((0x100000000ull + W - 1) / W);  // i / W = hi32(i * magic) for i < 65536
   const uint32_t fail = uint32_t(S) * W;
-  const uint32_t dead_row = live[dead] ? uint32_t(dead) * W : fail;
+  const uint32_t dead_row = DeadEnds && live[dead] ? uint32_t(dead) * W : fail;
   for (uint32_t i0 = threadIdx.x; i0 < n; i0 += kBatch * nt) {
     int32_t d[kBatch];
 #pragma unroll
@@ -54,7 +57,7 @@ __device__ __forceinline__ void stage_walk_table(uint16_t* T, const int32_t* __r
       if (i < n && c != uint32_t(M) + 2) {
         uint32_t v = uint32_t(d[k]) < uint32_t(S) ? uint32_t(d[k]) * W : fail;
         if (c == uint32_t(M) + 1) v = s * W;
-        if (d[k] == dead || s == uint32_t(dead)) v = dead_row;
+        if (d[k] == dead || (DeadEnds && s == uint32_t(dead))) v = dead_row;
         T[i] = uint16_t(v);
       }
     }

@@ -67,6 +67,30 @@ class OracleWalk:
         return self.state >= 0 and bool(self.accept[self.state])
 
 
+def random_bundle(S: int, M: int, V: int, seed: int, max_len: int = 40) -> FsaTensors:
+    """A bundle of arbitrary tables: targets outside the table, symbol ids at
+    and above M, empty tokens, tokens longer than 16 symbols, EOS inside the
+    vocabulary and a live set that need not be closed (``dead`` live in half
+    of them)."""
+    g = np.random.default_rng(seed)
+    trans = g.integers(-2, S + 2, size=S * M).astype(np.int32)
+    keep = g.random(S * M) < 0.9
+    trans[keep] = g.integers(0, S, size=int(keep.sum()))
+    dead = int(g.integers(0, S))
+    live = (g.random(S) < 0.7).astype(np.uint8)
+    live[dead] = seed % 2
+    lens = g.integers(0, max_len + 1, size=V)
+    lens[g.random(V) < 0.7] //= 8
+    off = np.zeros(V + 1, dtype=np.int32)
+    np.cumsum(lens, out=off[1:])
+    sym = g.integers(0, M, size=int(off[-1]))
+    bad = g.random(sym.size) < 0.01
+    sym[bad] = np.minimum(M + g.integers(0, 4, size=int(bad.sum())), 255)
+    t = torch.from_numpy
+    return FsaTensors(trans=t(trans), accept=t((g.random(S) < 0.3).astype(np.uint8)), live=t(live), num_symbols=M,
+                      dead=dead, offsets=t(off), symbols=t(sym.astype(np.int32)), eos_id=int(g.integers(0, V)))
+
+
 def reachable(tok_next: np.ndarray, start: int) -> list[int]:
     seen, todo = {start}, [start]
     while todo:

@@ -18,7 +18,7 @@ from bpdecode_amd.grammar.pda import CompiledGrammar
 from bpdecode_amd.grammar.regular import residual_dfa
 from bpdecode_amd.ops import FsaTensors
 from oracle import dense as OD
-from tests._util import TOY_PATTERNS, TOY_VOCAB, bits_of, oracle_table
+from tests._util import TOY_PATTERNS, TOY_VOCAB, bits_of, oracle_table, random_bundle
 
 pytestmark = pytest.mark.gpu
 
@@ -414,30 +414,6 @@ def test_device_built_bundles_equal_host_built(dev, serving_vocab):
     d2 = FsaTensors.build(dfa, serving_vocab, device=dev)
     assert h2.tok_next is None and d2.tok_next is None
     assert torch.equal(d2.live.cpu(), h2.live) and torch.equal(d2.trans.cpu(), h2.trans)
-
-
-def random_bundle(S: int, M: int, V: int, seed: int, max_len: int = 40) -> FsaTensors:
-    """A bundle of arbitrary tables: targets outside the table, symbol ids at
-    and above M, empty tokens, tokens longer than 16 symbols, EOS inside the
-    vocabulary and a live set that need not be closed (``dead`` live in half
-    of them)."""
-    g = np.random.default_rng(seed)
-    trans = g.integers(-2, S + 2, size=S * M).astype(np.int32)
-    keep = g.random(S * M) < 0.9
-    trans[keep] = g.integers(0, S, size=int(keep.sum()))
-    dead = int(g.integers(0, S))
-    live = (g.random(S) < 0.7).astype(np.uint8)
-    live[dead] = seed % 2
-    lens = g.integers(0, max_len + 1, size=V)
-    lens[g.random(V) < 0.7] //= 8
-    off = np.zeros(V + 1, dtype=np.int32)
-    np.cumsum(lens, out=off[1:])
-    sym = g.integers(0, M, size=int(off[-1]))
-    bad = g.random(sym.size) < 0.01
-    sym[bad] = np.minimum(M + g.integers(0, 4, size=int(bad.sum())), 255)
-    t = torch.from_numpy
-    return FsaTensors(trans=t(trans), accept=t((g.random(S) < 0.3).astype(np.uint8)), live=t(live), num_symbols=M,
-                      dead=dead, offsets=t(off), symbols=t(sym.astype(np.int32)), eos_id=int(g.integers(0, V)))
 
 
 @pytest.mark.parametrize("S,M,V", [(1, 1, 1), (1, 1, 700), (5, 3, 63), (71, 30, 5001), (72, 110, 513), (73, 110, 1025),

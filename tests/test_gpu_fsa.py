@@ -22,7 +22,7 @@ from bpdecode_amd.grammar.pda import CompiledGrammar
 from bpdecode_amd.grammar.regular import residual_dfa
 from bpdecode_amd.ops import FsaTensors
 from oracle import dense as OD
-from tests._util import TOY_PATTERNS, TOY_VOCAB, bits_of, oracle_table
+from tests._util import TOY_PATTERNS, TOY_VOCAB, bits_of, oracle_table, random_bundle
 
 pytestmark = pytest.mark.gpu
 
@@ -326,3 +326,30 @@ def test_walking_commit_with_a_live_array_not_closed(dev):
     toks = np.array([t for _ in range(S) for t in range(V)], dtype=np.int64)
     nxt = ops.advance_state(gd, torch.from_numpy(st).to(dev), torch.from_numpy(toks).to(dev))
     assert nxt.cpu().numpy().tolist() == tn[st, toks].tolist()
+
+
+@pytest.mark.parametrize("S,M,V", [(1, 1, 1), (5, 3, 63), (71, 30, 1500), (72, 110, 513), (73, 110, 1025), (820, 45, 2049),
+                                   (900, 60, 700), (40, 253, 511), (40, 254, 511)])
+@pytest.mark.parametrize("rows", [1, 2, 3, 17, 300])
+def test_staged_walk_matches_the_general_walk(dev, monkeypatch, S, M, V, rows):
+    """Masks and packed bits from the table staged in LDS (blocks of 512 and
+    1024 threads, the largest staged table, one state or symbol more than
+    fits, rows past one block's 256) equal those walked through memory, for
+    arbitrary tables and states below 0 and past the table; out-of-range
+    states set the flag either way."""
+    _log(f"case staged walk S={S} M={M} V={V} rows={rows}")
+    fd = random_bundle(S, M, V, seed=S + rows).to(dev)
+    g = torch.Generator().manual_seed(rows)
+    st = torch.randint(-2, S + 1, (rows,), generator=g, dtype=torch.int32).to(dev)
+    lg = torch.randn(rows, V + 3, generator=g)
+    got = {}
+    for form in ("lds", "global"):
+        monkeypatch.setenv("BPD_FSA_TABLE", form)
+        err = torch.zeros(1, dtype=torch.int32, device=dev)
+        out = [ops.fsa_compute_mask(fd, st, err=err)]
+        for dt in (torch.float32, torch.bfloat16):
+            x = lg.to(dt).to(dev)
+            out.append(ops.fsa_mask_(x[:, :V], fd, st, neg_inf=-1e4, err=err))
+        got[form] = out + [err]
+    for a, b in zip(got["lds"], got["global"]):
+        assert torch.equal(a, b)
