@@ -84,6 +84,7 @@ _SIGNATURES = {
     "bpd_host_build_reachability": (cint, [vp, i32, i32, vp, vp]),
     "bpd_build_tok_next": (cint, [vp, i32, i32, i32, vp, vp, vp, vp, i64, i32, vp, i32, vp, vp]),
     "bpd_dense_table_bits": (cint, [vp, i32, i64, vp, vp]),
+    "bpd_bit_rows": (cint, [vp, i64, i32, vp, i64, vp, vp, vp]),
     "bpd_narrow_symbols": (cint, [vp, i64, vp, vp, vp]),
     "bpd_fsa_apply_mask": (cint, [C.POINTER(FsaTableC), vp, cint, i64, i64, vp, vp, f64, vp, vp]),
     "bpd_fsa_compute_mask": (cint, [C.POINTER(FsaTableC), vp, vp, i64, vp, vp, vp]),

@@ -284,6 +284,40 @@ __global__ __launch_bounds__(kBitsThreads) void dense_bits_kernel(
   if (sub < kBitsLoads && at < words) bits[r * words + at] = mine;
 }
 
+// The rows' words of a packed allow-bit table, grid (ceil(words / 2048), rows);
+// zeros for a negative state or one outside the table (flagged).  A copy of
+// words 4-byte aligned at best (odd row lengths), 16 bytes per access.
+// 256 rows of V = 151,936: 4.9 MB in ROWS_US, where walking the tokens of 826
+// states' table takes 67 us.
+constexpr int kBitRowLoads = 2;
+
+__global__ __launch_bounds__(kBitsThreads) void bit_rows_kernel(
+    const uint32_t* __restrict__ table, int64_t words, int32_t num_states, const int32_t* __restrict__ states,
+    uint32_t* __restrict__ out, int32_t* __restrict__ err) {
+  const int64_t r = blockIdx.y;
+  const int32_t s = states[r];
+  const bool live_row = s >= 0 && s < num_states;
+  if (s >= num_states && err && blockIdx.x == 0 && threadIdx.x == 0) atomicOr(err, BPD_FLAG_STATE_RANGE);
+  const uint32_t* from = table + (live_row ? int64_t(s) * words : 0);
+  uint32_t* to = out + r * words;
+  I4u v[kBitRowLoads];
+#pragma unroll
+  for (int u = 0; u < kBitRowLoads; ++u) {
+    const int64_t w = ((int64_t(blockIdx.x) * kBitRowLoads + u) * kBitsThreads + threadIdx.x) * 4;
+    v[u] = I4u{0, 0, 0, 0};
+    if (live_row && w + 4 <= words) v[u] = *reinterpret_cast<const I4u*>(from + w);
+  }
+#pragma unroll
+  for (int u = 0; u < kBitRowLoads; ++u) {
+    const int64_t w = ((int64_t(blockIdx.x) * kBitRowLoads + u) * kBitsThreads + threadIdx.x) * 4;
+    if (w + 4 <= words) {
+      *reinterpret_cast<I4u*>(to + w) = v[u];
+    } else {
+      for (int64_t i = w; i < words; ++i) to[i] = live_row ? from[i] : 0u;
+    }
+  }
+}
+
 // tok_next builder over the staged walk table (walk.hpp), grid (tokens, rows /
 // rows_per_block): a thread holds one token's symbols and walks them from the
 // block's rows, four at a time; each row's results go out as one coalesced
@@ -549,6 +583,21 @@ extern "C" int bpd_dense_compute_mask(const int32_t* tok_next, int32_t num_state
   dense_bits_kernel<<<grid, kBitsThreads, 0, as_stream(stream)>>>(tok_next, num_states, vocab, states,
                                                           slots, rows, bits, words, err);
   BPD_LAUNCHED();
+  return BPD_OK;
+}
+
+extern "C" int bpd_bit_rows(const uint32_t* allow_bits, int64_t words, int32_t num_states,
+                            const int32_t* states, int64_t rows, uint32_t* out, int32_t* err, void* stream) {
+  BPD_REQUIRE(num_states > 0 && words >= 0 && rows >= 0, "bad shape");
+  if (rows == 0 || words == 0) return BPD_OK;
+  BPD_REQUIRE(allow_bits && states && out, "null pointer argument");
+  const unsigned gx = unsigned((words + 4 * kBitsThreads * kBitRowLoads - 1) / (4 * kBitsThreads * kBitRowLoads));
+  for (int64_t r0 = 0; r0 < rows; r0 += 65535) {  // the grid's second dimension
+    const int64_t n = rows - r0 < 65535 ? rows - r0 : 65535;
+    bit_rows_kernel<<<dim3(gx, unsigned(n)), kBitsThreads, 0, as_stream(stream)>>>(
+        allow_bits, words, num_states, states + r0, out + r0 * words, err);
+    BPD_LAUNCHED();
+  }
   return BPD_OK;
 }
 

@@ -260,6 +260,9 @@ class FsaTensors:
             if self.tok_next is None and on_dev:
                 st = torch.arange(self.num_states, dtype=torch.int32, device=self.device)
                 self.allow_bits = fsa_compute_mask(self, st)
+                # built here from the tables that c_fsa_table holds (a bundle
+                # made from this one by replace() has the field, not this)
+                self.__dict__["_walked_bits"] = self.allow_bits
             else:
                 base = self.densify()
                 self.tok_next = base.tok_next
@@ -593,6 +596,17 @@ def dense_table_bits(tok_next: torch.Tensor) -> torch.Tensor:
     return out
 
 
+def bit_rows(allow_bits: torch.Tensor, states: torch.Tensor) -> torch.Tensor:
+    """The packed rows of ``allow_bits`` [states, words] for one state per
+    row; zeros for a state outside the table."""
+    dev = _same_device(allow_bits, states)
+    st = _i32(states).view(-1)
+    S, W = allow_bits.shape
+    out = torch.empty((st.numel(), W), dtype=torch.int32, device=dev)
+    check(lib().bpd_bit_rows(ptr(allow_bits), W, S, ptr(st), st.numel(), ptr(out), None, _lib.stream_of(dev)))
+    return out
+
+
 def fsa_mask_(logits, fsa: FsaTensors, states, slots=None, neg_inf=float("-inf"), err=None):
     """Device mask of a bundle without ``tok_next``: every token walked from
     the row's state (``states[slots[b]]`` with ``slots``) by the symbol-class
@@ -771,6 +785,12 @@ def compute_mask(fsa: FsaTensors, states: torch.Tensor) -> torch.Tensor:
     if fsa.tok_next is not None:
         return dense_compute_mask(fsa.tok_next, states)
     if states.device.type == "cuda":
+        # the bundle's own allow-bit table, once it has one, holds every
+        # state's words: 256 rows of V = 151,936 are a 4.9 MB copy instead of a
+        # walk of every token from every row
+        bits = fsa.__dict__.get("_walked_bits")
+        if bits is not None and bits is fsa.allow_bits:
+            return bit_rows(bits, states)
         return fsa_compute_mask(fsa, states)
     rows, idx = _walked_rows(fsa, states)
     return dense_compute_mask(rows, idx)

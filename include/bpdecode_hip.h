@@ -140,6 +140,12 @@ int bpd_build_tok_next(const int32_t* trans, int32_t num_states, int32_t num_sym
 int bpd_dense_table_bits(const int32_t* tok_next, int32_t num_states, int64_t vocab, uint32_t* bits,
                          void* stream);
 
+/* bpd_bit_rows: out[r] = the packed row allow_bits[states[r]] (`words` uint32
+ * each); zeros for a state below 0 or at or above num_states, the latter
+ * flagged as BPD_FLAG_STATE_RANGE in `err` (may be NULL). */
+int bpd_bit_rows(const uint32_t* allow_bits, int64_t words, int32_t num_states,
+                 const int32_t* states, int64_t rows, uint32_t* out, int32_t* err, void* stream);
+
 /* bpd_narrow_symbols: the symbol classes of bpd_build_tok_next from int32
  * ids; *bad (zeroed by the caller, device memory) becomes non-zero when an id
  * lies outside [0, 255]. */

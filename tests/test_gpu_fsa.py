@@ -11,6 +11,8 @@ a host round trip.  Bit-exact."""
 
 from __future__ import annotations
 
+from dataclasses import replace
+
 import numpy as np
 import pytest
 import torch
@@ -353,3 +355,19 @@ def test_staged_walk_matches_the_general_walk(dev, monkeypatch, S, M, V, rows):
         got[form] = out + [err]
     for a, b in zip(got["lds"], got["global"]):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("S,V", [(1, 1), (7, 33), (5, 2048 * 32), (9, 2049 * 32 + 5), (6, 8191)])
+def test_packed_masks_from_the_allow_bit_table(dev, S, V):
+    """compute_mask of a bundle that built its allow-bit table copies rows of
+    it: the same words as the walk, on rows of any length and states outside
+    the table; a bundle derived from it with other tables walks those."""
+    host = random_bundle(S, 5, V, seed=V, max_len=6)
+    fd = host.to(dev)
+    st = torch.tensor([0, S - 1, -1, S, S + 5, -2, 0, S // 2], dtype=torch.int32, device=dev)
+    want = ops.compute_mask(fd, st)  # no table yet: the walk
+    fd.ensure_allow_bits()
+    assert torch.equal(ops.compute_mask(fd, st), want)
+    assert torch.equal(ops.compute_mask(fd, st.long()), want)
+    other = replace(fd, live=torch.zeros_like(fd.live), accept=torch.zeros_like(fd.accept))
+    assert not ops.compute_mask(other, st).any()
