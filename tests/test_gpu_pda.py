@@ -772,3 +772,96 @@ def test_token_records_repacked_when_workspace_overwritten(dev, json_case):
                 ok_o = OP.advance(t, mirror, toks)
                 assert ok.cpu().numpy().tolist() == ok_o.tolist(), call
                 assert np.array_equal(adv.cpu().numpy(), mirror), call
+
+
+def _fresh_rows_case(dev, capacity):
+    g = build_pda_tensors(CompiledGrammar.build(parse_gbnf(GRAMMARS[0])), VOCAB)
+    return OP.Table(g), CFGConstraintBatch(g, capacity=capacity, device=dev)
+
+
+def _first_allowed(t, rows):
+    bits = OP.compute_mask(t, rows)
+    allowed = np.unpackbits(bits.view(np.uint8), axis=1, bitorder="little")[:, :VOCAB.size].astype(bool)
+    return allowed, allowed[:, :-1].argmax(axis=1).astype(np.int32)
+
+
+@pytest.mark.parametrize("capacity,resets", [(1, 1), (240, 240), (241, 241), (700, 500)])
+def test_cfg_batch_turnover_in_one_launch(dev, capacity, resets):
+    """Slots added, reset and taken over between commits (below, at and
+    above the slots of one launch, broken rows among them) hold the initial
+    config-set at the next mask; the others keep theirs."""
+    _log(f"case turnover capacity={capacity} resets={resets}")
+    t, batch = _fresh_rows_case(dev, capacity)
+    rng = np.random.default_rng(capacity)
+    ids = list(range(capacity))
+    slots = [batch.add(i) for i in ids]
+    init = OP.init(t)
+    mirror = np.repeat(init[None], capacity, axis=0)
+    broken = np.zeros(capacity, dtype=bool)
+    for step in range(4):
+        allowed, toks = _first_allowed(t, mirror)
+        got = torch.zeros(capacity, VOCAB.size, device=dev)
+        batch.apply_mask(ids, got)
+        assert np.array_equal(~np.isneginf(got.cpu().numpy()), allowed & ~broken[:, None]), step
+        wrong = rng.random(capacity) < 0.2  # a token that no row takes
+        for r in np.nonzero(wrong)[0]:
+            bad = np.nonzero(~allowed[r])[0]
+            if bad.size:
+                toks[r] = bad[0]
+        batch.commit(ids, torch.from_numpy(toks).to(dev))
+        broken |= OP.advance(t, mirror, toks) == 0
+        for r in rng.choice(capacity, size=resets, replace=False).tolist():
+            if rng.random() < 0.5:
+                batch.reset(ids[r])
+            else:
+                batch.evict(ids[r])
+                ids[r] = ("next", step, r)
+                assert batch.add(ids[r]) == slots[r]
+            mirror[r], broken[r] = init, False
+    assert [batch.is_broken(i) for i in ids[:8]] == broken[:8].tolist()
+    assert np.array_equal(batch._configs.cpu().numpy()[slots], mirror)
+    batch.reset(ids[0])
+    assert np.array_equal(batch._configs.cpu().numpy()[slots[0]], init)
+
+
+def test_cfg_batch_resets_on_other_streams_and_between_replays(dev):
+    """Resets made on the default stream reach a captured mask, resets made
+    between its replays reach each replay, and a batch that moves to another
+    stream keeps the calls' order."""
+    _log("case resets, other stream and capture")
+    t, batch = _fresh_rows_case(dev, 6)
+    ids = list(range(6))
+    for i in ids:
+        batch.add(i)
+    init = np.repeat(OP.init(t)[None], 6, axis=0)
+    fresh, toks = _first_allowed(t, init)
+    moved = init.copy()
+    assert OP.advance(t, moved, toks).all()
+    after = _first_allowed(t, moved)[0]
+    tk = torch.from_numpy(toks).to(dev)
+    side = torch.cuda.Stream()
+    logits = torch.zeros(6, VOCAB.size, device=dev)
+    batch.apply_mask(ids, logits)  # the slot list is on the device from here on
+    with torch.cuda.stream(side):  # and a workspace of the capturing stream
+        pda_mask_(torch.zeros_like(logits), batch.g, batch.g.init_batch(6))
+    torch.cuda.synchronize()
+    batch.commit(ids, tk)
+    batch.reset(0)  # still queued when the capture begins
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        logits.zero_()
+        batch.apply_mask(ids, logits)
+    want = np.where(np.arange(6)[:, None] == 0, fresh, after)
+    for r in range(4):
+        graph.replay()
+        assert np.array_equal(~np.isneginf(logits.cpu().numpy()), want), r
+        batch.reset(r + 1)
+        want[r + 1] = fresh[r + 1]
+    with torch.cuda.stream(side):
+        side.wait_stream(torch.cuda.default_stream())
+        batch.reset(5)
+        assert not batch.is_broken(5)
+        lg = torch.zeros(6, VOCAB.size, device=dev)
+        batch.apply_mask(ids, lg)
+    side.synchronize()
+    assert np.array_equal(~np.isneginf(lg.cpu().numpy()), fresh)
