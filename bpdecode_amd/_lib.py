@@ -124,6 +124,8 @@ _SIGNATURES = {
     "bpd_soft_prior_workspace_bytes": (sz, [i64, i64, i32, i32]),
     "bpd_soft_prior": (cint, [vp, i64, i64, i64, i32, vp, vp, i32, vp, vp, C.POINTER(SoftClassesC),
                               i32, f32, vp, sz, vp, vp]),
+    "bpd_soft_prior_queued": (cint, [vp, i64, i64, i64, i32, vp, vp, i32, vp, vp, vp, i64,
+                                     C.POINTER(SoftClassesC), i32, f32, vp, sz, vp, vp]),
     "bpd_soft_prior_noalloc": (cint, [vp, i64, i64, i64, i32, vp, vp, i32, vp, vp,
                                       C.POINTER(SoftClassesC), i32, f32, vp, vp]),
     "bpd_host_soft_prior": (cint, [vp, i64, i64, i64, vp, i32, vp, vp, i32, vp, vp, i32, f32]),

@@ -451,6 +451,22 @@ class ConstraintBatch:
         plus ``alpha`` times the log-probability, under the row's own
         softmax, of staying on a live path for ``k - 1`` further tokens
         (``-inf`` on grammar-disallowed tokens)."""
+        if (self._fast and logits.dtype == torch.float32 and k >= 1 and self.fsa.tok_next is not None
+                and self._fast_logits(logits, len(seq_ids))):
+            fsa, V, B = self.fsa, self._V, len(seq_ids)
+            sc = fsa.ensure_soft_classes()
+            acc, live = fsa.accept.contiguous(), fsa.live.contiguous()
+            eos = fsa.eos_id if fsa.eos_id is not None and 0 <= fsa.eos_id < V else -1
+            stream = _lib.stream_of(self.device)
+            ws, ws_bytes = sc.workspace(B, self.device, stream)
+            slots, pend, n = self._slots_fused(seq_ids, True)
+            check(lib().bpd_soft_prior_queued(
+                logits.data_ptr(), B, V, logits.stride(0) if B > 1 else V, self._S, acc.data_ptr(), live.data_ptr(),
+                eos, self._pool_ptr, slots, pend, n, C.byref(sc.c_struct()), int(k), float(alpha), ws.data_ptr(),
+                ws_bytes, self._err_ptr, stream))
+            if n:
+                self._launched()
+            return logits
         slots = self._slots(seq_ids)
         ops.apply_soft_prior_(logits, self.fsa, self._state, k, alpha, slots=slots, err=self._err)
         return logits

@@ -729,6 +729,19 @@ PriorPlan prior_plan(int64_t rows, int64_t vocab, int32_t C, int32_t P, bool for
   return pl;
 }
 
+// Queued pool writes of a batch: the statistics launch, which needs no row's
+// state, makes them, and the launches after it read the pool.
+struct QueuedWrites {
+  int32_t* pool;
+  const int64_t* pending;  // count slots, then as many values
+  int32_t count;
+};
+
+__device__ __forceinline__ void make_queued_writes(const QueuedWrites& q) {
+  if (blockIdx.x == 0 && blockIdx.y == 0)
+    for (int32_t i = threadIdx.x; i < q.count; i += kPriorThreads) q.pool[q.pending[i]] = int32_t(q.pending[q.count + i]);
+}
+
 struct PriorWs {
   float* part;   // [rows, G, 2] chunk logsumexp partials
   float* mid;    // class-atomic: [rows, G, C, 2] class partials; pieces: [rows, P, 2]
@@ -773,7 +786,8 @@ __device__ inline int32_t narrow_class(uint32_t c) { return c == 0xFFFFu ? -1 : 
 template <bool Vec, bool Narrow>
 __global__ __launch_bounds__(kPriorThreads) void prior_stats_classes_kernel(
     const float* __restrict__ logits, int64_t ld, int64_t V, const int32_t* __restrict__ token_class,
-    const uint16_t* __restrict__ token_class16, int32_t C, PriorWs ws) {
+    const uint16_t* __restrict__ token_class16, int32_t C, PriorWs ws, QueuedWrites queued) {
+  make_queued_writes(queued);
   __shared__ int32_t cmax[kLdsClasses];
   __shared__ float csum[kLdsClasses];
   constexpr int kE = 4 * kStatLoads;
@@ -866,7 +880,8 @@ __global__ __launch_bounds__(kPriorThreads) void prior_stats_classes_kernel(
 template <int Cap>
 __global__ __launch_bounds__(kPriorThreads) void prior_stats_members_kernel(
     const float* __restrict__ logits, int64_t ld, int64_t V, const uint32_t* __restrict__ members,
-    int32_t C, PriorWs ws) {
+    int32_t C, PriorWs ws, QueuedWrites queued) {
+  make_queued_writes(queued);
   static_assert(kStatChunk == BPD_SOFT_MEMBER_CHUNK, "member lists are cut at the statistics chunk");
   extern __shared__ __align__(16) float smem[];
   float4* xs = reinterpret_cast<float4*>(smem);
@@ -952,7 +967,8 @@ __global__ __launch_bounds__(kPriorThreads) void prior_stats_members_kernel(
 // Dynamic LDS: 4 * C wave sums, then C class maxima and C sums (exact path).
 __global__ __launch_bounds__(kPriorThreads) void prior_stats_wave_kernel(
     const float* __restrict__ logits, int64_t ld, int64_t V, const uint16_t* __restrict__ token_class16,
-    int32_t C, PriorWs ws) {
+    int32_t C, PriorWs ws, QueuedWrites queued) {
+  make_queued_writes(queued);
   extern __shared__ __align__(16) float smem[];
   constexpr int kWaves = kPriorThreads / 64;
   float* wsum = smem;                                               // [kWaves][C]
@@ -1089,7 +1105,8 @@ __global__ __launch_bounds__(kPriorThreads) void prior_stats_wave_kernel(
 template <int Cap>
 __global__ __launch_bounds__(kPriorThreads) void prior_stats_list_kernel(
     const float* __restrict__ logits, int64_t ld, int64_t V, const uint32_t* __restrict__ members,
-    int32_t C, PriorWs ws) {
+    int32_t C, PriorWs ws, QueuedWrites queued) {
+  make_queued_writes(queued);
   static_assert(kWideChunk == 2 * BPD_SOFT_MEMBER_CHUNK, "a block covers two member chunks");
   extern __shared__ __align__(16) float smem[];
   constexpr int kWaves = kPriorThreads / 64;
@@ -1213,7 +1230,8 @@ __global__ __launch_bounds__(kPriorThreads) void prior_stats_list_kernel(
 template <bool Vec>
 __global__ __launch_bounds__(kPriorThreads) void prior_stats_pieces_kernel(
     const float* __restrict__ logits, int64_t ld, int64_t V, int64_t chunk, int G,
-    BpdSoftClasses cls, PriorWs ws) {
+    BpdSoftClasses cls, PriorWs ws, QueuedWrites queued) {
+  make_queued_writes(queued);
   const int g = blockIdx.x;
   const int64_t b = blockIdx.y;
   const int32_t P = cls.num_pieces;
@@ -1794,9 +1812,9 @@ namespace {
 // The prior lookahead on a caller-provided workspace (both entry points).
 int soft_prior_impl(float* logits, int64_t rows, int64_t vocab, int64_t ld, int32_t num_states,
                     const uint8_t* accept, const uint8_t* live, int32_t eos_id,
-                    const int32_t* states, const int64_t* slots, const BpdSoftClasses* classes,
-                    int32_t k, float alpha, void* workspace, size_t workspace_bytes, int32_t* err,
-                    void* stream) {
+                    const int32_t* states, const int64_t* slots, const QueuedWrites& queued,
+                    const BpdSoftClasses* classes, int32_t k, float alpha, void* workspace,
+                    size_t workspace_bytes, int32_t* err, void* stream) {
   BPD_REQUIRE(rows >= 0 && vocab > 0 && ld >= vocab, "bad logits shape");
   BPD_REQUIRE(num_states > 0 && num_states <= kPriorMaxStates, "1..%d states", kPriorMaxStates);
   BPD_REQUIRE(classes, "null classes");
@@ -1842,7 +1860,7 @@ int soft_prior_impl(float* logits, int64_t rows, int64_t vocab, int64_t ld, int3
   prior_stats_classes_kernel<VEC, NARROW><<<grid, kPriorThreads, 0, st>>>(logits, ld, vocab,    \
                                                                          cls.token_class,       \
                                                                          cls.token_class16,     \
-                                                                         cls.num_classes, ws)
+                                                                         cls.num_classes, ws, queued)
     const bool members = vocab % 4 == 0 && ld % 4 == 0 && aligned16(logits) && cls.chunk_members != nullptr &&
                          cls.num_classes < 65535 && std::strcmp(choice, "classes") != 0 &&
                          (cls.chunk_cap == 256 || cls.chunk_cap == 512 || cls.chunk_cap == 1024);
@@ -1850,22 +1868,22 @@ int soft_prior_impl(float* logits, int64_t rows, int64_t vocab, int64_t ld, int3
     const size_t llds = (size_t(kWideChunk) + size_t(kPriorThreads / 64 + 2) * cls.num_classes) * 4;
     if (pl.wide && list_ok && cls.chunk_cap == 256)
       prior_stats_list_kernel<256><<<grid, kPriorThreads, llds, st>>>(logits, ld, vocab, cls.chunk_members,
-                                                                      cls.num_classes, ws);
+                                                                      cls.num_classes, ws, queued);
     else if (pl.wide && list_ok && cls.chunk_cap == 512)
       prior_stats_list_kernel<512><<<grid, kPriorThreads, llds, st>>>(logits, ld, vocab, cls.chunk_members,
-                                                                      cls.num_classes, ws);
+                                                                      cls.num_classes, ws, queued);
     else if (pl.wide && list_ok)
       prior_stats_list_kernel<1024><<<grid, kPriorThreads, llds, st>>>(logits, ld, vocab, cls.chunk_members,
-                                                                       cls.num_classes, ws);
+                                                                       cls.num_classes, ws, queued);
     else if (pl.wide)
       prior_stats_wave_kernel<<<grid, kPriorThreads, size_t(cls.num_classes) * (kPriorThreads / 64 + 2) * 4, st>>>(
-          logits, ld, vocab, cls.token_class16, cls.num_classes, ws);
+          logits, ld, vocab, cls.token_class16, cls.num_classes, ws, queued);
     else if (members && cls.chunk_cap == 256)
-      prior_stats_members_kernel<256><<<grid, kPriorThreads, mlds, st>>>(logits, ld, vocab, cls.chunk_members, cls.num_classes, ws);
+      prior_stats_members_kernel<256><<<grid, kPriorThreads, mlds, st>>>(logits, ld, vocab, cls.chunk_members, cls.num_classes, ws, queued);
     else if (members && cls.chunk_cap == 512)
-      prior_stats_members_kernel<512><<<grid, kPriorThreads, mlds, st>>>(logits, ld, vocab, cls.chunk_members, cls.num_classes, ws);
+      prior_stats_members_kernel<512><<<grid, kPriorThreads, mlds, st>>>(logits, ld, vocab, cls.chunk_members, cls.num_classes, ws, queued);
     else if (members)
-      prior_stats_members_kernel<1024><<<grid, kPriorThreads, mlds, st>>>(logits, ld, vocab, cls.chunk_members, cls.num_classes, ws);
+      prior_stats_members_kernel<1024><<<grid, kPriorThreads, mlds, st>>>(logits, ld, vocab, cls.chunk_members, cls.num_classes, ws, queued);
     else if (narrow && nvec) BPD_PRIOR_STATS(true, true);
     else if (narrow) BPD_PRIOR_STATS(false, true);
     else if (vec) BPD_PRIOR_STATS(true, false);
@@ -1876,9 +1894,9 @@ int soft_prior_impl(float* logits, int64_t rows, int64_t vocab, int64_t ld, int3
     chunk = (chunk + 3) / 4 * 4;
     const dim3 grid = dim3(unsigned(pl.G + pl.Gp), unsigned(rows));
     if (vec) {
-      prior_stats_pieces_kernel<true><<<grid, kPriorThreads, 0, st>>>(logits, ld, vocab, chunk, pl.G, cls, ws);
+      prior_stats_pieces_kernel<true><<<grid, kPriorThreads, 0, st>>>(logits, ld, vocab, chunk, pl.G, cls, ws, queued);
     } else {
-      prior_stats_pieces_kernel<false><<<grid, kPriorThreads, 0, st>>>(logits, ld, vocab, chunk, pl.G, cls, ws);
+      prior_stats_pieces_kernel<false><<<grid, kPriorThreads, 0, st>>>(logits, ld, vocab, chunk, pl.G, cls, ws, queued);
     }
   }
   BPD_LAUNCHED();
@@ -1929,7 +1947,19 @@ extern "C" int bpd_soft_prior(float* logits, int64_t rows, int64_t vocab, int64_
                               const BpdSoftClasses* classes, int32_t k, float alpha,
                               void* workspace, size_t workspace_bytes, int32_t* err, void* stream) {
   return soft_prior_impl(logits, rows, vocab, ld, num_states, accept, live, eos_id, states, slots,
-                         classes, k, alpha, workspace, workspace_bytes, err, stream);
+                         QueuedWrites{}, classes, k, alpha, workspace, workspace_bytes, err, stream);
+}
+
+extern "C" int bpd_soft_prior_queued(float* logits, int64_t rows, int64_t vocab, int64_t ld,
+                                     int32_t num_states, const uint8_t* accept, const uint8_t* live,
+                                     int32_t eos_id, int32_t* states, const int64_t* slots,
+                                     const int64_t* pending, int64_t num_pending,
+                                     const BpdSoftClasses* classes, int32_t k, float alpha,
+                                     void* workspace, size_t workspace_bytes, int32_t* err, void* stream) {
+  if (int rc = check_pending(pending, num_pending, slots, rows)) return rc;
+  return soft_prior_impl(logits, rows, vocab, ld, num_states, accept, live, eos_id, states, slots,
+                         QueuedWrites{states, pending, int32_t(num_pending)}, classes, k, alpha, workspace,
+                         workspace_bytes, err, stream);
 }
 
 // Workspace of the allocation-free entry point: a file-scope device array,
@@ -1983,7 +2013,8 @@ extern "C" int bpd_soft_prior_noalloc(float* logits, int64_t rows, int64_t vocab
   void* ws = nullptr;
   if (int rc = scratch_address(stream, &ws)) return rc;
   return soft_prior_impl(logits, rows, vocab, ld, num_states, accept, live, eos_id, states, slots,
-                         classes, k, alpha, ws, size_t(BPD_SOFT_PRIOR_SCRATCH_BYTES), err, stream);
+                         QueuedWrites{}, classes, k, alpha, ws, size_t(BPD_SOFT_PRIOR_SCRATCH_BYTES), err,
+                         stream);
 }
 
 // Token classes of the prior recurrence (once per grammar, host side).

@@ -550,6 +550,12 @@ int bpd_soft_prior(float* logits, int64_t rows, int64_t vocab, int64_t ld, int32
                    const int32_t* states, const int64_t* slots, const BpdSoftClasses* classes,
                    int32_t k, float alpha, void* workspace, size_t workspace_bytes, int32_t* err,
                    void* stream);
+/* The same with queued pool writes (`pending`, as bpd_dense_apply_mask). */
+int bpd_soft_prior_queued(float* logits, int64_t rows, int64_t vocab, int64_t ld, int32_t num_states,
+                          const uint8_t* accept, const uint8_t* live, int32_t eos_id,
+                          int32_t* states, const int64_t* slots, const int64_t* pending,
+                          int64_t num_pending, const BpdSoftClasses* classes, int32_t k, float alpha,
+                          void* workspace, size_t workspace_bytes, int32_t* err, void* stream);
 int bpd_host_soft_prior(float* logits, int64_t rows, int64_t vocab, int64_t ld,
                         const int32_t* tok_next, int32_t num_states, const uint8_t* accept,
                         const uint8_t* live, int32_t eos_id, const int32_t* states,

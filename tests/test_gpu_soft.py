@@ -149,6 +149,45 @@ def test_apply_soft_carries_queued_writes(dev):
     assert nxt == [int(fsa.tok_next[s, tok]) if s >= 0 else -1 for s in states]
 
 
+@pytest.mark.parametrize("vocab", ["v17", "v20"])
+@pytest.mark.parametrize("stats", ["list", "wave", "members", "classes", "pieces"])
+def test_prior_carries_queued_writes(dev, vocab, stats, monkeypatch):
+    """add / evict / reset before apply_soft_prior: its first launch makes
+    them, its rows read them, and the pool holds them for the next commit."""
+    if stats == "pieces":
+        monkeypatch.setenv("BPD_SOFT_PRIOR_PIECES", "1")
+    else:
+        monkeypatch.setenv("BPD_SOFT_STATS", stats)
+    voc = TOY_VOCAB if vocab == "v17" else TOY_VOCAB20
+    fsa = FsaTensors.build("a[012]+|b0", voc).densify().to(dev)
+    batch = ConstraintBatch(fsa, capacity=300, device=dev)
+    ids = list(range(290))
+    for i in ids:
+        batch.add(i)
+    tok = voc.token_bytes.index(b"a")
+    batch.commit(ids, torch.full((290,), tok, dtype=torch.int64, device=dev))
+    after = int(fsa.tok_next[fsa.start, tok])
+    states = [after] * 290
+    for queued in (3, 250, 290):  # 250 fit one launch's queue, 290 are flushed first
+        for i in range(queued):
+            batch.reset(ids[i])
+        states[:queued] = [fsa.start] * queued
+        batch.evict(ids[-1])
+        batch.add(("new", queued))
+        ids[-1], states[-1] = ("new", queued), fsa.start
+        x = torch.randn(290, voc.size, generator=torch.Generator().manual_seed(queued)) * 3
+        got = x.to(dev)
+        batch.apply_soft_prior(ids, got, 3, 0.5)
+        want = x.clone()
+        ops.apply_soft_prior_(want, fsa.to("cpu"), torch.tensor(states, dtype=torch.int32), 3, 0.5)
+        assert torch.equal(torch.isneginf(got.cpu()), torch.isneginf(want))
+        assert torch.allclose(got.cpu(), want, rtol=1e-5, atol=1e-5)
+        states = batch.commit(ids, torch.full((290,), tok, dtype=torch.int64, device=dev)).tolist()
+        assert states == [batch.state_of(i) for i in ids]
+        batch.commit(ids, torch.full((290,), voc.token_bytes.index(b"0"), dtype=torch.int64, device=dev))
+        states = [int(fsa.tok_next[s, voc.token_bytes.index(b"0")]) if s >= 0 else -1 for s in states]
+
+
 # ------------------------------------------------------- prior-weighted --
 # The toy vocabulary with three more tokens: V = 20, a multiple of 4, so the
 # vectorised kernels apply (V = 17 takes the scalar ones).
