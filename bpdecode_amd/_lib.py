@@ -122,6 +122,7 @@ _SIGNATURES = {
     "bpd_soft_apply_queued": (cint, [vp, cint, i64, i64, i64, vp, i32, vp, vp, vp, i64, f32, vp, vp]),
     "bpd_host_soft_classes": (cint, [vp, i32, i64, C.POINTER(SoftClassesC)]),
     "bpd_soft_prior_workspace_bytes": (sz, [i64, i64, i32, i32]),
+    "bpd_soft_prior_workspace_full": (sz, [i64, i64, C.POINTER(SoftClassesC)]),
     "bpd_soft_prior": (cint, [vp, i64, i64, i64, i32, vp, vp, i32, vp, vp, C.POINTER(SoftClassesC),
                               i32, f32, vp, sz, vp, vp]),
     "bpd_soft_prior_queued": (cint, [vp, i64, i64, i64, i32, vp, vp, i32, vp, vp, vp, i64,

@@ -642,6 +642,7 @@ namespace {
 
 constexpr int kPriorThreads = 256;
 constexpr int kPriorOutThreads = 256;
+constexpr int64_t kComputeUnits = 256;
 constexpr int kPriorMaxStates = 4096;
 constexpr int kPieceMembers = 256;
 constexpr int kLdsClasses = 1024;                          // class-atomic stats up to this many classes
@@ -649,7 +650,21 @@ constexpr int kStatLoads = 4;                              // float4 loads per t
 constexpr int64_t kStatChunk = kPriorThreads * 4 * kStatLoads;  // tokens per block
 constexpr size_t kPriorMaxLds = 60 * 1024;
 constexpr float kLog2e = 1.4426950408889634f;
-typedef float F4v __attribute__((ext_vector_type(4)));  // float4 for the non-temporal builtins
+typedef float F4u __attribute__((ext_vector_type(4), aligned(4)));  // 16 bytes at any float
+
+// Tokens t .. t + 3 of a row of V; -inf beyond it.
+__device__ __forceinline__ float4 load_tokens(const float* __restrict__ row, int64_t t, int64_t V) {
+  float4 x = make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
+  if (t + 4 <= V) {
+    const F4u v = *reinterpret_cast<const F4u*>(row + t);
+    x = make_float4(v[0], v[1], v[2], v[3]);
+  } else {
+    if (t < V) x.x = row[t];
+    if (t + 1 < V) x.y = row[t + 1];
+    if (t + 2 < V) x.z = row[t + 2];
+  }
+  return x;
+}
 
 // 2^x by the hardware exponential (v_exp_f32); used for x <= 0.
 __device__ inline float exp2_fast(float x) { return __builtin_amdgcn_exp2f(x); }
@@ -745,8 +760,9 @@ __device__ __forceinline__ void make_queued_writes(const QueuedWrites& q) {
 struct PriorWs {
   float* part;   // [rows, G, 2] chunk logsumexp partials
   float* mid;    // class-atomic: [rows, G, C, 2] class partials; pieces: [rows, P, 2]
-  float* lse;    // [rows]
+  float* lse;    // [rows]; with the member lists the EOS logits
   float* zcls;   // [rows, C]
+  float* vals;   // [rows, member chunks, cap] the members' logits, or null
 };
 
 size_t prior_mid_floats(int64_t rows, const PriorPlan& pl, int32_t C, int32_t P) {
@@ -763,12 +779,17 @@ PriorWs prior_ws(void* base, int64_t rows, const PriorPlan& pl, int32_t C, int32
   w.lse = reinterpret_cast<float*>(p);
   p += align256(size_t(rows) * 4);
   w.zcls = reinterpret_cast<float*>(p);
+  w.vals = nullptr;
   return w;
 }
 
 size_t prior_ws_bytes(int64_t rows, const PriorPlan& pl, int32_t C, int32_t P) {
   return align256(size_t(rows) * pl.G * 8) + align256(prior_mid_floats(rows, pl, C, P) * 4) +
          align256(size_t(rows) * 4) + align256(size_t(rows) * C * 4);
+}
+
+size_t prior_vals_bytes(int64_t rows, int64_t vocab, int32_t cap) {
+  return size_t(rows) * ((vocab + BPD_SOFT_MEMBER_CHUNK - 1) / BPD_SOFT_MEMBER_CHUNK) * cap * 4;
 }
 
 size_t prior_lds_bytes(int32_t S, int32_t C, int32_t P, int64_t pairs, bool pairs_in_lds, bool pieces) {
@@ -1105,7 +1126,7 @@ __global__ __launch_bounds__(kPriorThreads) void prior_stats_wave_kernel(
 template <int Cap>
 __global__ __launch_bounds__(kPriorThreads) void prior_stats_list_kernel(
     const float* __restrict__ logits, int64_t ld, int64_t V, const uint32_t* __restrict__ members,
-    int32_t C, PriorWs ws, QueuedWrites queued) {
+    int32_t C, int32_t eos, PriorWs ws, QueuedWrites queued) {
   make_queued_writes(queued);
   static_assert(kWideChunk == 2 * BPD_SOFT_MEMBER_CHUNK, "a block covers two member chunks");
   extern __shared__ __align__(16) float smem[];
@@ -1135,8 +1156,7 @@ __global__ __launch_bounds__(kPriorThreads) void prior_stats_list_kernel(
 #pragma unroll
   for (int u = 0; u < kWideLoads; ++u) {
     const int64_t t = base + (int64_t(u) * kPriorThreads + threadIdx.x) * 4;
-    x[u] = t < V ? *reinterpret_cast<const float4*>(row + t)
-                 : make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
+    x[u] = load_tokens(row, t, V);
   }
   for (int32_t c = threadIdx.x; c < kWaves * C; c += kPriorThreads) wsum[c] = 0.0f;
   float m = -INFINITY;
@@ -1163,8 +1183,10 @@ __global__ __launch_bounds__(kPriorThreads) void prior_stats_list_kernel(
     for (int i = 0; i < kWaves; ++i) r = lse_merge_fast(r, Lse{wm[i], wl[i]});
     ws.part[(b * G + g) * 2] = r.m;
     ws.part[(b * G + g) * 2 + 1] = r.s;
+    if (eos >= base && eos < base + kWideChunk) ws.lse[b] = smem[eos - base];
   }
   const float* xf = smem;
+  float* vals = ws.vals ? ws.vals + (b * nchunks + 2 * int64_t(g)) * Cap + threadIdx.x : nullptr;
   float v[2 * kHalf];
   bool under = false;
 #pragma unroll
@@ -1174,6 +1196,7 @@ __global__ __launch_bounds__(kPriorThreads) void prior_stats_list_kernel(
       const int o = int(mm[j] >> 16) + (j / kHalf) * BPD_SOFT_MEMBER_CHUNK;
       const int ow = (o >> 8) & (kWaves - 1);
       v[j] = xf[o];
+      if (vals) vals[j * kPriorThreads] = v[j];
       if (v[j] != -INFINITY) {
         const float mw = wm[ow];
         under = under || v[j] - mw < -80.0f;
@@ -1361,13 +1384,12 @@ __device__ inline float prior_value(float x, float lse, int64_t t, float z, bool
 // kRoundThreads threads of its block: lc holds the class logsumexps of the
 // row (LDS, reused for zcls), z0 / z1 the state values (z0 initialised: 0
 // for live states, -inf else), flag / so the state flags and pair offsets,
-// pr the pairs (PairsInLds); writes zcls[b] and lse[b] to the workspace.
+// pr the pairs (PairsInLds).
 template <bool PairsInLds>
 __device__ __forceinline__ void prior_rounds_tail(float* lc, float* z0, float* z1, const uint8_t* flag,
                                                   const int32_t* so, const uint32_t* pr,
                                                   const BpdSoftClasses& cls, int32_t S, int32_t rounds,
-                                                  float lse, float lp_eos, int32_t sb, int64_t b,
-                                                  const PriorWs& ws) {
+                                                  float lse, float lp_eos, int32_t sb) {
   const int tid = threadIdx.x;
   const int32_t C = cls.num_classes;
   // eight lanes per state: lane l folds pairs l, l + 8, ... of its state
@@ -1481,19 +1503,94 @@ __device__ __forceinline__ void prior_rounds_tail(float* lc, float* z0, float* z
     }
   }
   __syncthreads();
-  for (int32_t c = tid; c < C; c += kRoundThreads) ws.zcls[b * C + c] = lc[c];
-  if (tid == 0) ws.lse[b] = lse;
 }
 
-template <bool PairsInLds, bool ClassStats>
-__global__ __launch_bounds__(kRoundThreads) void prior_rounds_kernel(
-    const float* __restrict__ logits, int64_t ld, int32_t S, int G, BpdSoftClasses cls,
+// What the output stage of the rounds kernel needs besides the rounds.
+struct PriorOut {
+  float* logits;
+  int64_t vocab;
+  float alpha;
+  int32_t* err;
+};
+
+// Output of row b by one of `splits` blocks: member chunks split, split +
+// splits, ... of BPD_SOFT_MEMBER_CHUNK tokens, one float4 per thread.  A chunk
+// is staged as -inf; the threads put x - lse + alpha * z there for the members
+// of a class with a finite value (EOS: its log softmax when the state
+// accepts), and it leaves as 16-byte stores.  Two stages take turns, so a
+// chunk costs one barrier, and the next chunk's list is in flight meanwhile.
+// `stage`: two chunks of LDS.
+__device__ __forceinline__ void prior_out_chunks(const PriorOut& out, int64_t ld, int64_t b, const float* z,
+                                                 float4* stage, const BpdSoftClasses& cls,
+                                                 const float* __restrict__ vals, float lse, float x_eos,
+                                                 bool acc_s, int32_t eos, int split, int splits) {
+  static_assert(kRoundThreads * 4 == BPD_SOFT_MEMBER_CHUNK, "one float4 per thread");
+  const int tid = threadIdx.x;
+  const float4 ninf = make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
+  const int64_t V = out.vocab;
+  const int nchunks = int((V + BPD_SOFT_MEMBER_CHUNK - 1) / BPD_SOFT_MEMBER_CHUNK);
+  float* row = out.logits + b * ld;
+  const int32_t cap = cls.chunk_cap;
+  stage[tid] = ninf;
+  stage[kRoundThreads + tid] = ninf;
+  uint32_t mm = 0xFFFFFFFFu;
+  float xv = 0.0f;
+  auto fetch = [&](int ch) {
+    mm = 0xFFFFFFFFu;
+    if (ch < nchunks && tid < cap) {
+      mm = cls.chunk_members[int64_t(ch) * cap + tid];
+      if (vals) {
+        xv = vals[(b * nchunks + ch) * cap + tid];
+      } else if (mm != 0xFFFFFFFFu) {
+        xv = row[int64_t(ch) * BPD_SOFT_MEMBER_CHUNK + (mm >> 16)];
+      }
+    }
+  };
+  fetch(split);
+  __syncthreads();
+  int turn = 0;
+  for (int ch = split; ch < nchunks; ch += splits, turn ^= 1) {
+    float4* st = stage + turn * kRoundThreads;
+    const int64_t base = int64_t(ch) * BPD_SOFT_MEMBER_CHUNK;
+    if (mm != 0xFFFFFFFFu && base + int64_t(mm >> 16) != eos) {
+      const float zv = z[mm & 0xFFFFu];
+      if (zv != -INFINITY) {
+        const float lp = xv - lse;
+        reinterpret_cast<float*>(st)[mm >> 16] = out.alpha != 0.0f ? fmaf(out.alpha, zv, lp) : lp;
+      }
+    }
+    if (tid == 0 && acc_s && eos >= base && eos < base + BPD_SOFT_MEMBER_CHUNK)
+      reinterpret_cast<float*>(st)[eos - base] = x_eos - lse;
+    fetch(ch + splits);
+    __syncthreads();
+    const float4 o = st[tid];
+    st[tid] = ninf;
+    const int64_t t = base + tid * 4;
+    if (t + 4 <= V) {
+      __builtin_nontemporal_store(F4u{o.x, o.y, o.z, o.w}, reinterpret_cast<F4u*>(row + t));
+    } else {
+      if (t < V) row[t] = o.x;
+      if (t + 1 < V) row[t + 1] = o.y;
+      if (t + 2 < V) row[t + 2] = o.z;
+    }
+  }
+}
+
+// Out: the member-list output follows in the same launch, grid (splits, rows),
+// every block of a row running its rounds (the EOS logit then comes from the
+// statistics: another block of the row may have written its output already).
+// [128, 151936], 71 states, k = 4: ROUNDS_US us, where a launch of one block
+// per row took 10.0 and a gathering output launch after it 21.4; the rounds
+// are a chain of LDS latencies that leaves a block room for a second one.
+template <bool PairsInLds, bool ClassStats, bool Out>
+__global__ __launch_bounds__(kRoundThreads, 8) void prior_rounds_kernel(
+    const float* logits, int64_t ld, int32_t S, int G, BpdSoftClasses cls,
     const uint8_t* __restrict__ accept, const uint8_t* __restrict__ live, int32_t eos,
     const int32_t* __restrict__ states, const int64_t* __restrict__ slots, int32_t rounds,
-    PriorWs ws) {
+    PriorWs ws, PriorOut out) {
   extern __shared__ __align__(16) float lds[];
   __shared__ float lse_sh;
-  const int64_t b = blockIdx.x;
+  const int64_t b = Out ? blockIdx.y : blockIdx.x;
   const int tid = threadIdx.x;
   const int32_t C = cls.num_classes, P = cls.num_pieces, NP = cls.num_pairs;
   float* lc = lds;                                        // [C] class logsumexp, later zcls
@@ -1505,7 +1602,7 @@ __global__ __launch_bounds__(kRoundThreads) void prior_rounds_kernel(
 
   // global loads: the EOS logit, the pairs, the class partials, the row
   // partials, the state flags and offsets
-  const float x_eos = eos >= 0 ? logits[b * ld + eos] : -INFINITY;
+  const float x_eos = eos >= 0 ? (Out ? ws.lse[b] : logits[b * ld + eos]) : -INFINITY;
   uint32_t pv[kPairRegs];
   if (PairsInLds) {
 #pragma unroll
@@ -1609,7 +1706,17 @@ __global__ __launch_bounds__(kRoundThreads) void prior_rounds_kernel(
   __syncthreads();
   const float lse = lse_sh;
   const float lp_eos = eos >= 0 ? x_eos - lse : -INFINITY;
-  prior_rounds_tail<PairsInLds>(lc, z0, z1, flag, so, pr, cls, S, rounds, lse, lp_eos, sb, b, ws);
+  prior_rounds_tail<PairsInLds>(lc, z0, z1, flag, so, pr, cls, S, rounds, lse, lp_eos, sb);
+  if (Out) {
+    const bool live_row = sb >= 0 && sb < S;
+    if (sb >= S && out.err && blockIdx.x == 0 && tid == 0) atomicOr(out.err, BPD_FLAG_STATE_RANGE);
+    float4* stage = reinterpret_cast<float4*>(lds + (C + 3) / 4 * 4);  // over what the rounds needed
+    prior_out_chunks(out, ld, b, lc, stage, cls, ws.vals, lse, x_eos, live_row && accept[sb] != 0, eos,
+                     int(blockIdx.x), int(gridDim.x));
+  } else {
+    for (int32_t c = tid; c < C; c += kRoundThreads) ws.zcls[b * C + c] = lc[c];
+    if (tid == 0) ws.lse[b] = lse;
+  }
 }
 
 constexpr int kOutLoads = 4;          // float4 loads in flight per thread (prior_out_kernel)
@@ -1694,82 +1801,6 @@ __global__ __launch_bounds__(kPriorOutThreads) void prior_out_kernel(
   }
 }
 
-
-// Member-list output, grid (ceil(V / 4096), rows): block g rewrites the
-// 4096-token member chunk g of its row.  The chunk is staged in LDS as -inf;
-// the threads take the chunk's member list (Cap slots, 0xFFFFFFFF empty),
-// gather the logits of the members whose class has a finite lookahead value
-// from the row's state and write x - lse + alpha * z there (EOS: its log
-// softmax when the state accepts); the chunk then goes out as coalesced
-// float4 non-temporal stores (every 128-byte line written whole; nothing
-// reads the rows again in this call).  Needs vocab, ld and the logits
-// aligned to 4 floats.
-template <int Cap>
-__global__ __launch_bounds__(kPriorOutThreads) void prior_out_list_kernel(
-    float* __restrict__ logits, int64_t ld, int64_t V, const uint32_t* __restrict__ members, int32_t C,
-    const float* __restrict__ lse_in, const float* __restrict__ zcls, int32_t S,
-    const uint8_t* __restrict__ accept, int32_t eos, const int32_t* __restrict__ states,
-    const int64_t* __restrict__ slots, float alpha, int32_t* __restrict__ err) {
-  constexpr int kSlots = Cap / kPriorOutThreads;
-  constexpr int kGroups = BPD_SOFT_MEMBER_CHUNK / 4 / kPriorOutThreads;  // float4 groups per thread
-  __shared__ float4 outs[BPD_SOFT_MEMBER_CHUNK / 4];
-  __shared__ float zs[kLdsClasses];
-  const int64_t b = blockIdx.y;
-  const int64_t base = int64_t(blockIdx.x) * BPD_SOFT_MEMBER_CHUNK;
-  const int32_t s = states[slots ? slots[b] : b];
-  float* row = logits + b * ld;
-  const float4 ninf = make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
-  if (s < 0 || s >= S) {
-    if (s >= S && err && blockIdx.x == 0 && threadIdx.x == 0) atomicOr(err, BPD_FLAG_STATE_RANGE);
-#pragma unroll
-    for (int q = 0; q < kGroups; ++q) {
-      const int64_t t = base + (int64_t(q) * kPriorOutThreads + threadIdx.x) * 4;
-      if (t < V) *reinterpret_cast<float4*>(row + t) = ninf;
-    }
-    return;
-  }
-  uint32_t mm[kSlots];
-#pragma unroll
-  for (int j = 0; j < kSlots; ++j) mm[j] = members[int64_t(blockIdx.x) * Cap + j * kPriorOutThreads + threadIdx.x];
-  const float* zrow = zcls + b * C;
-  for (int32_t c = threadIdx.x; c < C; c += kPriorOutThreads) zs[c] = zrow[c];
-#pragma unroll
-  for (int q = 0; q < kGroups; ++q) outs[q * kPriorOutThreads + threadIdx.x] = ninf;
-  const float lse = lse_in[b];
-  const bool acc_s = accept[s] != 0;
-  __syncthreads();
-  // gathers of the members that keep a finite value (all issued, then used)
-  float xv[kSlots], zv[kSlots];
-#pragma unroll
-  for (int j = 0; j < kSlots; ++j) {
-    zv[j] = -INFINITY;
-    if (mm[j] != 0xFFFFFFFFu) {
-      const int64_t t = base + int64_t(mm[j] >> 16);
-      if (t != eos) zv[j] = zs[mm[j] & 0xFFFFu];
-    }
-    xv[j] = zv[j] != -INFINITY ? row[base + int64_t(mm[j] >> 16)] : 0.0f;
-  }
-  float* of = reinterpret_cast<float*>(outs);
-#pragma unroll
-  for (int j = 0; j < kSlots; ++j) {
-    if (zv[j] != -INFINITY) {
-      const float lp = xv[j] - lse;
-      of[mm[j] >> 16] = alpha != 0.0f ? fmaf(alpha, zv[j], lp) : lp;
-    }
-  }
-  if (threadIdx.x == 0 && eos >= base && eos < base + BPD_SOFT_MEMBER_CHUNK && eos < V)
-    of[eos - base] = acc_s ? row[eos] - lse : -INFINITY;
-  __syncthreads();
-#pragma unroll
-  for (int q = 0; q < kGroups; ++q) {
-    const int64_t t = base + (int64_t(q) * kPriorOutThreads + threadIdx.x) * 4;
-    if (t < V) {
-      const float4 o = outs[q * kPriorOutThreads + threadIdx.x];
-      __builtin_nontemporal_store(F4v{o.x, o.y, o.z, o.w}, reinterpret_cast<F4v*>(row + t));
-    }
-  }
-}
-
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 bool force_pieces() {
@@ -1807,6 +1838,12 @@ extern "C" size_t bpd_soft_prior_workspace_bytes(int64_t rows, int64_t vocab, in
   return m > w ? m : w;
 }
 
+extern "C" size_t bpd_soft_prior_workspace_full(int64_t rows, int64_t vocab, const BpdSoftClasses* classes) {
+  if (!classes || rows <= 0 || vocab <= 0) return 0;
+  return align256(bpd_soft_prior_workspace_bytes(rows, vocab, classes->num_classes, classes->num_pieces)) +
+         prior_vals_bytes(rows, vocab, classes->chunk_members && classes->chunk_cap > 0 ? classes->chunk_cap : 0);
+}
+
 namespace {
 
 // The prior lookahead on a caller-provided workspace (both entry points).
@@ -1834,8 +1871,7 @@ int soft_prior_impl(float* logits, int64_t rows, int64_t vocab, int64_t ld, int3
   // output pass over each 4096-token chunk's members (the default)
   const bool list_ok = std::strcmp(choice, "list") == 0 && cls.chunk_members != nullptr &&
                        cls.num_classes < 65535 &&
-                       (cls.chunk_cap == 256 || cls.chunk_cap == 512 || cls.chunk_cap == 1024) &&
-                       vocab % 4 == 0 && ld % 4 == 0 && aligned16(logits);
+                       (cls.chunk_cap == 256 || cls.chunk_cap == 512 || cls.chunk_cap == 1024);
   const bool wide_ok = (std::strcmp(choice, "wave") == 0 && cls.token_class16 != nullptr &&
                         cls.num_classes < 65535 && vocab % 4 == 0 && ld % 4 == 0 && aligned16(logits) &&
                         (reinterpret_cast<uintptr_t>(cls.token_class16) & 7u) == 0) ||
@@ -1849,7 +1885,13 @@ int soft_prior_impl(float* logits, int64_t rows, int64_t vocab, int64_t ld, int3
   BPD_REQUIRE(lds <= kPriorMaxLds, "%d states and %d classes exceed the LDS budget", num_states,
               cls.num_classes);
   hipStream_t st = as_stream(stream);
-  const PriorWs ws = prior_ws(workspace, rows, pl, cls.num_classes, cls.num_pieces);
+  PriorWs ws = prior_ws(workspace, rows, pl, cls.num_classes, cls.num_pieces);
+  const int64_t nchunks = (vocab + BPD_SOFT_MEMBER_CHUNK - 1) / BPD_SOFT_MEMBER_CHUNK;
+  // room for the members' logits: the output then reads them in order instead
+  // of gathering them from the rows
+  const size_t common = align256(bpd_soft_prior_workspace_bytes(rows, vocab, cls.num_classes, cls.num_pieces));
+  if (workspace_bytes >= common + prior_vals_bytes(rows, vocab, cls.chunk_cap))
+    ws.vals = reinterpret_cast<float*>(static_cast<char*>(workspace) + common);
   const bool vec = vocab % 4 == 0 && ld % 4 == 0 && aligned16(logits) && aligned16(cls.token_class);
   if (pl.class_stats) {
     const dim3 grid = dim3(unsigned(pl.G), unsigned(rows));
@@ -1866,15 +1908,13 @@ int soft_prior_impl(float* logits, int64_t rows, int64_t vocab, int64_t ld, int3
                          (cls.chunk_cap == 256 || cls.chunk_cap == 512 || cls.chunk_cap == 1024);
     const size_t mlds = size_t(kStatChunk) * sizeof(float) + size_t(cls.num_classes) * 8;
     const size_t llds = (size_t(kWideChunk) + size_t(kPriorThreads / 64 + 2) * cls.num_classes) * 4;
-    if (pl.wide && list_ok && cls.chunk_cap == 256)
-      prior_stats_list_kernel<256><<<grid, kPriorThreads, llds, st>>>(logits, ld, vocab, cls.chunk_members,
-                                                                      cls.num_classes, ws, queued);
-    else if (pl.wide && list_ok && cls.chunk_cap == 512)
-      prior_stats_list_kernel<512><<<grid, kPriorThreads, llds, st>>>(logits, ld, vocab, cls.chunk_members,
-                                                                      cls.num_classes, ws, queued);
-    else if (pl.wide && list_ok)
-      prior_stats_list_kernel<1024><<<grid, kPriorThreads, llds, st>>>(logits, ld, vocab, cls.chunk_members,
-                                                                       cls.num_classes, ws, queued);
+#define BPD_PRIOR_STATS_LIST(CAP)                                                                       \
+  prior_stats_list_kernel<CAP><<<grid, kPriorThreads, llds, st>>>(logits, ld, vocab, cls.chunk_members, \
+                                                                  cls.num_classes, eos_id, ws, queued)
+    if (pl.wide && list_ok && cls.chunk_cap == 256) BPD_PRIOR_STATS_LIST(256);
+    else if (pl.wide && list_ok && cls.chunk_cap == 512) BPD_PRIOR_STATS_LIST(512);
+    else if (pl.wide && list_ok) BPD_PRIOR_STATS_LIST(1024);
+#undef BPD_PRIOR_STATS_LIST
     else if (pl.wide)
       prior_stats_wave_kernel<<<grid, kPriorThreads, size_t(cls.num_classes) * (kPriorThreads / 64 + 2) * 4, st>>>(
           logits, ld, vocab, cls.token_class16, cls.num_classes, ws, queued);
@@ -1900,15 +1940,28 @@ int soft_prior_impl(float* logits, int64_t rows, int64_t vocab, int64_t ld, int3
     }
   }
   BPD_LAUNCHED();
-#define BPD_PRIOR_ROUNDS(LDSP, CLS)                                                                  \
-  prior_rounds_kernel<LDSP, CLS><<<unsigned(rows), kRoundThreads, lds, st>>>(                       \
-      logits, ld, num_states, pl.G, cls, accept, live, eos_id, states, slots, k - 1, ws)
-  if (pairs_in_lds && pl.class_stats) BPD_PRIOR_ROUNDS(true, true);
-  else if (pairs_in_lds) BPD_PRIOR_ROUNDS(true, false);
-  else if (pl.class_stats) BPD_PRIOR_ROUNDS(false, true);
-  else BPD_PRIOR_ROUNDS(false, false);
+#define BPD_PRIOR_ROUNDS(LDSP, CLS, OUT)                                                             \
+  prior_rounds_kernel<LDSP, CLS, OUT><<<rgrid, kRoundThreads, rlds, st>>>(                          \
+      logits, ld, num_states, pl.G, cls, accept, live, eos_id, states, slots, k - 1, ws,            \
+      PriorOut{logits, vocab, alpha, err})
+  const bool list = list_ok && pl.class_stats;
+  dim3 rgrid = dim3(unsigned(rows));
+  size_t rlds = lds;
+  if (list) {
+    // two blocks per CU where the rows alone are fewer, at most one per chunk
+    const int64_t want = (2 * kComputeUnits + rows - 1) / rows;
+    rgrid = dim3(unsigned(std::min(want, nchunks)), unsigned(rows));
+    rlds = std::max(lds, size_t(cls.num_classes + 3) / 4 * 16 + 2 * size_t(BPD_SOFT_MEMBER_CHUNK) * 4);
+  }
+  if (list && pairs_in_lds) BPD_PRIOR_ROUNDS(true, true, true);
+  else if (list) BPD_PRIOR_ROUNDS(false, true, true);
+  else if (pairs_in_lds && pl.class_stats) BPD_PRIOR_ROUNDS(true, true, false);
+  else if (pairs_in_lds) BPD_PRIOR_ROUNDS(true, false, false);
+  else if (pl.class_stats) BPD_PRIOR_ROUNDS(false, true, false);
+  else BPD_PRIOR_ROUNDS(false, false, false);
 #undef BPD_PRIOR_ROUNDS
   BPD_LAUNCHED();
+  if (list) return BPD_OK;
   const dim3 ogrid = dim3(unsigned((vocab + 4 * kOutLoads * kPriorOutThreads - 1) /
                                    (4 * kOutLoads * kPriorOutThreads)),
                           unsigned(rows));
@@ -1919,22 +1972,13 @@ int soft_prior_impl(float* logits, int64_t rows, int64_t vocab, int64_t ld, int3
   prior_out_kernel<VEC, ZL, NW><<<ogrid, kPriorOutThreads, 0, st>>>(                            \
       logits, ld, vocab, cls.token_class, cls.token_class16, cls.num_classes, ws.lse, ws.zcls,   \
       num_states, accept, eos_id, states, slots, alpha, err)
-  const dim3 lgrid = dim3(unsigned((vocab + BPD_SOFT_MEMBER_CHUNK - 1) / BPD_SOFT_MEMBER_CHUNK), unsigned(rows));
-#define BPD_PRIOR_OUT_LIST(CAP)                                                                      \
-  prior_out_list_kernel<CAP><<<lgrid, kPriorOutThreads, 0, st>>>(                                   \
-      logits, ld, vocab, cls.chunk_members, cls.num_classes, ws.lse, ws.zcls, num_states, accept, eos_id, \
-      states, slots, alpha, err)
-  if (list_ok && pl.class_stats && cls.chunk_cap == 256) BPD_PRIOR_OUT_LIST(256);
-  else if (list_ok && pl.class_stats && cls.chunk_cap == 512) BPD_PRIOR_OUT_LIST(512);
-  else if (list_ok && pl.class_stats) BPD_PRIOR_OUT_LIST(1024);
-  else if (onarrow && z_lds) BPD_PRIOR_OUT(true, true, true);
+  if (onarrow && z_lds) BPD_PRIOR_OUT(true, true, true);
   else if (onarrow) BPD_PRIOR_OUT(true, false, true);
   else if (vec && z_lds) BPD_PRIOR_OUT(true, true, false);
   else if (vec) BPD_PRIOR_OUT(true, false, false);
   else if (z_lds) BPD_PRIOR_OUT(false, true, false);
   else BPD_PRIOR_OUT(false, false, false);
 #undef BPD_PRIOR_OUT
-#undef BPD_PRIOR_OUT_LIST
   BPD_LAUNCHED();
   return BPD_OK;
 }

@@ -108,7 +108,7 @@ class SoftClasses:
         """Workspace for ``rows`` rows, kept per stream so a step allocates
         nothing once it has run at this size."""
         vocab = int(self.token_class.numel())
-        need = int(lib().bpd_soft_prior_workspace_bytes(rows, vocab, self.num_classes, self.num_pieces))
+        need = int(lib().bpd_soft_prior_workspace_full(rows, vocab, C.byref(self.c_struct())))
         key = (device, stream)
         ws = self._ws.get(key)
         if ws is None or ws.numel() < need:

@@ -514,7 +514,9 @@ int bpd_host_soft_apply(void* logits, int dtype, int64_t rows, int64_t vocab, in
  * with token_class16 set its statistics pass reads the narrow map instead of
  * token_class.
  * Workspace: bpd_soft_prior_workspace_bytes(rows, vocab, num_classes, num_pieces)
- * bytes (no initial contents needed; calls that overlap on one workspace race).
+ * bytes (no initial contents needed; calls that overlap on one workspace race);
+ * with the bpd_soft_prior_workspace_full bytes the output pass reads the
+ * members' logits from there instead of gathering them from the rows.
  */
 typedef struct BpdSoftClasses {
   int32_t num_classes, num_members, num_pieces, num_pairs;
@@ -545,6 +547,7 @@ int bpd_host_soft_classes(const int32_t* tok_next, int32_t num_states, int64_t v
                           BpdSoftClasses* out);
 size_t bpd_soft_prior_workspace_bytes(int64_t rows, int64_t vocab, int32_t num_classes,
                                       int32_t num_pieces);
+size_t bpd_soft_prior_workspace_full(int64_t rows, int64_t vocab, const BpdSoftClasses* classes);
 int bpd_soft_prior(float* logits, int64_t rows, int64_t vocab, int64_t ld, int32_t num_states,
                    const uint8_t* accept, const uint8_t* live, int32_t eos_id,
                    const int32_t* states, const int64_t* slots, const BpdSoftClasses* classes,

@@ -3,6 +3,8 @@
 
 from __future__ import annotations
 
+from dataclasses import replace
+
 import numpy as np
 import pytest
 import torch
@@ -249,6 +251,40 @@ def test_prior_unaligned_vocab(dev):
     ops.apply_soft_prior_(w[:, :V], fsa.to(dev), st.to(dev), 4, 1.0)
     assert close(w[:, :V].cpu().double().numpy(), want)
     assert torch.equal(w[:, V:].cpu(), wide[:, V:])
+
+
+@pytest.mark.parametrize("rows,vocab,pad,offset", [
+    (1, 4095, 0, 0), (3, 4096, 1, 1), (2, 4097, 2, 3), (5, 8191, 0, 2), (1, 8193, 3, 0), (600, 4099, 0, 0),
+])
+@pytest.mark.parametrize("eos", [0, 4094, -1])
+def test_prior_row_shapes(dev, rows, vocab, pad, offset, eos):
+    """Member-list kernels at the edges of their chunks (4096 tokens a stage,
+    8192 a statistics block), at every alignment of the rows, with more rows
+    than blocks in flight; nothing outside the rows' columns is written."""
+    S, C = 6, 9
+    rng = np.random.default_rng(vocab + rows)
+    columns = rng.integers(-1, S, size=(S, C + 1))
+    columns[:, C] = -1  # tokens rejected everywhere: most of them, at most 1024 a chunk are not
+    tn = columns[:, np.where(rng.random(vocab) < 0.1, rng.integers(0, C, size=vocab), C)]
+    tn[:, eos] = np.where(np.arange(S) % 2 == 0, np.arange(S), -1)
+    fsa = FsaTensors.build("a", TOY_VOCAB).densify()
+    fsa = replace(fsa, tok_next=torch.from_numpy(tn).to(torch.int32), trans=torch.zeros(S, dtype=torch.int32),
+                  accept=(torch.arange(S) % 2 == 0).to(torch.uint8), live=torch.ones(S, dtype=torch.uint8),
+                  num_symbols=1, eos_id=eos % vocab, allow_bits=None, soft_classes=None)
+    st = torch.from_numpy(rng.integers(-1, S, size=rows)).to(torch.int32)
+    flat = torch.randn(offset + rows * (vocab + pad), generator=torch.Generator().manual_seed(rows)) * 3
+    flat[rng.random(flat.numel()) < 0.01] = -float("inf")
+    view = flat[offset:].view(rows, vocab + pad)[:, :vocab]
+    want = OS.prior_lookahead(view.double().numpy(), tn, np.ones(S, dtype=np.uint8), np.arange(S) % 2 == 0,
+                              eos % vocab, st.numpy(), 3, 0.5)
+    got = flat.to(dev)
+    fd = fsa.to(dev)
+    assert fd.ensure_soft_classes().chunk_cap > 0
+    out = got[offset:].view(rows, vocab + pad)[:, :vocab]
+    ops.apply_soft_prior_(out, fd, st.to(dev), 3, 0.5)
+    assert close(out.cpu().double().numpy(), want)
+    view.copy_(out.cpu())
+    assert torch.equal(got.cpu(), flat)
 
 
 @pytest.fixture(scope="module")
