@@ -1579,11 +1579,11 @@ __device__ __forceinline__ void prior_out_chunks(const PriorOut& out, int64_t ld
 // Out: the member-list output follows in the same launch, grid (splits, rows),
 // every block of a row running its rounds (the EOS logit then comes from the
 // statistics: another block of the row may have written its output already).
-// [128, 151936], 71 states, k = 4: ROUNDS_US us, where a launch of one block
-// per row took 10.0 and a gathering output launch after it 21.4; the rounds
-// are a chain of LDS latencies that leaves a block room for a second one.
+// [128, 151936], 71 states, k = 4: 24.0 us (9.6 until the rounds are done),
+// where a launch of one block per row took 10.0 and a gathering output launch
+// after it 21.4; two blocks per CU, whose rounds share its LDS, 24.9.
 template <bool PairsInLds, bool ClassStats, bool Out>
-__global__ __launch_bounds__(kRoundThreads, 8) void prior_rounds_kernel(
+__global__ __launch_bounds__(kRoundThreads) void prior_rounds_kernel(
     const float* logits, int64_t ld, int32_t S, int G, BpdSoftClasses cls,
     const uint8_t* __restrict__ accept, const uint8_t* __restrict__ live, int32_t eos,
     const int32_t* __restrict__ states, const int64_t* __restrict__ slots, int32_t rounds,
@@ -1948,8 +1948,8 @@ int soft_prior_impl(float* logits, int64_t rows, int64_t vocab, int64_t ld, int3
   dim3 rgrid = dim3(unsigned(rows));
   size_t rlds = lds;
   if (list) {
-    // two blocks per CU where the rows alone are fewer, at most one per chunk
-    const int64_t want = (2 * kComputeUnits + rows - 1) / rows;
+    // one block per CU where the rows alone are fewer, at most one per chunk
+    const int64_t want = (kComputeUnits + rows - 1) / rows;
     rgrid = dim3(unsigned(std::min(want, nchunks)), unsigned(rows));
     rlds = std::max(lds, size_t(cls.num_classes + 3) / 4 * 16 + 2 * size_t(BPD_SOFT_MEMBER_CHUNK) * 4);
   }
