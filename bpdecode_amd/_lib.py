@@ -78,6 +78,9 @@ _SIGNATURES = {
     "bpd_dense_apply_mask": (cint, [vp, cint, i64, i64, i64, vp, i32, vp, vp, vp, i64, f64, vp, vp]),
     "bpd_dense_apply_mask_bits": (cint, [vp, cint, i64, i64, i64, vp, i64, i32, vp, vp, vp, i64, f64,
                                          vp, vp]),
+    "bpd_dense_apply_mask_padded": (cint, [vp, cint, i64, i64, i64, i64, vp, i64, i32, vp, vp, vp, i64, f64,
+                                           vp, vp]),
+    "bpd_dense_advance_strided": (cint, [vp, i32, i64, vp, vp, vp, i64, vp, cint, i64, i64, vp, cint, vp, vp]),
     "bpd_dense_advance": (cint, [vp, i32, i64, vp, vp, vp, i64, vp, cint, i64, vp, cint, vp, vp]),
     "bpd_dense_compute_mask": (cint, [vp, i32, i64, vp, vp, i64, vp, vp, vp]),
     "bpd_build_reachability": (cint, [vp, i32, i32, vp, vp, vp]),
@@ -90,6 +93,8 @@ _SIGNATURES = {
     "bpd_fsa_compute_mask": (cint, [C.POINTER(FsaTableC), vp, vp, i64, vp, vp, vp]),
     "bpd_fsa_advance": (cint, [C.POINTER(FsaTableC), vp, vp, vp, i64, vp, cint, i64, vp, cint, vp,
                                 vp]),
+    "bpd_fsa_advance_strided": (cint, [C.POINTER(FsaTableC), vp, vp, vp, i64, vp, cint, i64, i64, vp, cint, vp,
+                                        vp]),
     "bpd_host_dense_apply_mask": (cint, [vp, cint, i64, i64, i64, vp, i32, vp, vp, f64]),
     "bpd_host_dense_apply_mask_bits": (cint, [vp, cint, i64, i64, i64, vp, i64, i32, vp, vp, f64]),
     "bpd_host_dense_advance": (cint, [vp, i32, i64, vp, vp, vp, cint, i64, vp, cint]),

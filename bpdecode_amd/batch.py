@@ -206,11 +206,11 @@ class ConstraintBatch:
             self._f_mask = lib().bpd_dense_apply_mask_bits
             if tn is not None:
                 self._tn_ptr = tn.data_ptr()
-                self._f_advance = lib().bpd_dense_advance
+                self._f_advance = lib().bpd_dense_advance_strided
                 self._walk_table = None
             else:
                 self._walk_table = C.byref(self.fsa.c_fsa_table())
-                self._f_advance = lib().bpd_fsa_advance
+                self._f_advance = lib().bpd_fsa_advance_strided
 
     # --- pool -----------------------------------------------------------
     def _unstage(self) -> None:
@@ -415,6 +415,30 @@ class ConstraintBatch:
             apply_mask_(logits, self.fsa, pool[slots], neg_inf)
         return logits
 
+    def apply_mask_padded(self, seq_ids: Sequence[Hashable], scores: torch.Tensor,
+                          neg_inf: float = float("-inf")) -> torch.Tensor:
+        """In place: ``apply_mask`` on the first ``vocab`` columns of
+        ``scores`` [len(seq_ids), columns], and ``neg_inf`` in the columns
+        beyond them (a padded lm_head); one launch on the device."""
+        V = self.fsa.vocab_size
+        code = _DENSE_CODES.get(scores.dtype)
+        B, cols = scores.shape
+        if (self._fast and self.cache is None and code is not None and B == len(seq_ids) and cols >= V
+                and scores.device == self.device and (scores.stride(1) == 1 or cols <= 1)
+                and (B <= 1 or scores.stride(0) >= cols)):
+            slots, pend, n = self._slots_fused(seq_ids, True)
+            check(lib().bpd_dense_apply_mask_padded(
+                scores.data_ptr(), code, B, V, cols, scores.stride(0) if B > 1 else cols, self._bits_ptr, self._W,
+                self._S, self._pool_ptr, slots, pend, n, float(neg_inf), self._err_ptr,
+                _lib.stream_of(self.device)))
+            if n:
+                self._launched()
+            return scores
+        if scores.shape[1] > V:
+            scores[:, V:] = neg_inf
+        self.apply_mask(seq_ids, scores[:, :V], neg_inf)
+        return scores
+
     def _fast_logits(self, logits: torch.Tensor, rows: int) -> bool:
         """Logits the device dense path takes as they are: [rows, vocab] on
         this device with unit column stride."""
@@ -423,6 +447,7 @@ class ConstraintBatch:
         B, V = logits.shape
         return B == rows and V == self._V and (logits.stride(1) == 1 or V <= 1) and (
             B <= 1 or logits.stride(0) >= V)
+
 
     def apply_soft(self, seq_ids: Sequence[Hashable], logits: torch.Tensor, alpha: float = 1.0):
         """In place: ``logits += alpha * lookahead[state]`` (and mask)."""
@@ -478,7 +503,7 @@ class ConstraintBatch:
         does."""
         B = len(seq_ids)
         if (self._fast and tokens.device == self.device and tokens.dim() == 1
-                and tokens.numel() == B and tokens.is_contiguous()):
+                and tokens.numel() == B):
             code = _TOKEN_CODES.get(tokens.dtype)
             if code is not None:
                 slots, pend, n = self._slots_fused(seq_ids, B <= _COMMIT_FUSED_ROWS)
@@ -486,12 +511,13 @@ class ConstraintBatch:
                 if self._walk_table is None:
                     check(self._f_advance(
                         self._tn_ptr, self._S, self._V, self._pool_ptr, slots, pend, n,
-                        tokens.data_ptr(), code, B, out.data_ptr(), 1, self._err_ptr,
+                        tokens.data_ptr(), code, tokens.stride(0), B, out.data_ptr(), 1, self._err_ptr,
                         _lib.stream_of(self.device)))
                 else:
                     check(self._f_advance(
                         self._walk_table, self._pool_ptr, slots, pend, n, tokens.data_ptr(),
-                        code, B, out.data_ptr(), 1, self._err_ptr, _lib.stream_of(self.device)))
+                        code, tokens.stride(0), B, out.data_ptr(), 1, self._err_ptr,
+                        _lib.stream_of(self.device)))
                 if n:
                     self._launched()
                 return out

@@ -164,7 +164,7 @@ __global__ __launch_bounds__(kAdvThreads) void dense_advance_block_kernel(
     const int32_t* __restrict__ tok_next, int32_t num_states, int64_t vocab,
     int32_t* __restrict__ states, const int64_t* __restrict__ slots,
     const int64_t* __restrict__ pending, int32_t num_pending, const void* __restrict__ tokens,
-    int tok_dtype, int64_t rows, int32_t* __restrict__ next_out, int write_back,
+    int tok_dtype, int64_t tok_stride, int64_t rows, int32_t* __restrict__ next_out, int write_back,
     int32_t* __restrict__ err) {
   __shared__ int64_t pslot[BPD_MAX_FUSED_PENDING];
   __shared__ int32_t pval[BPD_MAX_FUSED_PENDING];
@@ -176,7 +176,7 @@ __global__ __launch_bounds__(kAdvThreads) void dense_advance_block_kernel(
   for (int i = 0; i < kAdvPerThread; ++i) {
     const int64_t b = int64_t(i) * kAdvThreads + threadIdx.x;
     slot[i] = b < rows ? (slots ? slots[b] : b) : -1;
-    tk[i] = b < rows ? read_token(tokens, tok_dtype, b) : 0;
+    tk[i] = b < rows ? read_token(tokens, tok_dtype, b * tok_stride) : 0;
   }
   int32_t st[kAdvPerThread];
 #pragma unroll
@@ -213,12 +213,12 @@ __global__ void dense_advance_gather_kernel(const int32_t* __restrict__ tok_next
                                             const int32_t* __restrict__ states,
                                             const int64_t* __restrict__ slots,
                                             const void* __restrict__ tokens, int tok_dtype,
-                                            int64_t rows, int32_t* __restrict__ next_out,
-                                            int32_t* __restrict__ err) {
+                                            int64_t tok_stride, int64_t rows,
+                                            int32_t* __restrict__ next_out, int32_t* __restrict__ err) {
   const int64_t b = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (b >= rows) return;
   const int64_t slot = slots ? slots[b] : b;
-  next_out[b] = advance_one(tok_next, num_states, vocab, states[slot], tokens, tok_dtype, b, err);
+  next_out[b] = advance_one(tok_next, num_states, vocab, states[slot], tokens, tok_dtype, b * tok_stride, err);
 }
 
 __global__ void dense_scatter_kernel(int32_t* __restrict__ states, const int64_t* __restrict__ slots,
@@ -531,11 +531,32 @@ extern "C" int bpd_dense_apply_mask_bits(void* logits, int dtype, int64_t rows, 
                      slots, pending, num_pending, neg_inf, err, stream);
 }
 
+extern "C" int bpd_dense_apply_mask_padded(void* logits, int dtype, int64_t rows, int64_t vocab, int64_t cols,
+                                           int64_t ld, const uint32_t* allow_bits, int64_t words,
+                                           int32_t num_states, int32_t* states, const int64_t* slots,
+                                           const int64_t* pending, int64_t num_pending, double neg_inf,
+                                           int32_t* err, void* stream) {
+  BPD_REQUIRE(words == (vocab + 31) / 32, "allow-bit rows must hold ceil(vocab/32) words");
+  BPD_REQUIRE(cols >= vocab, "fewer columns than tokens");
+  // a column past the table's words, or past vocab in its last one, is rejected
+  return launch_fill(logits, dtype, rows, cols, ld, allow_bits, words, true, num_states, states,
+                     slots, pending, num_pending, neg_inf, err, stream);
+}
+
 extern "C" int bpd_dense_advance(const int32_t* tok_next, int32_t num_states, int64_t vocab,
                                  int32_t* states, const int64_t* slots, const int64_t* pending,
                                  int64_t num_pending, const void* tokens, int token_dtype,
                                  int64_t rows, int32_t* next_out, int write_back, int32_t* err,
                                  void* stream) {
+  return bpd_dense_advance_strided(tok_next, num_states, vocab, states, slots, pending, num_pending, tokens,
+                                   token_dtype, 1, rows, next_out, write_back, err, stream);
+}
+
+extern "C" int bpd_dense_advance_strided(const int32_t* tok_next, int32_t num_states, int64_t vocab,
+                                         int32_t* states, const int64_t* slots, const int64_t* pending,
+                                         int64_t num_pending, const void* tokens, int token_dtype,
+                                         int64_t token_stride, int64_t rows, int32_t* next_out,
+                                         int write_back, int32_t* err, void* stream) {
   BPD_REQUIRE(token_dtype_ok(token_dtype), "unknown token dtype code %d", token_dtype);
   BPD_REQUIRE(num_states > 0 && vocab > 0, "empty tok_next table");
   BPD_REQUIRE(rows >= 0, "negative row count");
@@ -552,8 +573,8 @@ extern "C" int bpd_dense_advance(const int32_t* tok_next, int32_t num_states, in
   if (rows <= int64_t(kAdvThreads) * kAdvPerThread) {
     dense_advance_block_kernel<<<1, kAdvThreads, 0, s>>>(tok_next, num_states, vocab, states,
                                                          slots, pending, int32_t(num_pending),
-                                                         tokens, token_dtype, rows, next_out,
-                                                         write_back, err);
+                                                         tokens, token_dtype, token_stride, rows,
+                                                         next_out, write_back, err);
     BPD_LAUNCHED();
     return BPD_OK;
   }
@@ -562,7 +583,7 @@ extern "C" int bpd_dense_advance(const int32_t* tok_next, int32_t num_states, in
               kAdvThreads * kAdvPerThread);
   const unsigned g = unsigned((rows + 255) / 256);
   dense_advance_gather_kernel<<<g, 256, 0, s>>>(tok_next, num_states, vocab, states, slots,
-                                                tokens, token_dtype, rows, next_out, err);
+                                                tokens, token_dtype, token_stride, rows, next_out, err);
   BPD_LAUNCHED();
   if (write_back) {
     dense_scatter_kernel<<<g, 256, 0, s>>>(states, slots, next_out, rows);

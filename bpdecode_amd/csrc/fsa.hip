@@ -233,12 +233,12 @@ __global__ __launch_bounds__(kFsaThreads) void fsa_mask_kernel(
 // out of range and states >= S give -1 and set the error flags).
 __global__ __launch_bounds__(kFsaAdvThreads) void fsa_advance_kernel(
     FsaView f, const int32_t* __restrict__ states, const int64_t* __restrict__ slots,
-    const void* __restrict__ tokens, int tok_dtype, int64_t rows, int32_t* __restrict__ next_out,
+    const void* __restrict__ tokens, int tok_dtype, int64_t tok_stride, int64_t rows, int32_t* __restrict__ next_out,
     int32_t* __restrict__ err) {
   const int64_t b = int64_t(blockIdx.x) * kFsaAdvThreads + threadIdx.x;
   if (b >= rows) return;
   const int32_t s = states[slots ? slots[b] : b];
-  int64_t t = read_token(tokens, tok_dtype, b);
+  int64_t t = read_token(tokens, tok_dtype, b * tok_stride);
   if (t < 0) t += f.V;
   int32_t res = -1;
   if (t < 0 || t >= f.V) {
@@ -283,7 +283,7 @@ template <bool InLds>
 __global__ __launch_bounds__(kFsaCommitThreads) void fsa_advance_block_kernel(
     FsaView f, int32_t* __restrict__ states, const int64_t* __restrict__ slots,
     const int64_t* __restrict__ pending, int32_t num_pending, const void* __restrict__ tokens,
-    int tok_dtype, int64_t rows, int32_t* __restrict__ next_out, int write_back,
+    int tok_dtype, int64_t tok_stride, int64_t rows, int32_t* __restrict__ next_out, int write_back,
     int32_t* __restrict__ err) {
   extern __shared__ __align__(16) uint16_t tr16[];
   __shared__ int64_t pslot[BPD_MAX_FUSED_PENDING];
@@ -297,7 +297,7 @@ __global__ __launch_bounds__(kFsaCommitThreads) void fsa_advance_block_kernel(
     tk[i] = 0;
     if (b < rows) {
       slot[i] = slots ? slots[b] : b;
-      tk[i] = read_token(tokens, tok_dtype, b);
+      tk[i] = read_token(tokens, tok_dtype, b * tok_stride);
     }
   }
   const int64_t n = int64_t(f.S) * f.NS;
@@ -547,6 +547,14 @@ extern "C" int bpd_fsa_advance(const BpdFsaTable* table, int32_t* states, const 
                                const int64_t* pending, int64_t num_pending, const void* tokens,
                                int token_dtype, int64_t rows, int32_t* next_out, int write_back,
                                int32_t* err, void* stream) {
+  return bpd_fsa_advance_strided(table, states, slots, pending, num_pending, tokens, token_dtype, 1, rows,
+                                 next_out, write_back, err, stream);
+}
+
+extern "C" int bpd_fsa_advance_strided(const BpdFsaTable* table, int32_t* states, const int64_t* slots,
+                                       const int64_t* pending, int64_t num_pending, const void* tokens,
+                                       int token_dtype, int64_t token_stride, int64_t rows,
+                                       int32_t* next_out, int write_back, int32_t* err, void* stream) {
   if (int rc = check_fsa(table)) return rc;
   BPD_REQUIRE(token_dtype_ok(token_dtype), "unknown token dtype code %d", token_dtype);
   BPD_REQUIRE(table->vocab > 0, "empty vocabulary");
@@ -571,12 +579,12 @@ extern "C" int bpd_fsa_advance(const BpdFsaTable* table, int32_t* states, const 
                 "token records must be 16-byte aligned");
     if (staged && table->num_states < 65535 && lds <= kFsaCommitLds && lds <= room)
       fsa_advance_block_kernel<true><<<1, kFsaCommitThreads, lds, s>>>(
-          v, states, slots, pending, int32_t(num_pending), tokens, token_dtype, rows, next_out,
-          write_back, err);
+          v, states, slots, pending, int32_t(num_pending), tokens, token_dtype, token_stride, rows,
+          next_out, write_back, err);
     else
       fsa_advance_block_kernel<false><<<1, kFsaCommitThreads, 0, s>>>(
-          v, states, slots, pending, int32_t(num_pending), tokens, token_dtype, rows, next_out,
-          write_back, err);
+          v, states, slots, pending, int32_t(num_pending), tokens, token_dtype, token_stride, rows,
+          next_out, write_back, err);
     BPD_LAUNCHED();
     return BPD_OK;
   }
@@ -584,7 +592,8 @@ extern "C" int bpd_fsa_advance(const BpdFsaTable* table, int32_t* states, const 
   BPD_REQUIRE(num_pending == 0, "batches above %d rows take no queued writes",
               kFsaCommitThreads * kFsaCommitPerThread);
   const unsigned g = unsigned((rows + kFsaAdvThreads - 1) / kFsaAdvThreads);
-  fsa_advance_kernel<<<g, kFsaAdvThreads, 0, s>>>(v, states, slots, tokens, token_dtype, rows, next_out, err);
+  fsa_advance_kernel<<<g, kFsaAdvThreads, 0, s>>>(v, states, slots, tokens, token_dtype, token_stride, rows,
+                                              next_out, err);
   BPD_LAUNCHED();
   if (write_back) {
     fsa_scatter_kernel<<<g, kFsaAdvThreads, 0, s>>>(states, slots, next_out, rows);

@@ -100,6 +100,16 @@ int bpd_dense_apply_mask_bits(void* logits, int dtype, int64_t rows, int64_t voc
                               int32_t* states, const int64_t* slots, const int64_t* pending,
                               int64_t num_pending, double neg_inf, int32_t* err, void* stream);
 
+/* bpd_dense_apply_mask_padded: the same mask over logits of `cols` >= vocab
+ * columns (a padded lm_head): the columns past vocab are rejected in every
+ * row.  The bits past vocab in a table row's last word are zero, as the
+ * builders leave them (hf.py:106-113 masks those columns on its own). */
+int bpd_dense_apply_mask_padded(void* logits, int dtype, int64_t rows, int64_t vocab, int64_t cols,
+                                int64_t ld, const uint32_t* allow_bits, int64_t words,
+                                int32_t num_states, int32_t* states, const int64_t* slots,
+                                const int64_t* pending, int64_t num_pending, double neg_inf,
+                                int32_t* err, void* stream);
+
 /* bpd_dense_advance: nxt = state(b) < 0 ? -1 : tok_next[state(b), t(b)], where
  * t(b) is tokens[b] read per token_dtype (BPD_INDEX_I32, BPD_INDEX_I64, or
  * BPD_INDEX_I64_LOW32 for the int32 cast ConstraintBatch.commit applies,
@@ -116,6 +126,14 @@ int bpd_dense_advance(const int32_t* tok_next, int32_t num_states, int64_t vocab
                       int32_t* states, const int64_t* slots, const int64_t* pending,
                       int64_t num_pending, const void* tokens, int token_dtype, int64_t rows,
                       int32_t* next_out, int write_back, int32_t* err, void* stream);
+
+/* The same with row b's id at tokens[b * token_stride] (a column of the ids
+ * that generate() keeps). */
+int bpd_dense_advance_strided(const int32_t* tok_next, int32_t num_states, int64_t vocab,
+                              int32_t* states, const int64_t* slots, const int64_t* pending,
+                              int64_t num_pending, const void* tokens, int token_dtype,
+                              int64_t token_stride, int64_t rows, int32_t* next_out, int write_back,
+                              int32_t* err, void* stream);
 
 /* bpd_dense_compute_mask: packed allow bits from tok_next (bit t of row b set
  * iff state(b) >= 0 and tok_next[state(b), t] != -1).  Dense counterpart of
@@ -217,6 +235,12 @@ int bpd_fsa_advance(const BpdFsaTable* table, int32_t* states, const int64_t* sl
                     const int64_t* pending, int64_t num_pending, const void* tokens,
                     int token_dtype, int64_t rows, int32_t* next_out, int write_back,
                     int32_t* err, void* stream);
+
+/* The same with row b's id at tokens[b * token_stride]. */
+int bpd_fsa_advance_strided(const BpdFsaTable* table, int32_t* states, const int64_t* slots,
+                            const int64_t* pending, int64_t num_pending, const void* tokens,
+                            int token_dtype, int64_t token_stride, int64_t rows, int32_t* next_out,
+                            int write_back, int32_t* err, void* stream);
 
 /* Host (CPU-tensor) forms of the dense entry points. */
 int bpd_host_dense_apply_mask(void* logits, int dtype, int64_t rows, int64_t vocab, int64_t ld,

@@ -371,3 +371,47 @@ def test_packed_masks_from_the_allow_bit_table(dev, S, V):
     assert torch.equal(ops.compute_mask(fd, st.long()), want)
     other = replace(fd, live=torch.zeros_like(fd.live), accept=torch.zeros_like(fd.accept))
     assert not ops.compute_mask(other, st).any()
+
+
+@pytest.mark.parametrize("dense", [True, False])
+@pytest.mark.parametrize("rows", [1, 5, 4097])
+def test_generation_step_padded_columns_and_strided_ids(dev, dense, rows):
+    """What generate() hands over: scores with columns beyond the vocabulary,
+    and the last column of the ids.  Words that the vocabulary fills partly
+    and columns past the table's words are filled; ids at a stride commit
+    like a contiguous copy (both kernels), outside ids are flagged."""
+    _log(f"case padded columns dense={dense} rows={rows}")
+    fsa = FsaTensors.build("(a[012]*)+|b0", TOY_VOCAB, dense=dense).to(dev)
+    V = fsa.vocab_size
+    tn = torch.from_numpy(oracle_table(fsa))
+    rng = torch.Generator().manual_seed(rows)
+    batch = ConstraintBatch(fsa, capacity=rows, device=dev)
+    ids = list(range(rows))
+    for i in ids:
+        batch.add(i)
+    state = torch.full((rows,), fsa.start)
+    for step, (pad, extra) in enumerate([(0, 0), (1, 3), (15, 0), (16, 1), (2100, 0)]):
+        for dtype in (torch.float32, torch.bfloat16):
+            wide = torch.randn(rows, V + pad + extra, generator=rng).to(dtype)
+            got = wide.to(dev)
+            batch.apply_mask_padded(ids, got[:, :V + pad], -5.0)
+            allowed = torch.zeros(rows, V, dtype=torch.bool)
+            allowed[state >= 0] = tn[state[state >= 0]] != -1
+            want = wide.clone()
+            want[:, :V] = torch.where(allowed, wide[:, :V], torch.tensor(-5.0, dtype=dtype))
+            want[:, V:V + pad] = -5.0
+            assert torch.equal(got.cpu(), want), (step, dtype)
+        text = torch.randint(0, V, (rows, 3 + step), generator=rng, dtype=torch.int64 if step % 2 else torch.int32)
+        state = torch.where(state >= 0, tn[state.clamp(min=0), text[:, -1].long()], torch.tensor(-1))
+        assert batch.commit(ids, text.to(dev)[:, -1]).tolist() == state.tolist()
+        one = torch.randint(0, V, (1,), generator=rng)  # the same id for every row: stride 0
+        state = torch.where(state >= 0, tn[state.clamp(min=0), one.expand(rows)], torch.tensor(-1))
+        assert batch.commit(ids, one.to(dev).expand(rows)).tolist() == state.tolist()
+        if step == 2:
+            for i in ids[::2]:
+                batch.reset(i)
+            state[::2] = fsa.start
+    batch.check_errors()
+    batch.commit(ids, torch.full((rows, 2), V, device=dev)[:, -1])
+    with pytest.raises(IndexError):
+        batch.check_errors()
