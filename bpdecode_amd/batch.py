@@ -448,7 +448,6 @@ class ConstraintBatch:
         return B == rows and V == self._V and (logits.stride(1) == 1 or V <= 1) and (
             B <= 1 or logits.stride(0) >= V)
 
-
     def apply_soft(self, seq_ids: Sequence[Hashable], logits: torch.Tensor, alpha: float = 1.0):
         """In place: ``logits += alpha * lookahead[state]`` (and mask)."""
         if self.fsa.lookahead is None:

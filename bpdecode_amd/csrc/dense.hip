@@ -412,14 +412,15 @@ __global__ __launch_bounds__(256) void build_tok_next_kernel(
   out[int64_t(r) * vocab + t] = res;
 }
 
-// int32 symbol ids to bytes, and *bad |= 1 where one lies outside [0, 255].
+// int32 symbol ids to bytes, and *bad = 1 where one lies outside [0, 255]
+// (a plain store: `bad` may be host memory).
 __global__ __launch_bounds__(256) void narrow_symbols_kernel(const int32_t* __restrict__ sym, int64_t n,
                                                              uint8_t* __restrict__ out,
                                                              int32_t* __restrict__ bad) {
   const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   const int32_t v = i < n ? sym[i] : 0;
   if (i < n) out[i] = uint8_t(v);
-  if (__any(v < 0 || v > 255) && (threadIdx.x & 63) == 0) atomicOr(bad, 1);
+  if (__any(v < 0 || v > 255) && (threadIdx.x & 63) == 0) *bad = 1;
 }
 
 // Reachability (the live set of a DFA): live[s] = 1 iff an accepting state

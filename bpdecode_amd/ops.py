@@ -356,20 +356,33 @@ def _unit_stride_rows(logits: torch.Tensor) -> tuple[torch.Tensor, bool]:
 
 
 def _symbols_u8(fsa: FsaTensors) -> torch.Tensor:
+    sym, check_ids = _narrowed_symbols(fsa)
+    check_ids()
+    return sym
+
+
+def _narrowed_symbols(fsa: FsaTensors):
+    """(symbol ids as bytes, a call that raises if one lies outside [0, 255]).
+    On the device one pass narrows and checks, and the call waits for that
+    pass alone: work enqueued before the call runs meanwhile."""
     sym = fsa.symbols
     if sym.device.type == "cuda" and sym.dtype == torch.int32 and sym.numel():
-        # one pass narrows and checks; one read-back instead of a minimum's
-        # and a maximum's
         sym = sym.contiguous()
         out = torch.empty(sym.numel(), dtype=torch.uint8, device=sym.device)
-        bad = torch.zeros(1, dtype=torch.int32, device=sym.device)
+        bad = torch.zeros(1, dtype=torch.int32, pin_memory=True)  # the pass stores to it directly
         check(lib().bpd_narrow_symbols(ptr(sym), sym.numel(), ptr(out), ptr(bad), _lib.stream_of(sym.device)))
-        if int(bad):
-            raise RuntimeError("symbol-class ids must lie in [0, 255]")
-        return out
+        done = torch.cuda.current_stream(sym.device).record_event()
+
+        def check_ids() -> None:
+            done.synchronize()
+            if int(bad):
+                raise RuntimeError("symbol-class ids must lie in [0, 255]")
+
+        return out, check_ids
     if sym.numel() and (int(sym.min()) < 0 or int(sym.max()) > 255):
         raise RuntimeError("symbol-class ids must lie in [0, 255]")
-    return sym.to(torch.uint8).contiguous() if sym.numel() else torch.zeros(1, dtype=torch.uint8, device=sym.device)
+    sym = sym.to(torch.uint8).contiguous() if sym.numel() else torch.zeros(1, dtype=torch.uint8, device=sym.device)
+    return sym, lambda: None
 
 
 def build_reachability(trans: torch.Tensor, accept: torch.Tensor, num_symbols: int) -> torch.Tensor:
@@ -412,12 +425,16 @@ def build_token_transitions(fsa: FsaTensors, rows=None) -> torch.Tensor:
     acc = fsa.accept.contiguous()
     live = fsa.live.contiguous()
     offs = _i32(fsa.offsets)
-    sym = _symbols_u8(fsa)
+    sym, check_ids = _narrowed_symbols(fsa)
     eos = fsa.eos_id if fsa.eos_id is not None else -1
     args = (ptr(trans), S, M, fsa.dead, ptr(acc), ptr(live), ptr(offs), ptr(sym), V, eos,
             ptr(row_states), n, ptr(out))
     if dev.type == "cuda":
-        check(lib().bpd_build_tok_next(*args, _lib.stream_of(dev)))
+        try:
+            # any byte is in bounds for the builder, so it starts at once
+            check(lib().bpd_build_tok_next(*args, _lib.stream_of(dev)))
+        finally:
+            check_ids()
     else:
         check(lib().bpd_host_build_tok_next(*args))
     return out

@@ -165,8 +165,8 @@ int bpd_bit_rows(const uint32_t* allow_bits, int64_t words, int32_t num_states,
                  const int32_t* states, int64_t rows, uint32_t* out, int32_t* err, void* stream);
 
 /* bpd_narrow_symbols: the symbol classes of bpd_build_tok_next from int32
- * ids; *bad (zeroed by the caller, device memory) becomes non-zero when an id
- * lies outside [0, 255]. */
+ * ids; *bad (zeroed by the caller, device or pinned host memory) becomes
+ * non-zero when an id lies outside [0, 255]. */
 int bpd_narrow_symbols(const int32_t* symbols, int64_t n, uint8_t* out, int32_t* bad, void* stream);
 
 /* bpd_build_reachability: live[s] = 1 iff an accepting state is reachable
