@@ -22,6 +22,7 @@ OK, ERR_INVALID, ERR_HIP, ERR_OVERFLOW, ERR_UNSUPPORTED = 0, 1, 2, 3, 4
 DTYPE_F32, DTYPE_F16, DTYPE_BF16, DTYPE_F64 = 0, 1, 2, 3
 INDEX_I32, INDEX_I64, INDEX_I64_LOW32 = 0, 1, 2
 MAX_FUSED_PENDING = 256  # BPD_MAX_FUSED_PENDING
+MAX_INLINE_VALUES = 960  # BPD_MAX_INLINE_VALUES
 FLAG_STATE_RANGE, FLAG_TOKEN_RANGE = 1, 2
 PDA_MAX_CONFIGS = 8
 PDA_MAX_DEPTH = 32
@@ -80,6 +81,8 @@ _SIGNATURES = {
                                          vp, vp]),
     "bpd_dense_apply_mask_padded": (cint, [vp, cint, i64, i64, i64, i64, vp, i64, i32, vp, vp, vp, i64, f64,
                                            vp, vp]),
+    "bpd_dense_apply_mask_inline": (cint, [vp, cint, i64, i64, i64, i64, vp, i64, i32, vp, vp, i64, vp, f64,
+                                           vp, vp]),
     "bpd_dense_advance_strided": (cint, [vp, i32, i64, vp, vp, vp, i64, vp, cint, i64, i64, vp, cint, vp, vp]),
     "bpd_dense_advance": (cint, [vp, i32, i64, vp, vp, vp, i64, vp, cint, i64, vp, cint, vp, vp]),
     "bpd_dense_compute_mask": (cint, [vp, i32, i64, vp, vp, i64, vp, vp, vp]),
@@ -125,6 +128,7 @@ _SIGNATURES = {
     "bpd_soft_build_lookahead": (cint, [vp, i32, i64, vp, vp, i32, i32, vp, vp, sz, vp]),
     "bpd_soft_apply": (cint, [vp, cint, i64, i64, i64, vp, i32, vp, vp, f32, vp, vp]),
     "bpd_soft_apply_queued": (cint, [vp, cint, i64, i64, i64, vp, i32, vp, vp, vp, i64, f32, vp, vp]),
+    "bpd_soft_apply_inline": (cint, [vp, cint, i64, i64, i64, vp, i32, vp, vp, i64, vp, f32, vp, vp]),
     "bpd_host_soft_classes": (cint, [vp, i32, i64, C.POINTER(SoftClassesC)]),
     "bpd_soft_prior_workspace_bytes": (sz, [i64, i64, i32, i32]),
     "bpd_soft_prior_workspace_full": (sz, [i64, i64, C.POINTER(SoftClassesC)]),

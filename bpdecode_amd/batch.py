@@ -14,6 +14,7 @@ from __future__ import annotations
 import array
 import ctypes as C
 import operator
+import struct
 from collections.abc import Hashable, Sequence
 
 import torch
@@ -290,17 +291,47 @@ class ConstraintBatch:
         for that stream.  Reusing it is safe: the copy is ordered after every
         launch already enqueued on the stream, the readers of what it held."""
         stream = _lib.stream_of(self.device)
-        n = len(values)
-        buf = self._ubufs.get(stream)
-        if buf is None or buf.numel() < n:
-            buf = torch.empty(max(n, self.capacity + 2 * _lib.MAX_FUSED_PENDING), dtype=torch.int64,
-                              device=self.device)
-            self._ubufs[stream] = buf
+        buf = self._upload_buffer(len(values), stream)
         addr, cnt = values.buffer_info()
         ptr = buf.data_ptr()
         if cnt:
             check(lib().bpd_stage_int64(ptr, addr, cnt, stream))
         return ptr, buf
+
+    def _upload_buffer(self, n: int, stream: int) -> torch.Tensor:
+        buf = self._ubufs.get(stream)
+        if buf is None or buf.numel() < n:
+            buf = torch.empty(max(n, self.capacity + 2 * _lib.MAX_FUSED_PENDING), dtype=torch.int64,
+                              device=self.device)
+            self._ubufs[stream] = buf
+        return buf
+
+    def _inline_rows(self, seq_ids: Sequence[Hashable], stream: int) -> tuple | None:
+        """(slot list and queued writes as int32 bytes, slot list, queued
+        writes, upload buffer) for a launch that takes them in its arguments;
+        None where there is nothing new, or too much, or an upload was staged.
+        After the launch: :meth:`_launched_inline`."""
+        pend = self._pending
+        B, n = len(seq_ids), len(pend)
+        if self._staged is not None or B == 0 or n > _lib.MAX_FUSED_PENDING or B + 2 * n > _lib.MAX_INLINE_VALUES:
+            return None
+        same = self._same_ids(seq_ids)
+        if same and not n:
+            return None
+        vals = self._slot_vals if same else self._lookup(seq_ids)
+        try:
+            packed = struct.pack(f"{B + 2 * n}i", *vals, *pend, *pend.values())
+        except struct.error:  # beyond 32 bits
+            return None
+        return packed, vals, n, self._upload_buffer(B, stream)
+
+    def _launched_inline(self, seq_ids: Sequence[Hashable], rows: tuple) -> None:
+        """The launch wrote the slot list to the upload buffer and the queued
+        writes to the pool."""
+        _, vals, n, buf = rows
+        self._remember(seq_ids, vals, buf.data_ptr(), buf)
+        if n:
+            self._pending = {}
 
     def _remember(self, seq_ids: Sequence[Hashable], slot_vals, ptr: int, buf: torch.Tensor | None,
                   tensor: torch.Tensor | None = None) -> None:
@@ -392,12 +423,16 @@ class ConstraintBatch:
             if code is None:
                 raise RuntimeError(f"logits dtype {logits.dtype} is not supported")
             B = len(seq_ids)
-            slots, pend, n = self._slots_fused(seq_ids, True)
             ld = logits.stride(0) if B > 1 else self._V
+            stream = _lib.stream_of(self.device)
+            inline = self._inline_rows(seq_ids, stream)
+            if inline is not None:
+                self._mask_inline(seq_ids, inline, logits, code, self._V, ld, neg_inf, stream)
+                return logits
+            slots, pend, n = self._slots_fused(seq_ids, True)
             check(self._f_mask(
                 logits.data_ptr(), code, B, self._V, ld, self._bits_ptr, self._W, self._S,
-                self._pool_ptr, slots, pend, n, float(neg_inf), self._err_ptr,
-                _lib.stream_of(self.device)))
+                self._pool_ptr, slots, pend, n, float(neg_inf), self._err_ptr, stream))
             if n:
                 self._launched()
             return logits
@@ -426,11 +461,16 @@ class ConstraintBatch:
         if (self._fast and self.cache is None and code is not None and B == len(seq_ids) and cols >= V
                 and scores.device == self.device and (scores.stride(1) == 1 or cols <= 1)
                 and (B <= 1 or scores.stride(0) >= cols)):
+            ld = scores.stride(0) if B > 1 else cols
+            stream = _lib.stream_of(self.device)
+            inline = self._inline_rows(seq_ids, stream)
+            if inline is not None:
+                self._mask_inline(seq_ids, inline, scores, code, cols, ld, neg_inf, stream)
+                return scores
             slots, pend, n = self._slots_fused(seq_ids, True)
             check(lib().bpd_dense_apply_mask_padded(
-                scores.data_ptr(), code, B, V, cols, scores.stride(0) if B > 1 else cols, self._bits_ptr, self._W,
-                self._S, self._pool_ptr, slots, pend, n, float(neg_inf), self._err_ptr,
-                _lib.stream_of(self.device)))
+                scores.data_ptr(), code, B, V, cols, ld, self._bits_ptr, self._W, self._S, self._pool_ptr, slots,
+                pend, n, float(neg_inf), self._err_ptr, stream))
             if n:
                 self._launched()
             return scores
@@ -438,6 +478,13 @@ class ConstraintBatch:
             scores[:, V:] = neg_inf
         self.apply_mask(seq_ids, scores[:, :V], neg_inf)
         return scores
+
+    def _mask_inline(self, seq_ids, inline: tuple, x: torch.Tensor, code: int, cols: int, ld: int, neg_inf: float,
+                     stream: int) -> None:
+        check(lib().bpd_dense_apply_mask_inline(
+            x.data_ptr(), code, len(seq_ids), self._V, cols, ld, self._bits_ptr, self._W, self._S, self._pool_ptr,
+            inline[0], inline[2], inline[3].data_ptr(), float(neg_inf), self._err_ptr, stream))
+        self._launched_inline(seq_ids, inline)
 
     def _fast_logits(self, logits: torch.Tensor, rows: int) -> bool:
         """Logits the device dense path takes as they are: [rows, vocab] on
@@ -457,11 +504,19 @@ class ConstraintBatch:
         if (self._fast and code is not None and self._fast_logits(logits, len(seq_ids))
                 and la.dtype == torch.float32 and la.is_contiguous() and la.shape[1] == self._V):
             B = len(seq_ids)
+            ld = logits.stride(0) if B > 1 else self._V
+            stream = _lib.stream_of(self.device)
+            inline = self._inline_rows(seq_ids, stream) if self._V else None
+            if inline is not None:
+                check(lib().bpd_soft_apply_inline(
+                    logits.data_ptr(), code, B, self._V, ld, la.data_ptr(), int(la.shape[0]), self._pool_ptr,
+                    inline[0], inline[2], inline[3].data_ptr(), float(alpha), None, stream))
+                self._launched_inline(seq_ids, inline)
+                return logits
             slots, pend, n = self._slots_fused(seq_ids, True)
             check(lib().bpd_soft_apply_queued(
-                logits.data_ptr(), code, B, self._V, logits.stride(0) if B > 1 else self._V, la.data_ptr(),
-                int(la.shape[0]), self._pool_ptr, slots, pend, n, float(alpha), None,
-                _lib.stream_of(self.device)))
+                logits.data_ptr(), code, B, self._V, ld, la.data_ptr(), int(la.shape[0]), self._pool_ptr, slots,
+                pend, n, float(alpha), None, stream))
             if n:
                 self._launched()
             return logits

@@ -50,12 +50,17 @@ template <> struct Elem<8> { using T = uint64_t; };
 // row and 4 consecutive chunks; logical blocks are numbered column-group
 // major, so one XCD's L2 serves a contiguous band of table columns to every
 // row.  The block with logical index 0 also applies the queued pool writes.
-template <int E, bool Bits>
+// N: slots and queued writes come in the arguments (rows.hpp), and block 0
+// leaves the slots in slots_out: [33, 100003] fp16 and two requests turning
+// over: a step of 16.1 us, 18.5 with an upload before the launch (256 rows of
+// V = 151,936 bf16: 28.1 and 30.4).
+template <int E, bool Bits, int N>
 __global__ __launch_bounds__(kFillThreads) void dense_fill_kernel(
     uint8_t* __restrict__ logits, int64_t ld_bytes, const void* __restrict__ table,
     int64_t table_ld, int64_t vocab, int32_t num_states, int32_t* states,
     const int64_t* __restrict__ slots, const int64_t* __restrict__ pending, int32_t num_pending,
-    uint32_t rows, uint32_t chunks, uint64_t fill, int32_t* __restrict__ err) {
+    uint32_t rows, uint32_t chunks, uint64_t fill, int32_t* __restrict__ err, InlineRows<N> inl,
+    int64_t* __restrict__ slots_out) {
   using T = typename Elem<E>::T;
   const uint32_t lb = logical_block();
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -63,10 +68,12 @@ __global__ __launch_bounds__(kFillThreads) void dense_fill_kernel(
   const uint32_t cg = lb / rows;
   const uint32_t r = lb - cg * rows;
   const uint32_t chunk = cg * kFillWaves + wave;
-  if (lb == 0 && wave == 0)
+  if (N > 0 && lb == 0) store_inline_rows(inl.v, rows, num_pending, states, slots_out);
+  if (N == 0 && lb == 0 && wave == 0)
     for (int32_t i = lane; i < num_pending; i += 64) states[pending[i]] = int32_t(pending[num_pending + i]);
   if (chunk >= chunks) return;
-  const int32_t s = wave_row_state(states, slots, pending, num_pending, r, lane);
+  const int32_t s = N > 0 ? wave_row_state_inline(states, inl.v, rows, num_pending, r, lane)
+                          : wave_row_state(states, slots, pending, num_pending, r, lane);
   const bool live = s >= 0 && s < num_states;
   if (s >= num_states && err && lane == 0 && chunk == 0) atomicOr(err, BPD_FLAG_STATE_RANGE);
   const int64_t c0 = int64_t(chunk) * kChunkCols;
@@ -472,13 +479,15 @@ namespace {
 int launch_fill(void* logits, int dtype, int64_t rows, int64_t vocab, int64_t ld, const void* table,
                 int64_t table_ld, bool bits, int32_t num_states, int32_t* states,
                 const int64_t* slots, const int64_t* pending, int64_t num_pending, double neg_inf,
-                int32_t* err, void* stream) {
+                int32_t* err, void* stream, const int32_t* inline_values = nullptr,
+                int64_t* slots_out = nullptr) {
   const int E = dense_elem_bytes(dtype);
   BPD_REQUIRE(E != 0, "unknown logits dtype code %d", dtype);
   BPD_REQUIRE(rows >= 0 && vocab >= 0 && ld >= vocab, "bad logits shape rows=%lld vocab=%lld ld=%lld",
               (long long)rows, (long long)vocab, (long long)ld);
   BPD_REQUIRE(num_states > 0, "empty grammar table");
-  if (int rc = check_pending(pending, num_pending, slots, rows)) return rc;
+  if (!inline_values)
+    if (int rc = check_pending(pending, num_pending, slots, rows)) return rc;
   uint64_t fill = 0;
   if (int rc = fill_bits64(dtype, neg_inf, &fill)) return rc;
   if (rows == 0) return BPD_OK;
@@ -492,18 +501,29 @@ int launch_fill(void* logits, int dtype, int64_t rows, int64_t vocab, int64_t ld
   hipStream_t s = as_stream(stream);
   uint8_t* lg = static_cast<uint8_t*>(logits);
   const int32_t np = int32_t(num_pending);
-#define BPD_FILL(EB, BITS)                                                                      \
-  dense_fill_kernel<EB, BITS><<<dim3(unsigned(blocks)), dim3(kFillThreads), 0, s>>>(            \
+#define BPD_FILL(EB, BITS, N, INL)                                                              \
+  dense_fill_kernel<EB, BITS, N><<<dim3(unsigned(blocks)), dim3(kFillThreads), 0, s>>>(         \
       lg, ld * EB, table, table_ld, vocab, num_states, states, slots, pending, np,              \
-      uint32_t(rows), uint32_t(chunks), fill, err)
+      uint32_t(rows), uint32_t(chunks), fill, err, INL, slots_out)
+  if (inline_values) {
+    return with_inline_rows(inline_values, rows + 2 * num_pending, [&](const auto& inl) -> int {
+      constexpr int N = int(sizeof(inl.v) / sizeof(inl.v[0]));
+      if (E == 2) BPD_FILL(2, true, N, inl);
+      else if (E == 4) BPD_FILL(4, true, N, inl);
+      else BPD_FILL(8, true, N, inl);
+      BPD_LAUNCHED();
+      return BPD_OK;
+    });
+  }
+  const InlineRows<0> none{};
   if (bits) {
-    if (E == 2) BPD_FILL(2, true);
-    else if (E == 4) BPD_FILL(4, true);
-    else BPD_FILL(8, true);
+    if (E == 2) BPD_FILL(2, true, 0, none);
+    else if (E == 4) BPD_FILL(4, true, 0, none);
+    else BPD_FILL(8, true, 0, none);
   } else {
-    if (E == 2) BPD_FILL(2, false);
-    else if (E == 4) BPD_FILL(4, false);
-    else BPD_FILL(8, false);
+    if (E == 2) BPD_FILL(2, false, 0, none);
+    else if (E == 4) BPD_FILL(4, false, 0, none);
+    else BPD_FILL(8, false, 0, none);
   }
 #undef BPD_FILL
   BPD_LAUNCHED();
@@ -542,6 +562,18 @@ extern "C" int bpd_dense_apply_mask_padded(void* logits, int dtype, int64_t rows
   // a column past the table's words, or past vocab in its last one, is rejected
   return launch_fill(logits, dtype, rows, cols, ld, allow_bits, words, true, num_states, states,
                      slots, pending, num_pending, neg_inf, err, stream);
+}
+
+extern "C" int bpd_dense_apply_mask_inline(void* logits, int dtype, int64_t rows, int64_t vocab, int64_t cols,
+                                           int64_t ld, const uint32_t* allow_bits, int64_t words,
+                                           int32_t num_states, int32_t* states, const int32_t* values,
+                                           int64_t num_pending, int64_t* slots_out, double neg_inf,
+                                           int32_t* err, void* stream) {
+  BPD_REQUIRE(words == (vocab + 31) / 32, "allow-bit rows must hold ceil(vocab/32) words");
+  BPD_REQUIRE(cols >= vocab, "fewer columns than tokens");
+  if (int rc = check_inline(values, rows, num_pending, states, slots_out)) return rc;
+  return launch_fill(logits, dtype, rows, cols, ld, allow_bits, words, true, num_states, states, nullptr,
+                     nullptr, num_pending, neg_inf, err, stream, values, slots_out);
 }
 
 extern "C" int bpd_dense_advance(const int32_t* tok_next, int32_t num_states, int64_t vocab,

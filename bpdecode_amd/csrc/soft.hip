@@ -331,22 +331,26 @@ __device__ __forceinline__ uint32_t soft_value(uint32_t bits, float bias, float 
 // 40.2 us, non-temporal stores made no difference.
 constexpr int kApplyThreads = 256;
 
-template <int D, int U>
+// N_ARGS: slots and queued writes come in the arguments (rows.hpp), and block 0
+// leaves the slots in slots_out.
+template <int D, int U, int N_ARGS>
 __global__ __launch_bounds__(kApplyThreads) void soft_apply_kernel(
     uint8_t* __restrict__ logits, int64_t ld_bytes, int64_t V, const float* __restrict__ la, int32_t S,
     int32_t* states, const int64_t* __restrict__ slots, const int64_t* __restrict__ pending,
     int32_t num_pending, uint32_t rows, uint32_t chunks, float alpha, uint32_t ninf,
-    int32_t* __restrict__ err) {
+    int32_t* __restrict__ err, InlineRows<N_ARGS> inl, int64_t* __restrict__ slots_out) {
   constexpr int E = D == BPD_DTYPE_F32 ? 4 : 2;
   constexpr int N = 16 / E;
   const uint32_t lb = logical_block();
   const uint32_t cg = lb / rows;
   const uint32_t r = lb - cg * rows;
   const int lane = threadIdx.x & 63;
-  if (lb == 0 && threadIdx.x < 64)
+  if (N_ARGS > 0 && lb == 0) store_inline_rows(inl.v, rows, num_pending, states, slots_out);
+  if (N_ARGS == 0 && lb == 0 && threadIdx.x < 64)
     for (int32_t i = lane; i < num_pending; i += 64) states[pending[i]] = int32_t(pending[num_pending + i]);
   if (cg >= chunks) return;
-  const int32_t s = wave_row_state(states, slots, pending, num_pending, r, lane);
+  const int32_t s = N_ARGS > 0 ? wave_row_state_inline(states, inl.v, rows, num_pending, r, lane)
+                               : wave_row_state(states, slots, pending, num_pending, r, lane);
   const bool on = s >= 0 && s < S;
   if (s >= S && err && cg == 0 && threadIdx.x == 0) atomicOr(err, BPD_FLAG_STATE_RANGE);
   uint8_t* row = logits + int64_t(r) * ld_bytes;
@@ -466,7 +470,8 @@ namespace {
 template <int D>
 int launch_soft_apply(uint8_t* logits, int64_t rows, int64_t vocab, int64_t ld_bytes, const float* lookahead,
                       int32_t num_states, int32_t* states, const int64_t* slots, const int64_t* pending,
-                      int64_t num_pending, float alpha, uint32_t ninf, int32_t* err, hipStream_t st) {
+                      int64_t num_pending, float alpha, uint32_t ninf, int32_t* err, hipStream_t st,
+                      const int32_t* values, int64_t* slots_out) {
   constexpr int64_t N = D == BPD_DTYPE_F32 ? 4 : 8;
   // Two groups per thread once that still gives every CU four blocks, else
   // one (a few rows: more blocks instead of more loads per thread).  At
@@ -478,30 +483,40 @@ int launch_soft_apply(uint8_t* logits, int64_t rows, int64_t vocab, int64_t ld_b
   const int64_t chunks = many ? wide : (vocab + kApplyThreads * N - 1) / (kApplyThreads * N);
   const int64_t blocks = (chunks * rows + kXcds - 1) / kXcds * kXcds;
   BPD_REQUIRE(blocks < (int64_t(1) << 31), "batch too large for one launch");
-#define BPD_SOFT_APPLY(U)                                                                              \
-  soft_apply_kernel<D, U><<<dim3(unsigned(blocks)), kApplyThreads, 0, st>>>(                           \
+#define BPD_SOFT_APPLY(U, NA, INL)                                                                     \
+  soft_apply_kernel<D, U, NA><<<dim3(unsigned(blocks)), kApplyThreads, 0, st>>>(                       \
       logits, ld_bytes, vocab, lookahead, num_states, states, slots, pending, int32_t(num_pending),    \
-      uint32_t(rows), uint32_t(chunks), alpha, ninf, err)
-  if (many)
-    BPD_SOFT_APPLY(int(kWide));
-  else
-    BPD_SOFT_APPLY(1);
+      uint32_t(rows), uint32_t(chunks), alpha, ninf, err, INL, slots_out)
+  auto launch = [&](const auto& inl, auto args) -> int {
+    constexpr int NA = decltype(args)::value;
+    if (many)
+      BPD_SOFT_APPLY(int(kWide), NA, inl);
+    else
+      BPD_SOFT_APPLY(1, NA, inl);
+    BPD_LAUNCHED();
+    return BPD_OK;
+  };
 #undef BPD_SOFT_APPLY
-  BPD_LAUNCHED();
-  return BPD_OK;
+  if (!values) return launch(InlineRows<0>{}, std::integral_constant<int, 0>{});
+  return with_inline_rows(values, rows + 2 * num_pending, [&](const auto& inl) {
+    return launch(inl, std::integral_constant<int, int(sizeof(inl.v) / sizeof(inl.v[0]))>{});
+  });
 }
 
 }  // namespace
 
-extern "C" int bpd_soft_apply_queued(void* logits, int dtype, int64_t rows, int64_t vocab, int64_t ld,
-                                     const float* lookahead, int32_t num_states, int32_t* states,
-                                     const int64_t* slots, const int64_t* pending, int64_t num_pending,
-                                     float alpha, int32_t* err, void* stream) {
+namespace {
+
+int soft_apply_impl(void* logits, int dtype, int64_t rows, int64_t vocab, int64_t ld, const float* lookahead,
+                    int32_t num_states, int32_t* states, const int64_t* slots, const int64_t* pending,
+                    int64_t num_pending, float alpha, int32_t* err, void* stream, const int32_t* values,
+                    int64_t* slots_out) {
   const int E = elem_bytes(dtype);
   BPD_REQUIRE(E != 0, "unknown logits dtype code %d", dtype);
   BPD_REQUIRE(rows >= 0 && vocab >= 0 && ld >= vocab, "bad logits shape");
   BPD_REQUIRE(num_states > 0, "empty lookahead table");
-  if (int rc = check_pending(pending, num_pending, slots, rows)) return rc;
+  if (!values)
+    if (int rc = check_pending(pending, num_pending, slots, rows)) return rc;
   uint32_t ninf = 0;
   if (int rc = fill_bits(dtype, -INFINITY, &ninf)) return rc;
   if (rows == 0 || (vocab == 0 && num_pending == 0)) return BPD_OK;
@@ -512,7 +527,27 @@ extern "C" int bpd_soft_apply_queued(void* logits, int dtype, int64_t rows, int6
                 : dtype == BPD_DTYPE_F16 ? launch_soft_apply<BPD_DTYPE_F16>
                                          : launch_soft_apply<BPD_DTYPE_BF16>;
   return launch(lg, rows, vocab, ld * E, lookahead, num_states, states, slots, pending, num_pending, alpha,
-                ninf, err, st);
+                ninf, err, st, values, slots_out);
+}
+
+}  // namespace
+
+extern "C" int bpd_soft_apply_queued(void* logits, int dtype, int64_t rows, int64_t vocab, int64_t ld,
+                                     const float* lookahead, int32_t num_states, int32_t* states,
+                                     const int64_t* slots, const int64_t* pending, int64_t num_pending,
+                                     float alpha, int32_t* err, void* stream) {
+  return soft_apply_impl(logits, dtype, rows, vocab, ld, lookahead, num_states, states, slots, pending,
+                         num_pending, alpha, err, stream, nullptr, nullptr);
+}
+
+extern "C" int bpd_soft_apply_inline(void* logits, int dtype, int64_t rows, int64_t vocab, int64_t ld,
+                                     const float* lookahead, int32_t num_states, int32_t* states,
+                                     const int32_t* values, int64_t num_pending, int64_t* slots_out,
+                                     float alpha, int32_t* err, void* stream) {
+  BPD_REQUIRE(vocab > 0, "empty vocabulary");
+  if (int rc = check_inline(values, rows, num_pending, states, slots_out)) return rc;
+  return soft_apply_impl(logits, dtype, rows, vocab, ld, lookahead, num_states, states, nullptr, nullptr,
+                         num_pending, alpha, err, stream, values, slots_out);
 }
 
 extern "C" int bpd_soft_apply(void* logits, int dtype, int64_t rows, int64_t vocab, int64_t ld,

@@ -56,6 +56,9 @@ extern "C" {
 
 /* Queued state-pool writes a dense mask or commit launch applies itself. */
 #define BPD_MAX_FUSED_PENDING 256
+/* Values (slots and queued writes) that the *_inline entries take in a
+ * launch's arguments. */
+#define BPD_MAX_INLINE_VALUES 960
 
 /* Bits OR-ed into the optional `err` word by kernels (device int32). */
 #define BPD_FLAG_STATE_RANGE 1 /* a state >= num_states was read */
@@ -108,6 +111,18 @@ int bpd_dense_apply_mask_padded(void* logits, int dtype, int64_t rows, int64_t v
                                 int64_t ld, const uint32_t* allow_bits, int64_t words,
                                 int32_t num_states, int32_t* states, const int64_t* slots,
                                 const int64_t* pending, int64_t num_pending, double neg_inf,
+                                int32_t* err, void* stream);
+
+/* bpd_dense_apply_mask_inline: bpd_dense_apply_mask_padded with the slot list
+ * and the queued pool writes from HOST memory: `values` holds rows slots, then
+ * num_pending slots and as many values (rows + 2 * num_pending <=
+ * BPD_MAX_INLINE_VALUES).  They travel in the launch's arguments (the array is
+ * free on return), and the launch leaves the slots in slots_out (device, rows
+ * int64) for the launches after it. */
+int bpd_dense_apply_mask_inline(void* logits, int dtype, int64_t rows, int64_t vocab, int64_t cols,
+                                int64_t ld, const uint32_t* allow_bits, int64_t words,
+                                int32_t num_states, int32_t* states, const int32_t* values,
+                                int64_t num_pending, int64_t* slots_out, double neg_inf,
                                 int32_t* err, void* stream);
 
 /* bpd_dense_advance: nxt = state(b) < 0 ? -1 : tok_next[state(b), t(b)], where
@@ -499,6 +514,13 @@ int bpd_soft_apply(void* logits, int dtype, int64_t rows, int64_t vocab, int64_t
 int bpd_soft_apply_queued(void* logits, int dtype, int64_t rows, int64_t vocab, int64_t ld,
                           const float* lookahead, int32_t num_states, int32_t* states,
                           const int64_t* slots, const int64_t* pending, int64_t num_pending,
+                          float alpha, int32_t* err, void* stream);
+
+/* The same with `values` in the launch's arguments, as
+ * bpd_dense_apply_mask_inline. */
+int bpd_soft_apply_inline(void* logits, int dtype, int64_t rows, int64_t vocab, int64_t ld,
+                          const float* lookahead, int32_t num_states, int32_t* states,
+                          const int32_t* values, int64_t num_pending, int64_t* slots_out,
                           float alpha, int32_t* err, void* stream);
 
 int bpd_host_soft_build_lookahead(const int32_t* tok_next, int32_t num_states, int64_t vocab,

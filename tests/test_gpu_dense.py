@@ -444,3 +444,52 @@ def test_table_builder_refuses_wide_symbols(dev):
         fsa.symbols[7] = bad
         with pytest.raises(RuntimeError, match="symbol-class ids"):
             ops.build_token_transitions(fsa.to(dev))
+
+
+@pytest.mark.parametrize("form", ["mask", "padded", "soft"])
+@pytest.mark.parametrize("rows,queued", [(1, 0), (1, 1), (60, 2), (61, 2), (63, 1), (200, 60), (201, 60), (319, 1),
+                                         (450, 255), (451, 255), (960, 0), (961, 0)])
+def test_slots_and_writes_in_the_launch(dev, rows, queued, form):
+    """Slot lists and queued writes at the sizes where they change from one
+    set of launch arguments to the next and to an upload (64, 320 and 960
+    values), with queued slots inside and outside the launch's rows and rows
+    in an order of their own; a launch after it reads the slots it left."""
+    _log(f"case launch arguments rows={rows} queued={queued} {form}")
+    fsa = FsaTensors.build("a[012]+|b0", TOY_VOCAB).with_lookahead(3).to(dev)
+    V, tn, la = fsa.vocab_size, fsa.tok_next.cpu(), fsa.lookahead.cpu()
+    S = fsa.num_states
+    g = np.random.default_rng(rows + queued)
+    batch = ConstraintBatch(fsa, capacity=rows + 20, device=dev)
+    every = list(range(rows + 20))
+    for i in every:
+        batch.add(i)
+    state = g.integers(-1, S, size=rows + 20)
+    batch._state.copy_(torch.from_numpy(state).to(torch.int32))
+    ids = g.permutation(rows + 20)[:rows].tolist()
+    for i in g.permutation(rows + 20)[:queued].tolist():
+        batch.reset(i)
+        state[i] = fsa.start
+    for again in range(2):  # the second call's slots come from the first's launch
+        x = torch.randn(rows, V + 3, generator=torch.Generator().manual_seed(rows))
+        st = torch.from_numpy(state[ids])
+        allowed = torch.zeros(rows, V, dtype=torch.bool)
+        allowed[st >= 0] = tn[st[st >= 0]] != -1
+        got, want = x.to(dev), x.clone()
+        if form == "mask":
+            batch.apply_mask(ids, got[:, :V])
+            want[:, :V][~allowed] = -float("inf")
+        elif form == "padded":
+            batch.apply_mask_padded(ids, got)
+            want[:, :V][~allowed] = -float("inf")
+            want[:, V:] = -float("inf")
+        else:
+            batch.apply_soft(ids, got[:, :V], 0.0)
+            keep = torch.zeros(rows, V, dtype=torch.bool)
+            keep[st >= 0] = la[st[st >= 0]] != -float("inf")
+            want[:, :V][~keep] = -float("inf")
+        assert torch.equal(got.cpu(), want), again
+        assert batch._pool.cpu().tolist() == state.tolist()
+    tok = torch.from_numpy(g.integers(0, V, size=rows)).to(dev)
+    nxt = [int(tn[state[i], t]) if state[i] >= 0 else -1 for i, t in zip(ids, tok.tolist())]
+    assert batch.commit(ids, tok).tolist() == nxt
+    batch.check_errors()
