@@ -23,6 +23,7 @@ DTYPE_F32, DTYPE_F16, DTYPE_BF16, DTYPE_F64 = 0, 1, 2, 3
 INDEX_I32, INDEX_I64, INDEX_I64_LOW32 = 0, 1, 2
 MAX_FUSED_PENDING = 256  # BPD_MAX_FUSED_PENDING
 MAX_INLINE_VALUES = 960  # BPD_MAX_INLINE_VALUES
+MAX_PRIOR_INLINE_VALUES = 320  # BPD_MAX_PRIOR_INLINE_VALUES
 FLAG_STATE_RANGE, FLAG_TOKEN_RANGE = 1, 2
 PDA_MAX_CONFIGS = 8
 PDA_MAX_DEPTH = 32
@@ -135,6 +136,8 @@ _SIGNATURES = {
     "bpd_soft_prior": (cint, [vp, i64, i64, i64, i32, vp, vp, i32, vp, vp, C.POINTER(SoftClassesC),
                               i32, f32, vp, sz, vp, vp]),
     "bpd_soft_prior_queued": (cint, [vp, i64, i64, i64, i32, vp, vp, i32, vp, vp, vp, i64,
+                                     C.POINTER(SoftClassesC), i32, f32, vp, sz, vp, vp]),
+    "bpd_soft_prior_inline": (cint, [vp, i64, i64, i64, i32, vp, vp, i32, vp, vp, i64, vp,
                                      C.POINTER(SoftClassesC), i32, f32, vp, sz, vp, vp]),
     "bpd_soft_prior_noalloc": (cint, [vp, i64, i64, i64, i32, vp, vp, i32, vp, vp,
                                       C.POINTER(SoftClassesC), i32, f32, vp, vp]),

@@ -306,14 +306,15 @@ class ConstraintBatch:
             self._ubufs[stream] = buf
         return buf
 
-    def _inline_rows(self, seq_ids: Sequence[Hashable], stream: int) -> tuple | None:
+    def _inline_rows(self, seq_ids: Sequence[Hashable], stream: int,
+                     limit: int = _lib.MAX_INLINE_VALUES) -> tuple | None:
         """(slot list and queued writes as int32 bytes, slot list, queued
         writes, upload buffer) for a launch that takes them in its arguments;
         None where there is nothing new, or too much, or an upload was staged.
         After the launch: :meth:`_launched_inline`."""
         pend = self._pending
         B, n = len(seq_ids), len(pend)
-        if self._staged is not None or B == 0 or n > _lib.MAX_FUSED_PENDING or B + 2 * n > _lib.MAX_INLINE_VALUES:
+        if self._staged is not None or B == 0 or n > _lib.MAX_FUSED_PENDING or B + 2 * n > limit:
             return None
         same = self._same_ids(seq_ids)
         if same and not n:
@@ -538,11 +539,16 @@ class ConstraintBatch:
             eos = fsa.eos_id if fsa.eos_id is not None and 0 <= fsa.eos_id < V else -1
             stream = _lib.stream_of(self.device)
             ws, ws_bytes = sc.workspace(B, self.device, stream)
+            rows = (logits.data_ptr(), B, V, logits.stride(0) if B > 1 else V, self._S, acc.data_ptr(),
+                    live.data_ptr(), eos, self._pool_ptr)
+            rest = (C.byref(sc.c_struct()), int(k), float(alpha), ws.data_ptr(), ws_bytes, self._err_ptr, stream)
+            inline = self._inline_rows(seq_ids, stream, _lib.MAX_PRIOR_INLINE_VALUES)
+            if inline is not None:
+                check(lib().bpd_soft_prior_inline(*rows, inline[0], inline[2], inline[3].data_ptr(), *rest))
+                self._launched_inline(seq_ids, inline)
+                return logits
             slots, pend, n = self._slots_fused(seq_ids, True)
-            check(lib().bpd_soft_prior_queued(
-                logits.data_ptr(), B, V, logits.stride(0) if B > 1 else V, self._S, acc.data_ptr(), live.data_ptr(),
-                eos, self._pool_ptr, slots, pend, n, C.byref(sc.c_struct()), int(k), float(alpha), ws.data_ptr(),
-                ws_bytes, self._err_ptr, stream))
+            check(lib().bpd_soft_prior_queued(*rows, slots, pend, n, *rest))
             if n:
                 self._launched()
             return logits

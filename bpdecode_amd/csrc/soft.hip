@@ -780,16 +780,27 @@ PriorPlan prior_plan(int64_t rows, int64_t vocab, int32_t C, int32_t P, bool for
 }
 
 // Queued pool writes of a batch: the statistics launch, which needs no row's
-// state, makes them, and the launches after it read the pool.
+// state, makes them, and the launches after it read the pool.  They come in
+// device memory, or (rows > 0) with the slot list in the launch's arguments
+// (rows.hpp), which it then leaves in slots_out.
+constexpr int kPriorInline = BPD_MAX_PRIOR_INLINE_VALUES;
+
 struct QueuedWrites {
   int32_t* pool;
   const int64_t* pending;  // count slots, then as many values
   int32_t count;
+  int32_t rows;
+  int64_t* slots_out;
+  InlineRows<kPriorInline> inl;
 };
 
 __device__ __forceinline__ void make_queued_writes(const QueuedWrites& q) {
-  if (blockIdx.x == 0 && blockIdx.y == 0)
+  if (blockIdx.x != 0 || blockIdx.y != 0) return;
+  if (q.rows > 0) {
+    store_inline_rows(q.inl.v, uint32_t(q.rows), q.count, q.pool, q.slots_out);
+  } else {
     for (int32_t i = threadIdx.x; i < q.count; i += kPriorThreads) q.pool[q.pending[i]] = int32_t(q.pending[q.count + i]);
+  }
 }
 
 struct PriorWs {
@@ -1416,15 +1427,15 @@ __device__ inline float prior_value(float x, float lse, int64_t t, float z, bool
 }
 
 // The rounds and the epilogue of the prior lookahead for row b, by the
-// kRoundThreads threads of its block: lc holds the class logsumexps of the
-// row (LDS, reused for zcls), z0 / z1 the state values (z0 initialised: 0
+// kRoundThreads threads of its block: lc holds the classes' log probabilities
+// less lse_rest (LDS, reused for zcls), z0 / z1 the state values (z0 initialised: 0
 // for live states, -inf else), flag / so the state flags and pair offsets,
 // pr the pairs (PairsInLds).
 template <bool PairsInLds>
 __device__ __forceinline__ void prior_rounds_tail(float* lc, float* z0, float* z1, const uint8_t* flag,
                                                   const int32_t* so, const uint32_t* pr,
                                                   const BpdSoftClasses& cls, int32_t S, int32_t rounds,
-                                                  float lse, float lp_eos, int32_t sb) {
+                                                  float lse_rest, float lp_eos, int32_t sb) {
   const int tid = threadIdx.x;
   const int32_t C = cls.num_classes;
   // eight lanes per state: lane l folds pairs l, l + 8, ... of its state
@@ -1457,14 +1468,14 @@ __device__ __forceinline__ void prior_rounds_tail(float* lc, float* z0, float* z
     }
     if (on && gl == 0) {
       const uint8_t f = flag[s];
-      float v = m == -INFINITY ? -INFINITY : m + logf(sm) - lse;
+      float v = m == -INFINITY ? -INFINITY : m + logf(sm) - lse_rest;
       if (f & 2) v = log_add_exp(v, lp_eos);
       zn[s] = (f & 1) ? v : -INFINITY;
     }
   };
   if (S <= kGroups) {
     // one state per group; a lane's first kRegPairs pairs are gathered once
-    // as (class logsumexp, next state), so a round reads only zc for them
+    // as (class log probability, next state), so a round reads only zc for them
     const int32_t s = grp;
     const bool on = s < S;
     const int32_t i0 = on ? so[s] : 0, i1 = on ? so[s + 1] : 0;
@@ -1557,8 +1568,8 @@ struct PriorOut {
 // `stage`: two chunks of LDS.
 __device__ __forceinline__ void prior_out_chunks(const PriorOut& out, int64_t ld, int64_t b, const float* z,
                                                  float4* stage, const BpdSoftClasses& cls,
-                                                 const float* __restrict__ vals, float lse, float x_eos,
-                                                 bool acc_s, int32_t eos, int split, int splits) {
+                                                 const float* __restrict__ vals, float lse, float low,
+                                                 float lp_eos, bool acc_s, int32_t eos, int split, int splits) {
   static_assert(kRoundThreads * 4 == BPD_SOFT_MEMBER_CHUNK, "one float4 per thread");
   const int tid = threadIdx.x;
   const float4 ninf = make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
@@ -1590,12 +1601,12 @@ __device__ __forceinline__ void prior_out_chunks(const PriorOut& out, int64_t ld
     if (mm != 0xFFFFFFFFu && base + int64_t(mm >> 16) != eos) {
       const float zv = z[mm & 0xFFFFu];
       if (zv != -INFINITY) {
-        const float lp = xv - lse;
+        const float lp = (xv - lse) - low;
         reinterpret_cast<float*>(st)[mm >> 16] = out.alpha != 0.0f ? fmaf(out.alpha, zv, lp) : lp;
       }
     }
     if (tid == 0 && acc_s && eos >= base && eos < base + BPD_SOFT_MEMBER_CHUNK)
-      reinterpret_cast<float*>(st)[eos - base] = x_eos - lse;
+      reinterpret_cast<float*>(st)[eos - base] = lp_eos;
     fetch(ch + splits);
     __syncthreads();
     const float4 o = st[tid];
@@ -1624,11 +1635,13 @@ __global__ __launch_bounds__(kRoundThreads) void prior_rounds_kernel(
     const int32_t* __restrict__ states, const int64_t* __restrict__ slots, int32_t rounds,
     PriorWs ws, PriorOut out) {
   extern __shared__ __align__(16) float lds[];
-  __shared__ float lse_sh;
+  // the row's logsumexp: rounded, and what that left out; the part of it that
+  // the classes are normalised by (all of it, unless it is not finite)
+  __shared__ float lse_sh, lse_low, lse_norm;
   const int64_t b = Out ? blockIdx.y : blockIdx.x;
   const int tid = threadIdx.x;
   const int32_t C = cls.num_classes, P = cls.num_pieces, NP = cls.num_pairs;
-  float* lc = lds;                                        // [C] class logsumexp, later zcls
+  float* lc = lds;                                        // [C] class log probability, later zcls
   float* z0 = lc + C;                                     // [S]
   float* z1 = z0 + S;                                     // [S]
   uint8_t* flag = reinterpret_cast<uint8_t*>(z1 + S);     // [S] bit 0 live, bit 1 accept
@@ -1671,7 +1684,13 @@ __global__ __launch_bounds__(kRoundThreads) void prior_rounds_kernel(
   if (tid < 64) {
     for (int i = tid + 64; i < G; i += 64) part = lse_merge(part, Lse{ws.part[(b * G + i) * 2], ws.part[(b * G + i) * 2 + 1]});
     part = wave_lse(part);
-    if (tid == 0) lse_sh = lse_value(part);
+    if (tid == 0) {
+      const float rest = part.s > 0.0f ? logf(part.s) : 0.0f;
+      lse_sh = lse_value(part);
+      const bool finite = fabsf(lse_sh) < INFINITY;
+      lse_low = finite ? (part.m - lse_sh) + rest : 0.0f;
+      lse_norm = finite ? lse_sh : 0.0f;
+    }
   }
   for (int32_t s = tid; s < S; s += kRoundThreads) {
     const bool lv = (s == tid ? lv0 : live[s]) != 0;
@@ -1721,7 +1740,9 @@ __global__ __launch_bounds__(kRoundThreads) void prior_rounds_kernel(
         }
       }
       csum = group8_sum(csum);
-      if (mq == 0 && c < C) lc[c] = csum > 0.0f ? cm + logf(csum) : -INFINITY;
+      // a probability at most: cm - lse is small and nearly exact, where the
+      // class logsumexp would round at the logits' size
+      if (mq == 0 && c < C) lc[c] = csum > 0.0f ? ((cm - lse_norm) - lse_low) + logf(csum) : -INFINITY;
     }
   } else {
     // [P] piece (max, sum) pairs, 8-byte aligned after the pairs
@@ -1735,18 +1756,18 @@ __global__ __launch_bounds__(kRoundThreads) void prior_rounds_kernel(
     for (int32_t c = tid; c < C; c += kRoundThreads) {
       Lse a{-INFINITY, 0.0f};
       for (int32_t p = cls.class_piece[c]; p < cls.class_piece[c + 1]; ++p) a = lse_merge(a, Lse{pc[p].x, pc[p].y});
-      lc[c] = lse_value(a);
+      lc[c] = a.m == -INFINITY ? -INFINITY : ((a.m - lse_norm) - lse_low) + logf(a.s);
     }
   }
   __syncthreads();
-  const float lse = lse_sh;
-  const float lp_eos = eos >= 0 ? x_eos - lse : -INFINITY;
-  prior_rounds_tail<PairsInLds>(lc, z0, z1, flag, so, pr, cls, S, rounds, lse, lp_eos, sb);
+  const float lse = lse_sh, low = lse_low;
+  const float lp_eos = eos >= 0 ? (x_eos - lse) - low : -INFINITY;
+  prior_rounds_tail<PairsInLds>(lc, z0, z1, flag, so, pr, cls, S, rounds, lse - lse_norm, lp_eos, sb);
   if (Out) {
     const bool live_row = sb >= 0 && sb < S;
     if (sb >= S && out.err && blockIdx.x == 0 && tid == 0) atomicOr(out.err, BPD_FLAG_STATE_RANGE);
     float4* stage = reinterpret_cast<float4*>(lds + (C + 3) / 4 * 4);  // over what the rounds needed
-    prior_out_chunks(out, ld, b, lc, stage, cls, ws.vals, lse, x_eos, live_row && accept[sb] != 0, eos,
+    prior_out_chunks(out, ld, b, lc, stage, cls, ws.vals, lse, low, lp_eos, live_row && accept[sb] != 0, eos,
                      int(blockIdx.x), int(gridDim.x));
   } else {
     for (int32_t c = tid; c < C; c += kRoundThreads) ws.zcls[b * C + c] = lc[c];
@@ -2036,9 +2057,30 @@ extern "C" int bpd_soft_prior_queued(float* logits, int64_t rows, int64_t vocab,
                                      const BpdSoftClasses* classes, int32_t k, float alpha,
                                      void* workspace, size_t workspace_bytes, int32_t* err, void* stream) {
   if (int rc = check_pending(pending, num_pending, slots, rows)) return rc;
-  return soft_prior_impl(logits, rows, vocab, ld, num_states, accept, live, eos_id, states, slots,
-                         QueuedWrites{states, pending, int32_t(num_pending)}, classes, k, alpha, workspace,
-                         workspace_bytes, err, stream);
+  QueuedWrites queued{};
+  queued.pool = states;
+  queued.pending = pending;
+  queued.count = int32_t(num_pending);
+  return soft_prior_impl(logits, rows, vocab, ld, num_states, accept, live, eos_id, states, slots, queued,
+                         classes, k, alpha, workspace, workspace_bytes, err, stream);
+}
+
+extern "C" int bpd_soft_prior_inline(float* logits, int64_t rows, int64_t vocab, int64_t ld,
+                                     int32_t num_states, const uint8_t* accept, const uint8_t* live,
+                                     int32_t eos_id, int32_t* states, const int32_t* values,
+                                     int64_t num_pending, int64_t* slots_out, const BpdSoftClasses* classes,
+                                     int32_t k, float alpha, void* workspace, size_t workspace_bytes,
+                                     int32_t* err, void* stream) {
+  if (int rc = check_inline(values, rows, num_pending, states, slots_out)) return rc;
+  BPD_REQUIRE(rows + 2 * num_pending <= kPriorInline, "at most %d values in this launch's arguments", kPriorInline);
+  QueuedWrites queued{};
+  queued.pool = states;
+  queued.count = int32_t(num_pending);
+  queued.rows = int32_t(rows);
+  queued.slots_out = slots_out;
+  std::memcpy(queued.inl.v, values, size_t(rows + 2 * num_pending) * 4);
+  return soft_prior_impl(logits, rows, vocab, ld, num_states, accept, live, eos_id, states, slots_out, queued,
+                         classes, k, alpha, workspace, workspace_bytes, err, stream);
 }
 
 // Workspace of the allocation-free entry point: a file-scope device array,

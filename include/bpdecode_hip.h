@@ -605,6 +605,14 @@ int bpd_soft_prior_queued(float* logits, int64_t rows, int64_t vocab, int64_t ld
                           int32_t* states, const int64_t* slots, const int64_t* pending,
                           int64_t num_pending, const BpdSoftClasses* classes, int32_t k, float alpha,
                           void* workspace, size_t workspace_bytes, int32_t* err, void* stream);
+/* The same with `values` in the statistics launch's arguments, as
+ * bpd_dense_apply_mask_inline, up to BPD_MAX_PRIOR_INLINE_VALUES of them. */
+#define BPD_MAX_PRIOR_INLINE_VALUES 320
+int bpd_soft_prior_inline(float* logits, int64_t rows, int64_t vocab, int64_t ld, int32_t num_states,
+                          const uint8_t* accept, const uint8_t* live, int32_t eos_id,
+                          int32_t* states, const int32_t* values, int64_t num_pending,
+                          int64_t* slots_out, const BpdSoftClasses* classes, int32_t k, float alpha,
+                          void* workspace, size_t workspace_bytes, int32_t* err, void* stream);
 int bpd_host_soft_prior(float* logits, int64_t rows, int64_t vocab, int64_t ld,
                         const int32_t* tok_next, int32_t num_states, const uint8_t* accept,
                         const uint8_t* live, int32_t eos_id, const int32_t* states,

@@ -170,7 +170,8 @@ def test_prior_carries_queued_writes(dev, vocab, stats, monkeypatch):
     batch.commit(ids, torch.full((290,), tok, dtype=torch.int64, device=dev))
     after = int(fsa.tok_next[fsa.start, tok])
     states = [after] * 290
-    for queued in (3, 250, 290):  # 250 fit one launch's queue, 290 are flushed first
+    # 14 fit a launch's arguments, 15 and 250 one upload, 290 are flushed first
+    for queued in (3, 14, 15, 250, 290):
         for i in range(queued):
             batch.reset(ids[i])
         states[:queued] = [fsa.start] * queued
