@@ -678,6 +678,13 @@ namespace {
 constexpr int kPriorThreads = 256;
 constexpr int kPriorOutThreads = 256;
 constexpr int64_t kComputeUnits = 256;
+// The rounds and the member-list output in one launch up to this many member
+// chunks in a batch (two for a CU).  There the launches' own time counts: 9
+// rows of 13 chunks 9.3 us, 13.8 as two launches.  Above, a CU's one block
+// cannot keep as many stores in flight as the output launch's blocks: 128
+// rows of 38 chunks 35.0 us against 11.1 + 17.5 with the rows out of the
+// caches (24.2 against 10.0 + 21.6 with rows just written).
+constexpr int64_t kFusedChunks = 2 * kComputeUnits;
 constexpr int kPriorMaxStates = 4096;
 constexpr int kPieceMembers = 256;
 constexpr int kLdsClasses = 1024;                          // class-atomic stats up to this many classes
@@ -834,8 +841,10 @@ size_t prior_ws_bytes(int64_t rows, const PriorPlan& pl, int32_t C, int32_t P) {
          align256(size_t(rows) * 4) + align256(size_t(rows) * C * 4);
 }
 
+// Room for the members' logits of a batch whose output is fused.
 size_t prior_vals_bytes(int64_t rows, int64_t vocab, int32_t cap) {
-  return size_t(rows) * ((vocab + BPD_SOFT_MEMBER_CHUNK - 1) / BPD_SOFT_MEMBER_CHUNK) * cap * 4;
+  const int64_t chunks = rows * ((vocab + BPD_SOFT_MEMBER_CHUNK - 1) / BPD_SOFT_MEMBER_CHUNK);
+  return chunks <= kFusedChunks ? size_t(chunks) * cap * 4 : 0;
 }
 
 size_t prior_lds_bytes(int32_t S, int32_t C, int32_t P, int64_t pairs, bool pairs_in_lds, bool pieces) {
@@ -1199,10 +1208,15 @@ __global__ __launch_bounds__(kPriorThreads) void prior_stats_list_kernel(
     mm[j] = ch < nchunks ? members[ch * Cap + (j % kHalf) * kPriorThreads + threadIdx.x] : 0xFFFFFFFFu;
   }
   float4 x[kWideLoads];
+  if (base + kWideChunk <= V) {
 #pragma unroll
-  for (int u = 0; u < kWideLoads; ++u) {
-    const int64_t t = base + (int64_t(u) * kPriorThreads + threadIdx.x) * 4;
-    x[u] = load_tokens(row, t, V);
+    for (int u = 0; u < kWideLoads; ++u) {
+      const F4u v = *reinterpret_cast<const F4u*>(row + base + (u * kPriorThreads + threadIdx.x) * 4);
+      x[u] = make_float4(v[0], v[1], v[2], v[3]);
+    }
+  } else {
+#pragma unroll
+    for (int u = 0; u < kWideLoads; ++u) x[u] = load_tokens(row, base + (u * kPriorThreads + threadIdx.x) * 4, V);
   }
   for (int32_t c = threadIdx.x; c < kWaves * C; c += kPriorThreads) wsum[c] = 0.0f;
   float m = -INFINITY;
@@ -1622,12 +1636,11 @@ __device__ __forceinline__ void prior_out_chunks(const PriorOut& out, int64_t ld
   }
 }
 
-// Out: the member-list output follows in the same launch, grid (splits, rows),
-// every block of a row running its rounds (the EOS logit then comes from the
-// statistics: another block of the row may have written its output already).
-// [128, 151936], 71 states, k = 4: 24.0 us (9.6 until the rounds are done),
-// where a launch of one block per row took 10.0 and a gathering output launch
-// after it 21.4; two blocks per CU, whose rounds share its LDS, 24.9.
+// Out (kFusedChunks): the member-list output follows in the same launch, grid
+// (splits, rows), every block of a row running its rounds (the EOS logit then
+// comes from the statistics: another block of the row may have written its
+// output already).  One block per CU: two share its LDS, and the rounds of
+// each wait for the other's reads ([128, 151936]: 24.9 us against 24.0).
 template <bool PairsInLds, bool ClassStats, bool Out>
 __global__ __launch_bounds__(kRoundThreads) void prior_rounds_kernel(
     const float* logits, int64_t ld, int32_t S, int G, BpdSoftClasses cls,
@@ -1771,7 +1784,10 @@ __global__ __launch_bounds__(kRoundThreads) void prior_rounds_kernel(
                      int(blockIdx.x), int(gridDim.x));
   } else {
     for (int32_t c = tid; c < C; c += kRoundThreads) ws.zcls[b * C + c] = lc[c];
-    if (tid == 0) ws.lse[b] = lse;
+    if (tid == 0) {
+      ws.lse[b] = lse;
+      ws.part[b * G * 2] = low;  // this block has read the row's partials
+    }
   }
 }
 
@@ -1854,6 +1870,73 @@ __global__ __launch_bounds__(kPriorOutThreads) void prior_out_kernel(
       const int64_t t = base + int64_t(u) * kPriorOutThreads + threadIdx.x;
       if (t < V) row[t] = prior_value(row[t], lse, t, zof(token_class[t]), acc_s, eos, alpha);
     }
+  }
+}
+
+// Member-list output of a large batch, grid (ceil(V / 4096), rows): block g
+// rewrites the 4096-token member chunk g of its row.  The chunk is staged in
+// LDS as -inf; the threads take the chunk's member list (Cap slots,
+// 0xFFFFFFFF empty) and put x - lse + alpha * z there for the members whose
+// class has a finite value (EOS: its log softmax when the state accepts); the
+// chunk then goes out as coalesced 16-byte non-temporal stores (every line
+// written whole; nothing reads the rows again in this call).
+template <int Cap>
+__global__ __launch_bounds__(kPriorOutThreads) void prior_out_list_kernel(
+    float* __restrict__ logits, int64_t ld, int64_t V, const uint32_t* __restrict__ members, int32_t C, int G,
+    PriorWs ws, int32_t S, const uint8_t* __restrict__ accept, int32_t eos, const int32_t* __restrict__ states,
+    const int64_t* __restrict__ slots, float alpha, int32_t* __restrict__ err) {
+  constexpr int kSlots = Cap / kPriorOutThreads;
+  constexpr int kGroups = BPD_SOFT_MEMBER_CHUNK / 4 / kPriorOutThreads;  // float4 groups per thread
+  __shared__ float4 outs[BPD_SOFT_MEMBER_CHUNK / 4];
+  __shared__ float zs[kLdsClasses];
+  const int64_t b = blockIdx.y;
+  const int64_t base = int64_t(blockIdx.x) * BPD_SOFT_MEMBER_CHUNK;
+  const int32_t s = states[slots ? slots[b] : b];
+  const bool live_row = s >= 0 && s < S;
+  if (s >= S && err && blockIdx.x == 0 && threadIdx.x == 0) atomicOr(err, BPD_FLAG_STATE_RANGE);
+  float* row = logits + b * ld;
+  const float4 ninf = make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
+#pragma unroll
+  for (int q = 0; q < kGroups; ++q) outs[q * kPriorOutThreads + threadIdx.x] = ninf;
+  if (!live_row) __syncthreads();  // the partial chunk below is read across threads
+  if (live_row) {  // the same in every thread
+    uint32_t mm[kSlots];
+    float xv[kSlots], zv[kSlots];
+#pragma unroll
+    for (int j = 0; j < kSlots; ++j) mm[j] = members[int64_t(blockIdx.x) * Cap + j * kPriorOutThreads + threadIdx.x];
+    const float* zrow = ws.zcls + b * C;
+    for (int32_t c = threadIdx.x; c < C; c += kPriorOutThreads) zs[c] = zrow[c];
+    const float lse = ws.lse[b], low = ws.part[b * G * 2];
+    const bool acc_s = accept[s] != 0;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kSlots; ++j) {
+      zv[j] = -INFINITY;
+      if (mm[j] != 0xFFFFFFFFu && base + int64_t(mm[j] >> 16) != eos) zv[j] = zs[mm[j] & 0xFFFFu];
+      xv[j] = zv[j] != -INFINITY ? row[base + int64_t(mm[j] >> 16)] : 0.0f;
+    }
+    float* of = reinterpret_cast<float*>(outs);
+#pragma unroll
+    for (int j = 0; j < kSlots; ++j) {
+      if (zv[j] != -INFINITY) {
+        const float lp = (xv[j] - lse) - low;
+        of[mm[j] >> 16] = alpha != 0.0f ? fmaf(alpha, zv[j], lp) : lp;
+      }
+    }
+    if (threadIdx.x == 0 && acc_s && eos >= base && eos < base + BPD_SOFT_MEMBER_CHUNK)
+      of[eos - base] = (row[eos] - lse) - low;
+    __syncthreads();
+  }
+  float* to = row + base + threadIdx.x * 4;
+  if (base + BPD_SOFT_MEMBER_CHUNK <= V) {
+#pragma unroll
+    for (int q = 0; q < kGroups; ++q) {
+      const float4 o = outs[q * kPriorOutThreads + threadIdx.x];
+      __builtin_nontemporal_store(F4u{o.x, o.y, o.z, o.w}, reinterpret_cast<F4u*>(to + q * kPriorOutThreads * 4));
+    }
+  } else {
+    for (int64_t t = threadIdx.x; base + t < V; t += kPriorOutThreads)
+      row[base + t] = reinterpret_cast<const float*>(outs)[t];
   }
 }
 
@@ -1946,7 +2029,7 @@ int soft_prior_impl(float* logits, int64_t rows, int64_t vocab, int64_t ld, int3
   // room for the members' logits: the output then reads them in order instead
   // of gathering them from the rows
   const size_t common = align256(bpd_soft_prior_workspace_bytes(rows, vocab, cls.num_classes, cls.num_pieces));
-  if (workspace_bytes >= common + prior_vals_bytes(rows, vocab, cls.chunk_cap))
+  if (rows * nchunks <= kFusedChunks && workspace_bytes >= common + prior_vals_bytes(rows, vocab, cls.chunk_cap))
     ws.vals = reinterpret_cast<float*>(static_cast<char*>(workspace) + common);
   const bool vec = vocab % 4 == 0 && ld % 4 == 0 && aligned16(logits) && aligned16(cls.token_class);
   if (pl.class_stats) {
@@ -2000,7 +2083,8 @@ int soft_prior_impl(float* logits, int64_t rows, int64_t vocab, int64_t ld, int3
   prior_rounds_kernel<LDSP, CLS, OUT><<<rgrid, kRoundThreads, rlds, st>>>(                          \
       logits, ld, num_states, pl.G, cls, accept, live, eos_id, states, slots, k - 1, ws,            \
       PriorOut{logits, vocab, alpha, err})
-  const bool list = list_ok && pl.class_stats;
+  const bool list_out = list_ok && pl.class_stats;
+  const bool list = list_out && rows * nchunks <= kFusedChunks;
   dim3 rgrid = dim3(unsigned(rows));
   size_t rlds = lds;
   if (list) {
@@ -2018,6 +2102,19 @@ int soft_prior_impl(float* logits, int64_t rows, int64_t vocab, int64_t ld, int3
 #undef BPD_PRIOR_ROUNDS
   BPD_LAUNCHED();
   if (list) return BPD_OK;
+  if (list_out) {
+    const dim3 lgrid = dim3(unsigned(nchunks), unsigned(rows));
+#define BPD_PRIOR_OUT_LIST(CAP)                                                                           \
+  prior_out_list_kernel<CAP><<<lgrid, kPriorOutThreads, 0, st>>>(                                         \
+      logits, ld, vocab, cls.chunk_members, cls.num_classes, pl.G, ws, num_states, accept, eos_id, states, \
+      slots, alpha, err)
+    if (cls.chunk_cap == 256) BPD_PRIOR_OUT_LIST(256);
+    else if (cls.chunk_cap == 512) BPD_PRIOR_OUT_LIST(512);
+    else BPD_PRIOR_OUT_LIST(1024);
+#undef BPD_PRIOR_OUT_LIST
+    BPD_LAUNCHED();
+    return BPD_OK;
+  }
   const dim3 ogrid = dim3(unsigned((vocab + 4 * kOutLoads * kPriorOutThreads - 1) /
                                    (4 * kOutLoads * kPriorOutThreads)),
                           unsigned(rows));
