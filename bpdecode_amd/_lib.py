@@ -107,6 +107,7 @@ _SIGNATURES = {
     "bpd_stage_int64": (cint, [vp, vp, i64, vp]),
     "bpd_pda_init": (cint, [C.POINTER(PdaTableC), vp]),
     "bpd_pda_reset": (cint, [vp, vp, i64, vp, vp, i64, cint, vp]),
+    "bpd_pda_rows": (cint, [vp, vp, i64, vp, vp, i64, i64, vp, vp]),
     "bpd_pda_feed": (cint, [C.POINTER(PdaTableC), vp, C.c_char_p, i64]),
     "bpd_host_frame_classify": (cint, [vp, i32, vp, vp, i32, i32, vp, vp, vp, vp, vp, i32]),
     "bpd_host_frame_lists": (cint, [C.POINTER(PdaTableC), i32, vp, vp, vp]),

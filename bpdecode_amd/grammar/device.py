@@ -21,6 +21,7 @@ from __future__ import annotations
 import array
 import ctypes as C
 import hashlib
+import struct
 from collections.abc import Hashable, Sequence
 from dataclasses import dataclass, field, replace
 
@@ -580,7 +581,20 @@ class CFGConstraintBatch:
 
         key = (self._version, tuple(seq_ids))
         if key != self._slot_key:
-            self._slot_tensor = index_tensor([self._slot_of[s] for s in seq_ids], self.device)
+            vals = [self._slot_of[s] for s in seq_ids]
+            n = len(vals) + len(self._resets)
+            if self.device.type == "cuda" and vals and n <= _lib.MAX_INLINE_VALUES and (
+                    not self._resets or _lib.stream_of(self.device) == 0):
+                # the list and the queued resets in one launch's arguments
+                out = torch.empty(len(vals), dtype=torch.int64, device=self.device)
+                resets, self._resets = self._resets, {}
+                with torch.cuda.device(self.device):
+                    check(lib().bpd_pda_rows(ptr(self._pool), ptr(self._flags), self.capacity, ptr(self._init),
+                                             struct.pack(f"{n}i", *vals, *resets), len(vals), len(resets),
+                                             ptr(out), _lib.stream_of(self.device)))
+                self._slot_tensor = out
+            else:
+                self._slot_tensor = index_tensor(vals, self.device)
             self._slot_key = key
         return self._slot_tensor
 

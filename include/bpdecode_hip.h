@@ -402,6 +402,13 @@ int bpd_pda_init(const BpdPdaTable* g, int32_t* config_out);
 int bpd_pda_reset(int32_t* configs, uint8_t* broken, int64_t capacity, const int32_t* init,
                   const int64_t* slots, int64_t n, int wait, void* stream);
 
+/* bpd_pda_rows: bpd_pda_reset for `resets` slots, and the batch's slot list to
+ * slots_out (device, rows int64), in one launch: HOST `values` holds rows
+ * slots, then the slots to reset (at most BPD_MAX_INLINE_VALUES in all). */
+int bpd_pda_rows(int32_t* configs, uint8_t* broken, int64_t capacity, const int32_t* init,
+                 const int32_t* values, int64_t rows, int64_t resets, int64_t* slots_out,
+                 void* stream);
+
 /* bpd_pda_feed: host only; consume `n` raw bytes into one config-set in place
  * (pda_advance_byte per byte, pda.hpp:211-236).  Returns 1 when every byte
  * kept the set non-empty (config updated), 0 when a byte emptied it (config
