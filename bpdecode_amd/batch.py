@@ -502,8 +502,11 @@ class ConstraintBatch:
             raise ValueError("fsa has no lookahead table; build with dense + with_lookahead")
         code = _SOFT_CODES.get(logits.dtype)
         la = self.fsa.lookahead
+        # a table that lies elsewhere (replace(fsa, lookahead=...)) goes to the
+        # checked path, which raises
         if (self._fast and code is not None and self._fast_logits(logits, len(seq_ids))
-                and la.dtype == torch.float32 and la.is_contiguous() and la.shape[1] == self._V):
+                and la.device == self.device and la.dtype == torch.float32 and la.is_contiguous()
+                and la.shape[1] == self._V):
             B = len(seq_ids)
             ld = logits.stride(0) if B > 1 else self._V
             stream = _lib.stream_of(self.device)
@@ -531,9 +534,12 @@ class ConstraintBatch:
         plus ``alpha`` times the log-probability, under the row's own
         softmax, of staying on a live path for ``k - 1`` further tokens
         (``-inf`` on grammar-disallowed tokens)."""
-        if (self._fast and logits.dtype == torch.float32 and k >= 1 and self.fsa.tok_next is not None
-                and self._fast_logits(logits, len(seq_ids))):
-            fsa, V, B = self.fsa, self._V, len(seq_ids)
+        fsa = self.fsa
+        tn = fsa.tok_next
+        if (self._fast and logits.dtype == torch.float32 and k >= 1 and tn is not None
+                and self._fast_logits(logits, len(seq_ids)) and tn.shape == (self._S, self._V)
+                and tn.device == fsa.accept.device == fsa.live.device == self.device):
+            V, B = self._V, len(seq_ids)
             sc = fsa.ensure_soft_classes()
             acc, live = fsa.accept.contiguous(), fsa.live.contiguous()
             eos = fsa.eos_id if fsa.eos_id is not None and 0 <= fsa.eos_id < V else -1
@@ -553,7 +559,7 @@ class ConstraintBatch:
                 self._launched()
             return logits
         slots = self._slots(seq_ids)
-        ops.apply_soft_prior_(logits, self.fsa, self._state, k, alpha, slots=slots, err=self._err)
+        ops.apply_soft_prior_(logits, fsa, self._state, k, alpha, slots=slots, err=self._err)
         return logits
 
     def commit(self, seq_ids: Sequence[Hashable], tokens: torch.Tensor) -> torch.Tensor:

@@ -749,7 +749,7 @@ def apply_soft_prior_(logits: torch.Tensor, fsa: FsaTensors, states: torch.Tenso
         raise ValueError("k must be >= 1")
     base = fsa if fsa.tok_next is not None else fsa.densify()
     tn = base.tok_next.contiguous()
-    dev = _same_device(logits, tn, states, slots)
+    dev = _same_device(logits, tn, base.accept, base.live, states, slots)
     work, copied = _unit_stride_rows(logits)
     B, V = work.shape
     S, TV = tn.shape

@@ -4,11 +4,15 @@ an absolute floor of 1e-5; -inf pattern exact)."""
 
 from __future__ import annotations
 
+from dataclasses import replace
+
 import numpy as np
 import pytest
 import torch
 
-from bpdecode_amd import ops, synth
+from bpdecode_amd import _lib, ops, synth
+from bpdecode_amd import batch as batch_mod
+from bpdecode_amd.batch import ConstraintBatch
 from bpdecode_amd.ops import FsaTensors, SoftClasses
 from oracle import soft as OS
 from tests._util import TOY_PATTERNS, TOY_VOCAB, reachable
@@ -142,3 +146,73 @@ def test_host_prior_non_contiguous_rows():
                               fsa.accept.numpy(), fsa.eos_id, st.numpy(), 3, 0.5)
     ops.apply_soft_prior_(view, fsa, st, 3, 0.5)
     assert close(wide[:, :V].double().numpy(), want)
+
+
+class _NoLaunch:
+    """Stands for the library: fails on a device launch and counts nothing
+    else (the sizes that a launch's preparation asks for are 0)."""
+
+    def __getattr__(self, name):
+        if "workspace" in name:
+            return lambda *args: 0
+        return lambda *args: pytest.fail(f"{name} was launched")
+
+
+def _device_form(monkeypatch, fsa: FsaTensors, rows: int) -> ConstraintBatch:
+    """A batch on the host that takes the device's fast path, with launches
+    refused: what its conditions let through reaches :class:`_NoLaunch`."""
+    batch = ConstraintBatch(fsa, capacity=rows)
+    for i in range(rows):
+        batch.add(i)
+    batch._fast = True
+    batch._S, batch._V, batch._W = fsa.num_states, fsa.vocab_size, (fsa.vocab_size + 31) // 32
+    batch._pool_ptr, batch._err_ptr, batch._bits_ptr = batch._pool.data_ptr(), 0, 0
+    fsa.ensure_soft_classes()
+    monkeypatch.setattr(_lib, "stream_of", lambda device: 0)
+    monkeypatch.setattr(batch_mod, "lib", _NoLaunch)
+    return batch
+
+
+def test_fast_path_refuses_a_lookahead_on_another_device(monkeypatch):
+    """The lookahead table's address goes to a kernel only if the table lies
+    on the batch's device ("meta" stands for another one)."""
+    fsa = FsaTensors.build("a[012]+|b0", TOY_VOCAB).densify().with_lookahead(3)
+    x = torch.zeros(2, fsa.vocab_size)
+    batch = _device_form(monkeypatch, replace(fsa, lookahead=fsa.lookahead.to("meta")), 2)
+    with pytest.raises(RuntimeError, match="same device"):
+        batch.apply_soft([0, 1], x)
+    batch = _device_form(monkeypatch, fsa, 2)
+    with pytest.raises(pytest.fail.Exception, match="bpd_soft_apply"):  # its own table goes on to the launch
+        batch.apply_soft([0, 1], x)
+
+
+@pytest.mark.parametrize("field", ["tok_next", "accept", "live"])
+def test_fast_path_refuses_prior_tables_on_another_device(monkeypatch, field):
+    fsa = FsaTensors.build("a[012]+|b0", TOY_VOCAB).densify()
+    x = torch.zeros(2, fsa.vocab_size)
+    batch = _device_form(monkeypatch, fsa, 2)
+    with pytest.raises(pytest.fail.Exception, match="bpd_soft_prior"):
+        batch.apply_soft_prior([0, 1], x)
+    batch.fsa = replace(fsa, **{field: getattr(fsa, field).to("meta")})
+    with pytest.raises(RuntimeError, match="same device"):
+        batch.apply_soft_prior([0, 1], x)
+
+
+@pytest.mark.parametrize("cut", [0, 1])
+def test_fast_path_refuses_a_prior_table_of_another_shape(monkeypatch, cut):
+    """Fewer columns than the logits are refused; fewer rows than the grammar
+    has states are no reason to refuse, but the states are then bounded by
+    the table and not by the grammar."""
+    fsa = FsaTensors.build("a[012]+|b0", TOY_VOCAB).densify()
+    S, V = fsa.tok_next.shape
+    batch = _device_form(monkeypatch, fsa, 2)
+    batch.fsa = replace(fsa, tok_next=fsa.tok_next[:S - cut, :V - 1 + cut].contiguous())
+    x = torch.zeros(2, V)
+    if cut:
+        batch.apply_soft_prior([0, 1], x)  # the general path, on the host here
+        want = torch.zeros(2, V)
+        ops.apply_soft_prior_(want, batch.fsa, torch.full((2,), fsa.start, dtype=torch.int32))
+        assert torch.equal(x, want)
+    else:
+        with pytest.raises(RuntimeError, match="columns"):
+            batch.apply_soft_prior([0, 1], x)
