@@ -11,6 +11,7 @@
 // row with an online (max, sum-exp) pair per thread and a tree merge in LDS.
 // Rounds ping-pong two logZ vectors in the caller's workspace.  A last pass
 // writes out[s, t] = logZ(tok_next[s, t]).
+#include <algorithm>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
@@ -481,7 +482,8 @@ int launch_soft_apply(uint8_t* logits, int64_t rows, int64_t vocab, int64_t ld_b
   const int64_t wide = (vocab + kApplyThreads * N * kWide - 1) / (kApplyThreads * N * kWide);
   const bool many = wide * rows >= 1024;
   const int64_t chunks = many ? wide : (vocab + kApplyThreads * N - 1) / (kApplyThreads * N);
-  const int64_t blocks = (chunks * rows + kXcds - 1) / kXcds * kXcds;
+  // an empty vocabulary has no chunks, but block 0 still makes the queued writes
+  const int64_t blocks = (std::max<int64_t>(chunks * rows, 1) + kXcds - 1) / kXcds * kXcds;
   BPD_REQUIRE(blocks < (int64_t(1) << 31), "batch too large for one launch");
 #define BPD_SOFT_APPLY(U, NA, INL)                                                                     \
   soft_apply_kernel<D, U, NA><<<dim3(unsigned(blocks)), kApplyThreads, 0, st>>>(                       \

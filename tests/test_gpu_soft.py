@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 import torch
 
-from bpdecode_amd import ops, synth
+from bpdecode_amd import _lib, ops, synth
 from bpdecode_amd._lib import check, lib, stream_of
 from bpdecode_amd.batch import ConstraintBatch
 from bpdecode_amd.ops import FsaTensors
@@ -149,6 +149,26 @@ def test_apply_soft_carries_queued_writes(dev):
     assert [batch.state_of(i) for i in ids] == states
     nxt = batch.commit(ids, torch.full((5,), tok, dtype=torch.int64, device=dev)).tolist()
     assert nxt == [int(fsa.tok_next[s, tok]) if s >= 0 else -1 for s in states]
+
+
+@pytest.mark.parametrize("rows", [1, 9])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_apply_soft_of_an_empty_vocabulary_makes_queued_writes(dev, rows, dtype):
+    """No logits to change, but the pool writes that travel with the call are
+    made."""
+    pool = torch.arange(12, dtype=torch.int32, device=dev)
+    la = torch.empty(3, 0, device=dev)
+    x = torch.empty(rows, 0, dtype=dtype, device=dev)
+    slots = torch.arange(rows, dtype=torch.int64, device=dev)
+    pending = torch.tensor([2, 7, 11, 1, -1, 2], dtype=torch.int64, device=dev)  # three slots, three values
+    code = {torch.float32: _lib.DTYPE_F32, torch.bfloat16: _lib.DTYPE_BF16}[dtype]
+    want = pool.clone()
+    for n in (0, 3):
+        check(lib().bpd_soft_apply_queued(x.data_ptr(), code, rows, 0, 0, la.data_ptr(), 3, pool.data_ptr(),
+                                          slots.data_ptr(), pending.data_ptr(), n, 0.5, None, stream_of(dev)))
+        if n:
+            want[pending[:3]] = pending[3:].to(torch.int32)
+        assert torch.equal(pool, want), n
 
 
 @pytest.mark.parametrize("vocab", ["v17", "v20"])
