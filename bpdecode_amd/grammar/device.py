@@ -514,8 +514,8 @@ class CFGConstraintBatch:
             return
         direct = _lib.stream_of(self.device) != 0
         if self._resets:
-            slots, self._resets = self._resets, {}
-            self._launch_resets(slots, 0, direct)
+            self._launch_resets(self._resets, 0, direct)
+            self._resets.clear()  # a launch that failed leaves them queued
         if direct:
             self._queueing = False
 
@@ -587,11 +587,11 @@ class CFGConstraintBatch:
                     not self._resets or _lib.stream_of(self.device) == 0):
                 # the list and the queued resets in one launch's arguments
                 out = torch.empty(len(vals), dtype=torch.int64, device=self.device)
-                resets, self._resets = self._resets, {}
                 with torch.cuda.device(self.device):
                     check(lib().bpd_pda_rows(ptr(self._pool), ptr(self._flags), self.capacity, ptr(self._init),
-                                             struct.pack(f"{n}i", *vals, *resets), len(vals), len(resets),
-                                             ptr(out), _lib.stream_of(self.device)))
+                                             struct.pack(f"{n}i", *vals, *self._resets), len(vals),
+                                             len(self._resets), ptr(out), _lib.stream_of(self.device)))
+                self._resets.clear()
                 self._slot_tensor = out
             else:
                 self._slot_tensor = index_tensor(vals, self.device)

@@ -6,6 +6,8 @@ checked against an independent recursive matcher of the grammar."""
 
 from __future__ import annotations
 
+import contextlib
+import ctypes
 import itertools
 import random
 
@@ -14,6 +16,7 @@ import pytest
 import torch
 
 from bpdecode_amd import synth
+from bpdecode_amd.grammar import device as pda_device
 from bpdecode_amd.grammar.device import (
     PDA_CONFIG_FLAT, CFGConstraintBatch, build_pda_tensors, pda_advance_state, pda_apply_mask_,
     _walk_order, pda_compute_mask, pda_mask_, pda_step,
@@ -468,3 +471,53 @@ def test_feed_rejects_a_malformed_config_set():
     with pytest.raises(RuntimeError, match="malformed"):
         g.feed(bad, b"x")
     assert not g.feed(c, b"]")
+
+
+@pytest.mark.parametrize("through", ["the next mask", "the slot list", "another stream"])
+def test_resets_stay_queued_when_their_launch_fails(monkeypatch, through):
+    """A launch that is refused (or fails) leaves the resets queued, and the
+    next use of the pool makes them: no slot keeps an evicted request's
+    config-set.  The device form on host tensors, the launches stood in for."""
+    calls, refuse = [], [True]
+
+    class Launches:
+        def _made(self, slots):
+            if refuse[0]:
+                return 2
+            calls.append(list(slots))
+            return 0
+
+        def bpd_pda_reset(self, pool, flags, capacity, init, addr, n, wait, stream):
+            return self._made((ctypes.c_int64 * n).from_address(addr))
+
+        def bpd_pda_rows(self, pool, flags, capacity, init, values, rows, resets, out, stream):
+            return self._made(np.frombuffer(values, dtype=np.int32)[rows:].tolist())
+
+    def failing_check(rc):
+        if rc:
+            raise RuntimeError("refused")
+
+    g, _ = tables(GRAMMARS[0], False)
+    batch = CFGConstraintBatch(g, 4)
+    stream = [0]
+    empty = torch.empty
+    monkeypatch.setattr(pda_device, "lib", Launches)
+    monkeypatch.setattr(pda_device, "check", failing_check)
+    monkeypatch.setattr(pda_device._lib, "stream_of", lambda device: stream[0])
+    monkeypatch.setattr(pda_device.torch, "empty", lambda *a, **kw: empty(*a, dtype=kw["dtype"]))
+    monkeypatch.setattr(pda_device.torch.cuda, "device", lambda device: contextlib.nullcontext())
+    batch.device, batch._queueing = torch.device("cuda", 0), True
+    for i in range(3):
+        batch.add(i)
+    if through == "another stream":
+        stream[0] = 7
+    use = (lambda: batch._slots([2, 0])) if through == "the slot list" else batch._flush
+    with pytest.raises(RuntimeError, match="refused"):
+        use()
+    assert list(batch._resets) == [0, 1, 2]
+    refuse[0] = False
+    use()
+    assert calls == [[0, 1, 2]] and not batch._resets
+    use()
+    assert calls == [[0, 1, 2]]
+    assert batch._queueing == (through != "another stream")
