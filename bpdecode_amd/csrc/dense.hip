@@ -50,6 +50,8 @@ template <> struct Elem<8> { using T = uint64_t; };
 // row and 4 consecutive chunks; logical blocks are numbered column-group
 // major, so one XCD's L2 serves a contiguous band of table columns to every
 // row.  The block with logical index 0 also applies the queued pool writes.
+// The columns of `vocab` past `tokens` (a padded lm_head) are rejected in
+// every row, whatever the bits past `tokens` in a row's last word.
 // N: slots and queued writes come in the arguments (rows.hpp), and block 0
 // leaves the slots in slots_out: [33, 100003] fp16 and two requests turning
 // over: a step of 16.1 us, 18.5 with an upload before the launch (256 rows of
@@ -57,7 +59,7 @@ template <> struct Elem<8> { using T = uint64_t; };
 template <int E, bool Bits, int N>
 __global__ __launch_bounds__(kFillThreads) void dense_fill_kernel(
     uint8_t* __restrict__ logits, int64_t ld_bytes, const void* __restrict__ table,
-    int64_t table_ld, int64_t vocab, int32_t num_states, int32_t* states,
+    int64_t table_ld, int64_t vocab, int64_t tokens, int32_t num_states, int32_t* states,
     const int64_t* __restrict__ slots, const int64_t* __restrict__ pending, int32_t num_pending,
     uint32_t rows, uint32_t chunks, uint64_t fill, int32_t* __restrict__ err, InlineRows<N> inl,
     int64_t* __restrict__ slots_out) {
@@ -84,7 +86,8 @@ __global__ __launch_bounds__(kFillThreads) void dense_fill_kernel(
   if (Bits) {
     const uint32_t* bw = static_cast<const uint32_t*>(table);
     const int64_t w = c0 / 32 + lane;
-    const uint32_t mine = (live && w < table_ld) ? bw[int64_t(s) * table_ld + w] : 0u;
+    uint32_t mine = (live && w < table_ld) ? bw[int64_t(s) * table_ld + w] : 0u;
+    if (w == tokens >> 5) mine &= (1u << (tokens & 31)) - 1;  // a caller's table may have bits there
     const uint32_t lanebit = 1u << (lane & 31);
 #pragma unroll
     for (int j = 0; j < kFillGroups; ++j) {
@@ -475,8 +478,9 @@ using namespace bpd;
 
 namespace {
 
-// Shared launch of the write-only mask (both table forms).
-int launch_fill(void* logits, int dtype, int64_t rows, int64_t vocab, int64_t ld, const void* table,
+// Shared launch of the write-only mask (both table forms): `vocab` columns,
+// of which the first `tokens` have verdicts in the table.
+int launch_fill(void* logits, int dtype, int64_t rows, int64_t vocab, int64_t tokens, int64_t ld, const void* table,
                 int64_t table_ld, bool bits, int32_t num_states, int32_t* states,
                 const int64_t* slots, const int64_t* pending, int64_t num_pending, double neg_inf,
                 int32_t* err, void* stream, const int32_t* inline_values = nullptr,
@@ -503,7 +507,7 @@ int launch_fill(void* logits, int dtype, int64_t rows, int64_t vocab, int64_t ld
   const int32_t np = int32_t(num_pending);
 #define BPD_FILL(EB, BITS, N, INL)                                                              \
   dense_fill_kernel<EB, BITS, N><<<dim3(unsigned(blocks)), dim3(kFillThreads), 0, s>>>(         \
-      lg, ld * EB, table, table_ld, vocab, num_states, states, slots, pending, np,              \
+      lg, ld * EB, table, table_ld, vocab, tokens, num_states, states, slots, pending, np,      \
       uint32_t(rows), uint32_t(chunks), fill, err, INL, slots_out)
   if (inline_values) {
     return with_inline_rows(inline_values, rows + 2 * num_pending, [&](const auto& inl) -> int {
@@ -537,7 +541,7 @@ extern "C" int bpd_dense_apply_mask(void* logits, int dtype, int64_t rows, int64
                                     int32_t* states, const int64_t* slots,
                                     const int64_t* pending, int64_t num_pending, double neg_inf,
                                     int32_t* err, void* stream) {
-  return launch_fill(logits, dtype, rows, vocab, ld, tok_next, vocab, false, num_states, states,
+  return launch_fill(logits, dtype, rows, vocab, vocab, ld, tok_next, vocab, false, num_states, states,
                      slots, pending, num_pending, neg_inf, err, stream);
 }
 
@@ -548,7 +552,7 @@ extern "C" int bpd_dense_apply_mask_bits(void* logits, int dtype, int64_t rows, 
                                          int64_t num_pending, double neg_inf, int32_t* err,
                                          void* stream) {
   BPD_REQUIRE(words == (vocab + 31) / 32, "allow-bit rows must hold ceil(vocab/32) words");
-  return launch_fill(logits, dtype, rows, vocab, ld, allow_bits, words, true, num_states, states,
+  return launch_fill(logits, dtype, rows, vocab, vocab, ld, allow_bits, words, true, num_states, states,
                      slots, pending, num_pending, neg_inf, err, stream);
 }
 
@@ -559,8 +563,7 @@ extern "C" int bpd_dense_apply_mask_padded(void* logits, int dtype, int64_t rows
                                            int32_t* err, void* stream) {
   BPD_REQUIRE(words == (vocab + 31) / 32, "allow-bit rows must hold ceil(vocab/32) words");
   BPD_REQUIRE(cols >= vocab, "fewer columns than tokens");
-  // a column past the table's words, or past vocab in its last one, is rejected
-  return launch_fill(logits, dtype, rows, cols, ld, allow_bits, words, true, num_states, states,
+  return launch_fill(logits, dtype, rows, cols, vocab, ld, allow_bits, words, true, num_states, states,
                      slots, pending, num_pending, neg_inf, err, stream);
 }
 
@@ -572,7 +575,7 @@ extern "C" int bpd_dense_apply_mask_inline(void* logits, int dtype, int64_t rows
   BPD_REQUIRE(words == (vocab + 31) / 32, "allow-bit rows must hold ceil(vocab/32) words");
   BPD_REQUIRE(cols >= vocab, "fewer columns than tokens");
   if (int rc = check_inline(values, rows, num_pending, states, slots_out)) return rc;
-  return launch_fill(logits, dtype, rows, cols, ld, allow_bits, words, true, num_states, states, nullptr,
+  return launch_fill(logits, dtype, rows, cols, vocab, ld, allow_bits, words, true, num_states, states, nullptr,
                      nullptr, num_pending, neg_inf, err, stream, values, slots_out);
 }
 

@@ -105,8 +105,8 @@ int bpd_dense_apply_mask_bits(void* logits, int dtype, int64_t rows, int64_t voc
 
 /* bpd_dense_apply_mask_padded: the same mask over logits of `cols` >= vocab
  * columns (a padded lm_head): the columns past vocab are rejected in every
- * row.  The bits past vocab in a table row's last word are zero, as the
- * builders leave them (hf.py:106-113 masks those columns on its own). */
+ * row, whatever the bits past vocab in a table row's last word
+ * (hf.py:106-113 masks those columns on its own). */
 int bpd_dense_apply_mask_padded(void* logits, int dtype, int64_t rows, int64_t vocab, int64_t cols,
                                 int64_t ld, const uint32_t* allow_bits, int64_t words,
                                 int32_t num_states, int32_t* states, const int64_t* slots,

@@ -415,3 +415,29 @@ def test_generation_step_padded_columns_and_strided_ids(dev, dense, rows):
     batch.commit(ids, torch.full((rows, 2), V, device=dev)[:, -1])
     with pytest.raises(IndexError):
         batch.check_errors()
+
+
+@pytest.mark.parametrize("V", [1, 17, 31, 32, 33, 2047, 2049, 8195])
+@pytest.mark.parametrize("pad", [1, 14, 15, 40, 2100])
+def test_padded_columns_are_rejected_whatever_the_table_tail_holds(dev, V, pad):
+    """A caller's own allow-bit table whose bits past the vocabulary are set:
+    the padded columns are filled all the same, in the launch that carries
+    the slots in its arguments and in the one that reads them."""
+    _log(f"case table tail V={V} pad={pad}")
+    fd = replace(random_bundle(3, 4, V, seed=V, max_len=3), tok_next=None).to(dev)
+    words = (V + 31) // 32
+    g = torch.Generator().manual_seed(V + pad)
+    bits = torch.randint(0, 2, (3, words * 32), generator=g, dtype=torch.bool)
+    bits[:, V:] = True
+    packed = (bits.view(3, words, 32).long() << torch.arange(32)).sum(-1)
+    fd.allow_bits = torch.where(packed >= 2**31, packed - 2**32, packed).to(torch.int32).to(dev)
+    batch = ConstraintBatch(fd, capacity=5, device=dev)
+    for i in range(5):
+        batch.add(i)
+    for step in range(2):
+        for dtype in (torch.float32, torch.bfloat16):
+            x = torch.randn(5, V + pad, generator=g).to(dtype)
+            got = batch.apply_mask_padded(list(range(5)), x.to(dev), -7.0)
+            want = torch.full_like(x, -7.0)
+            want[:, :V] = torch.where(bits[fd.start, :V], x[:, :V], want[:, :V])
+            assert torch.equal(got.cpu(), want), (step, dtype)
