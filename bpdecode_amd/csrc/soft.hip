@@ -681,11 +681,14 @@ constexpr int kPriorThreads = 256;
 constexpr int kPriorOutThreads = 256;
 constexpr int64_t kComputeUnits = 256;
 // The rounds and the member-list output in one launch up to this many member
-// chunks in a batch (two for a CU).  There the launches' own time counts: 9
-// rows of 13 chunks 9.3 us, 13.8 as two launches.  Above, a CU's one block
-// cannot keep as many stores in flight as the output launch's blocks: 128
-// rows of 38 chunks 35.0 us against 11.1 + 17.5 with the rows out of the
-// caches (24.2 against 10.0 + 21.6 with rows just written).
+// chunks in a batch, its blocks at most one per CU.  Two launches / one, whole
+// call, [rows, 151936] with 126 classes, rows just written: 1 row (38 chunks)
+// 18.8 / 17.5 us, 7 (266) 20.7 / 19.7, 13 (494) 22.5 / 21.4; past the line 27
+// (1,026) 28.9 / 27.5, 54 (2,052) 32.5 / 32.9, 128 (4,864) 49.5 / 43.5.  Rows out
+// of the caches: 13 rows 25.5 / 24.1, 27 30.6 / 29.6, 54 34.3 / 36.6, 128 52.4 /
+// 56.7: there a CU's one block keeps too few stores in flight.  Up to the line
+// one launch won at every size, grammar and cache state tried; the forms cross
+// between 1,000 and 1,500 chunks.
 constexpr int64_t kFusedChunks = 2 * kComputeUnits;
 constexpr int kPriorMaxStates = 4096;
 constexpr int kPieceMembers = 256;
@@ -1641,8 +1644,9 @@ __device__ __forceinline__ void prior_out_chunks(const PriorOut& out, int64_t ld
 // Out (kFusedChunks): the member-list output follows in the same launch, grid
 // (splits, rows), every block of a row running its rounds (the EOS logit then
 // comes from the statistics: another block of the row may have written its
-// output already).  One block per CU: two share its LDS, and the rounds of
-// each wait for the other's reads ([128, 151936]: 24.9 us against 24.0).
+// output already).  One block per CU at most: blocks beyond that start when
+// others end, a whole chain of rounds later ([9, 151936], 126 classes: 27.8 us a
+// call with 29 blocks a row, 20.3 with 28).
 template <bool PairsInLds, bool ClassStats, bool Out>
 __global__ __launch_bounds__(kRoundThreads) void prior_rounds_kernel(
     const float* logits, int64_t ld, int32_t S, int G, BpdSoftClasses cls,
@@ -2086,13 +2090,12 @@ int soft_prior_impl(float* logits, int64_t rows, int64_t vocab, int64_t ld, int3
       logits, ld, num_states, pl.G, cls, accept, live, eos_id, states, slots, k - 1, ws,            \
       PriorOut{logits, vocab, alpha, err})
   const bool list_out = list_ok && pl.class_stats;
-  const bool list = list_out && rows * nchunks <= kFusedChunks;
+  const bool list = list_out && rows <= kComputeUnits && rows * nchunks <= kFusedChunks;
   dim3 rgrid = dim3(unsigned(rows));
   size_t rlds = lds;
   if (list) {
-    // one block per CU where the rows alone are fewer, at most one per chunk
-    const int64_t want = (kComputeUnits + rows - 1) / rows;
-    rgrid = dim3(unsigned(std::min(want, nchunks)), unsigned(rows));
+    // at most one block per CU and one per chunk
+    rgrid = dim3(unsigned(std::min(kComputeUnits / rows, nchunks)), unsigned(rows));
     rlds = std::max(lds, size_t(cls.num_classes + 3) / 4 * 16 + 2 * size_t(BPD_SOFT_MEMBER_CHUNK) * 4);
   }
   if (list && pairs_in_lds) BPD_PRIOR_ROUNDS(true, true, true);

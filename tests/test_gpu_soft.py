@@ -276,12 +276,14 @@ def test_prior_unaligned_vocab(dev):
 
 @pytest.mark.parametrize("rows,vocab,pad,offset", [
     (1, 4095, 0, 0), (3, 4096, 1, 1), (2, 4097, 2, 3), (5, 8191, 0, 2), (1, 8193, 3, 0), (600, 4099, 0, 0),
+    (60, 20_003, 1, 3), (256, 8100, 0, 1), (257, 4095, 0, 0),
 ])
 @pytest.mark.parametrize("eos", [0, 4094, -1])
 def test_prior_row_shapes(dev, rows, vocab, pad, offset, eos):
     """Member-list kernels at the edges of their chunks (4096 tokens a stage,
     8192 a statistics block), at every alignment of the rows, with more rows
-    than blocks in flight; nothing outside the rows' columns is written."""
+    than blocks in flight, chunks that the blocks of a row share unevenly and
+    rows at and above the CUs; nothing outside the rows' columns is written."""
     S, C = 6, 9
     rng = np.random.default_rng(vocab + rows)
     columns = rng.integers(-1, S, size=(S, C + 1))
