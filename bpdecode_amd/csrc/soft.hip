@@ -5,9 +5,9 @@
 // Table build: k-1 rounds of logZ(s) = logsumexp_t logZ(tok_next[s, t])
 // (logaddexp with 0 for accepting s, -inf off the live set).  A round sums
 // over a state's tokens by the state they lead to, so up to kCountStates
-// states one pass over tok_next counts the tokens of every (state, next)
-// pair, and a round reads those counts alone, one wave per state.  Above
-// that, each round reads the table: one block per state reduces the vocab
+// states and from kCountVocab tokens on one pass over tok_next counts the
+// tokens of every (state, next) pair, and a round reads those counts alone,
+// one wave per state.  Elsewhere each round reads the table: one block per state reduces the vocab
 // row with an online (max, sum-exp) pair per thread and a tree merge in LDS.
 // Rounds ping-pong two logZ vectors in the caller's workspace.  A last pass
 // writes out[s, t] = logZ(tok_next[s, t]).
@@ -28,7 +28,12 @@ namespace {
 
 constexpr int kSoftThreads = 1024;
 constexpr int kMaxLdsStates = 8192;
-constexpr int kCountStates = 512;  // (state, next) counts up to this many states (1 MB)
+// (state, next) counts up to this many states: 1 MB of them.  They would pay
+// above it too, later in V for k = 2 and more for larger k (1,024 states, V =
+// 32,000: 95.5 us with table-reading rounds and 94.4 with counts for k = 2, 181.8
+// and 115.1 for k = 4), at four times the workspace.
+constexpr int kCountStates = 512;
+constexpr int64_t kCountVocab = 6144;  // and from this vocabulary on (bpd_soft_build_lookahead)
 
 struct Lse {
   float m, s;  // value = m + log(s); m = -inf <=> empty
@@ -141,10 +146,22 @@ constexpr int64_t kTableChunk = int64_t(kTableThreads) * 4 * kTableLoads;
 // t = base + (u kTableThreads + tid) 4; -1 past the row's end.
 __device__ __forceinline__ void load_entries(const int32_t* __restrict__ row, int64_t base, int64_t V,
                                              int32_t (&d)[4 * kTableLoads]) {
+  if (base + kTableChunk <= V) {
+#pragma unroll
+    for (int u = 0; u < kTableLoads; ++u) {
+      const I4u v = *reinterpret_cast<const I4u*>(row + base + (u * kTableThreads + int(threadIdx.x)) * 4);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) d[4 * u + q] = v[q];
+    }
+    return;
+  }
 #pragma unroll
   for (int u = 0; u < kTableLoads; ++u) {
-    const int64_t t = base + (int64_t(u) * kTableThreads + threadIdx.x) * 4;
-    if (t + 4 <= V) {
+    const int64_t t = base + (u * kTableThreads + int(threadIdx.x)) * 4;
+    if (base + u * kTableThreads * 4 >= V) {  // for the whole block: a short row costs few tests
+#pragma unroll
+      for (int q = 0; q < 4; ++q) d[4 * u + q] = -1;
+    } else if (t + 4 <= V) {
       const I4u v = *reinterpret_cast<const I4u*>(row + t);
 #pragma unroll
       for (int q = 0; q < 4; ++q) d[4 * u + q] = v[q];
@@ -243,16 +260,18 @@ __global__ __launch_bounds__(kTableThreads) void soft_table_kernel(const int32_t
   const float at_eos = accept[s] ? 0.0f : -INFINITY;
   __syncthreads();
   float* row = out + int64_t(s) * V;
+  const bool whole = base + kTableChunk <= V;  // no group is tested then
 #pragma unroll
   for (int u = 0; u < kTableLoads; ++u) {
-    const int64_t t = base + (int64_t(u) * kTableThreads + threadIdx.x) * 4;
+    if (base + u * kTableThreads * 4 >= V) break;
+    const int64_t t = base + (u * kTableThreads + int(threadIdx.x)) * 4;
     F4u v;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const int32_t e = d[4 * u + q];
       v[q] = t + q == eos ? at_eos : (e >= 0 && e < S) ? lz[e] : -INFINITY;
     }
-    if (t + 4 <= V) {
+    if (whole || t + 4 <= V) {
       *reinterpret_cast<F4u*>(row + t) = v;
     } else {
 #pragma unroll
@@ -434,10 +453,15 @@ extern "C" int bpd_soft_build_lookahead(const int32_t* tok_next, int32_t S, int6
   float* b = a + S;
   const dim3 grid = dim3(unsigned((V + kTableChunk - 1) / kTableChunk), unsigned(S));
   // The counts take one pass over the table whatever k is, so they pay from
-  // the first round on (71 states, V = 151,936, k = 3: 2 x 70.3 us of
-  // table-reading rounds against 9.0 us of counts and 2 x 4.2 us of rounds).
+  // the first round on where a row is long enough to be worth two launches
+  // (clearing and counting) instead of one.  Whole build with table-reading
+  // rounds / with counts, k = 2: 71 states V = 1,000 13.5 / 16.6 us, 4,096 15.3 /
+  // 15.8, 8,192 16.7 / 16.1, 16,384 19.4 / 16.4, 151,936 92.6 / 33.8; 512 states
+  // V = 4,096 17.5 / 21.4, 8,192 22.0 / 23.7 (k = 4 40.2 / 38.8), 16,384 33.8 / 32.5,
+  // 65,536 87.2 / 79.0: for k = 2 the forms cross between 4,096 and 8,192 up to
+  // some 300 states, for larger k below.
   // A workspace of the two vectors alone takes the table-reading rounds.
-  if (S <= kCountStates && k > 1 && workspace_bytes >= bpd_soft_workspace_bytes(0, S, k)) {
+  if (S <= kCountStates && V >= kCountVocab && k > 1 && workspace_bytes >= bpd_soft_workspace_bytes(0, S, k)) {
     uint32_t* counts = reinterpret_cast<uint32_t*>(b + S);
     const int32_t n = S * S;
     soft_clear_kernel<<<(n + 255) / 256, 256, 0, st>>>(counts, n);

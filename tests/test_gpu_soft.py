@@ -47,11 +47,12 @@ def test_build_lookahead_email_serving(dev):
     assert close(la, want)
 
 
-@pytest.mark.parametrize("S,V", [(1, 1), (2, 4097), (63, 4095), (65, 1000), (512, 4097), (513, 4097)])
+@pytest.mark.parametrize("S,V", [(1, 1), (2, 4097), (63, 4095), (65, 1000), (512, 4097), (513, 4097),
+                                 (1, 6144), (2, 6143), (63, 8191), (65, 8193), (512, 6145), (513, 6145)])
 @pytest.mark.parametrize("k", [1, 2, 4])
 def test_build_lookahead_state_counts(dev, S, V, k):
-    """Rounds from (state, next) counts up to 512 states, from the table
-    above; chunk edges, entries outside the table, states without tokens."""
+    """Rounds from (state, next) counts up to 512 states and from 6,144
+    tokens on, from the table elsewhere; chunk edges, entries outside the table, states without tokens."""
     g = np.random.default_rng(S + k)
     tn = g.integers(0, S, size=(S, V)).astype(np.int32)
     tn[g.random((S, V)) < 0.9] = -1
