@@ -91,6 +91,31 @@ def random_bundle(S: int, M: int, V: int, seed: int, max_len: int = 40) -> FsaTe
                       dead=dead, offsets=t(off), symbols=t(sym.astype(np.int32)), eos_id=int(g.integers(0, V)))
 
 
+def walked_allowed(fsa: FsaTensors, states) -> np.ndarray:
+    """[rows, vocab]: the tokens that mask.hpp's walk allows from each state,
+    restated in numpy for arbitrary tables: a walk fails on a symbol id at or
+    above ``num_symbols``, on a target outside the table and on a step into
+    ``dead``, and must end on a live state; EOS where the state accepts;
+    nothing from a state below 0 or past the table."""
+    S, M, V = fsa.num_states, fsa.num_symbols, fsa.vocab_size
+    trans, live, accept, off, sym = (t.cpu().numpy().astype(np.int64) for t in
+                                     (fsa.trans, fsa.live, fsa.accept, fsa.offsets, fsa.symbols))
+    st = np.asarray(states, dtype=np.int64)
+    inside = (st >= 0) & (st < S)
+    cur = np.repeat(np.where(inside, st, -1)[:, None], V, axis=1)
+    lens = off[1:] - off[:-1]
+    for k in range(int(lens.max())):
+        t = np.nonzero(lens > k)[0]
+        c, at = sym[off[t] + k], cur[:, t]
+        nxt = trans[np.clip(at, 0, None) * M + np.minimum(c, M - 1)[None, :]]
+        ok = (at >= 0) & (c < M)[None, :] & (nxt >= 0) & (nxt < S) & (nxt != fsa.dead)
+        cur[:, t] = np.where(ok, nxt, -1)
+    allowed = (cur >= 0) & (live[np.clip(cur, 0, None)] != 0)
+    if fsa.eos_id is not None and 0 <= fsa.eos_id < V:
+        allowed[:, fsa.eos_id] = inside & (accept[np.clip(st, 0, S - 1)] != 0)
+    return allowed
+
+
 def reachable(tok_next: np.ndarray, start: int) -> list[int]:
     seen, todo = {start}, [start]
     while todo:

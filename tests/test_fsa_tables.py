@@ -13,7 +13,7 @@ import torch
 
 from bpdecode_amd import synth
 from bpdecode_amd.ops import FsaTensors
-from tests._util import TOY_PATTERNS, TOY_VOCAB, oracle_table
+from tests._util import TOY_PATTERNS, TOY_VOCAB, oracle_table, walked_allowed
 
 
 def _walk_all(f: FsaTensors) -> np.ndarray:
@@ -77,3 +77,11 @@ def test_unclosed_live_array_keeps_the_int32_walk():
     c = g.c_fsa_table()
     assert not c.trans16 and c.tok_records
     assert torch.equal(f.live, FsaTensors.build("ab|c", TOY_VOCAB, dense=False).live)
+
+
+@pytest.mark.parametrize("pattern", TOY_PATTERNS)
+def test_restated_walk_allows_what_the_oracle_table_allows(pattern):
+    f = FsaTensors.build(pattern, TOY_VOCAB, dense=False)
+    st = [*range(f.num_states), -1, -2, f.num_states]
+    got = walked_allowed(f, st)
+    assert np.array_equal(got[:f.num_states], oracle_table(f) != -1) and not got[f.num_states:].any()

@@ -17,14 +17,14 @@ import numpy as np
 import pytest
 import torch
 
-from bpdecode_amd import ops, synth
+from bpdecode_amd import _lib, ops, synth
 from bpdecode_amd.batch import ConstraintBatch, MaskCache
 from bpdecode_amd.grammar.json_schema import json_schema_to_grammar
 from bpdecode_amd.grammar.pda import CompiledGrammar
 from bpdecode_amd.grammar.regular import residual_dfa
 from bpdecode_amd.ops import FsaTensors
 from oracle import dense as OD
-from tests._util import TOY_PATTERNS, TOY_VOCAB, bits_of, oracle_table, random_bundle
+from tests._util import TOY_PATTERNS, TOY_VOCAB, bits_of, oracle_table, random_bundle, walked_allowed
 
 pytestmark = pytest.mark.gpu
 
@@ -331,30 +331,37 @@ def test_walking_commit_with_a_live_array_not_closed(dev):
 
 
 @pytest.mark.parametrize("S,M,V", [(1, 1, 1), (5, 3, 63), (71, 30, 1500), (72, 110, 513), (73, 110, 1025), (820, 45, 2049),
-                                   (900, 60, 700), (40, 253, 511), (40, 254, 511)])
-@pytest.mark.parametrize("rows", [1, 2, 3, 17, 300])
+                                   (820, 45, 512), (820, 45, 513), (900, 60, 700), (40, 253, 511), (40, 254, 511)])
+@pytest.mark.parametrize("rows", [1, 2, 3, 4, 5, 17, 300])
 def test_staged_walk_matches_the_general_walk(dev, monkeypatch, S, M, V, rows):
-    """Masks and packed bits from the table staged in LDS (blocks of 512 and
-    1024 threads, the largest staged table, one state or symbol more than
-    fits, rows past one block's 256) equal those walked through memory, for
-    arbitrary tables and states below 0 and past the table; out-of-range
-    states set the flag either way."""
+    """Masks and packed bits as the walk restated on the host gives them, for
+    arbitrary tables and states below 0 and past the table, from the table
+    staged in LDS where the dispatch takes it (blocks of 512 and 1024
+    threads, the largest staged table, rows past one block's 256) and from
+    the walk through memory (one state or symbol more than fits, few rows of
+    a large table, and every shape by BPD_FSA_TABLE); out-of-range states set
+    the flag either way."""
     _log(f"case staged walk S={S} M={M} V={V} rows={rows}")
     fd = random_bundle(S, M, V, seed=S + rows).to(dev)
     g = torch.Generator().manual_seed(rows)
     st = torch.randint(-2, S + 1, (rows,), generator=g, dtype=torch.int32).to(dev)
     lg = torch.randn(rows, V + 3, generator=g)
-    got = {}
-    for form in ("lds", "global"):
+    allowed = torch.from_numpy(walked_allowed(fd, st.cpu().numpy()))
+    packed = torch.zeros(rows, (V + 31) // 32 * 32, dtype=torch.int64)
+    packed[:, :V] = allowed
+    packed = (packed.view(rows, -1, 32) << torch.arange(32)).sum(-1)
+    words = torch.where(packed >= 2**31, packed - 2**32, packed).to(torch.int32)
+    for form in ("by the dispatch", "global"):
         monkeypatch.setenv("BPD_FSA_TABLE", form)
         err = torch.zeros(1, dtype=torch.int32, device=dev)
-        out = [ops.fsa_compute_mask(fd, st, err=err)]
+        assert torch.equal(ops.fsa_compute_mask(fd, st, err=err).cpu(), words), form
         for dt in (torch.float32, torch.bfloat16):
-            x = lg.to(dt).to(dev)
-            out.append(ops.fsa_mask_(x[:, :V], fd, st, neg_inf=-1e4, err=err))
-        got[form] = out + [err]
-    for a, b in zip(got["lds"], got["global"]):
-        assert torch.equal(a, b)
+            x = lg.to(dt)
+            got = x.to(dev)
+            ops.fsa_mask_(got[:, :V], fd, st, neg_inf=-1e4, err=err)
+            x[:, :V] = torch.where(allowed, x[:, :V], torch.tensor(-1e4, dtype=dt))
+            assert torch.equal(got.cpu(), x), (form, dt)
+        assert int(err) == (_lib.FLAG_STATE_RANGE if bool((st >= S).any()) else 0), form
 
 
 @pytest.mark.parametrize("S,V", [(1, 1), (7, 33), (5, 2048 * 32), (9, 2049 * 32 + 5), (6, 8191)])
