@@ -475,10 +475,14 @@ int launch_fsa_mask(const BpdFsaTable& t, const int32_t* states, const int64_t* 
   // Staging a large table takes a launch of a few rows about 12 us whatever
   // they are, the walk through L2 8 us for one row, 9 for two and 12-20 for
   // three (826 states); up to 16 KB the staged walk is the faster one from the
-  // first row on (71 states: 7 us against 14).
+  // first row on (71 states: 7 us against 14).  A vocabulary of one tile or
+  // less leaves the walk through L2 ahead a little longer (800 states, V = 256,
+  // the call waited for: 3 rows 20.6 us and 24.5 staged, 4 rows 21.9 and 24.7, 8
+  // rows 27.1 and 26.0; V = 600: 3 rows 28.1 and 24.8).
   const size_t lds = walk_table_bytes(t.num_states, t.num_symbols);
   const bool large = lds > 16 * 1024;
-  bool staged = walk_table_fits(t.num_states, t.num_symbols, kWalkMaxLds) && (!large || rows > 2);
+  bool staged = walk_table_fits(t.num_states, t.num_symbols, kWalkMaxLds) &&
+                (!large || rows > (t.vocab <= 512 ? 4 : 2));
   // BPD_FSA_TABLE=global forces the global-memory form (tests cover both
   // forms on small grammars with it)
   if (const char* e = std::getenv("BPD_FSA_TABLE"))
