@@ -306,25 +306,29 @@ class ConstraintBatch:
             self._ubufs[stream] = buf
         return buf
 
-    def _inline_rows(self, seq_ids: Sequence[Hashable], stream: int,
-                     limit: int = _lib.MAX_INLINE_VALUES) -> tuple | None:
-        """(slot list and queued writes as int32 bytes, slot list, queued
-        writes, upload buffer) for a launch that takes them in its arguments;
-        None where there is nothing new, or too much, or an upload was staged.
-        After the launch: :meth:`_launched_inline`."""
-        pend = self._pending
-        B, n = len(seq_ids), len(pend)
-        if self._staged is not None or B == 0 or n > _lib.MAX_FUSED_PENDING or B + 2 * n > limit:
-            return None
-        same = self._same_ids(seq_ids)
-        if same and not n:
-            return None
-        vals = self._slot_vals if same else self._lookup(seq_ids)
-        try:
-            packed = struct.pack(f"{B + 2 * n}i", *vals, *pend, *pend.values())
-        except struct.error:  # beyond 32 bits
-            return None
-        return packed, vals, n, self._upload_buffer(B, stream)
+    def _rows_of(self, seq_ids: Sequence[Hashable], stream: int,
+                 limit: int = _lib.MAX_INLINE_VALUES) -> tuple:
+        """(values, slot address, queued-writes address, count) for a device
+        launch.  Where slots or queued writes are new and at most ``limit``
+        values, they travel in the launch's arguments: ``values`` is then
+        (slot list and queued writes as int32 bytes, slot list, queued writes,
+        upload buffer), and :meth:`_launched_inline` follows the launch.
+        Else ``values`` is None and the rest as from :meth:`_slots_fused`."""
+        if self._staged is None:
+            pend = self._pending
+            n = len(pend)
+            same = self._same_ids(seq_ids)
+            if same and not n:
+                return None, self._slot_ptr, None, 0
+            B = len(seq_ids)
+            if B and n <= _lib.MAX_FUSED_PENDING and B + 2 * n <= limit:
+                vals = self._slot_vals if same else self._lookup(seq_ids)
+                try:
+                    packed = struct.pack(f"{B + 2 * n}i", *vals, *pend, *pend.values())
+                    return (packed, vals, n, self._upload_buffer(B, stream)), 0, None, 0
+                except struct.error:  # beyond 32 bits
+                    pass
+        return None, *self._slots_fused(seq_ids, True)
 
     def _launched_inline(self, seq_ids: Sequence[Hashable], rows: tuple) -> None:
         """The launch wrote the slot list to the upload buffer and the queued
@@ -426,11 +430,10 @@ class ConstraintBatch:
             B = len(seq_ids)
             ld = logits.stride(0) if B > 1 else self._V
             stream = _lib.stream_of(self.device)
-            inline = self._inline_rows(seq_ids, stream)
+            inline, slots, pend, n = self._rows_of(seq_ids, stream)
             if inline is not None:
                 self._mask_inline(seq_ids, inline, logits, code, self._V, ld, neg_inf, stream)
                 return logits
-            slots, pend, n = self._slots_fused(seq_ids, True)
             check(self._f_mask(
                 logits.data_ptr(), code, B, self._V, ld, self._bits_ptr, self._W, self._S,
                 self._pool_ptr, slots, pend, n, float(neg_inf), self._err_ptr, stream))
@@ -464,11 +467,10 @@ class ConstraintBatch:
                 and (B <= 1 or scores.stride(0) >= cols)):
             ld = scores.stride(0) if B > 1 else cols
             stream = _lib.stream_of(self.device)
-            inline = self._inline_rows(seq_ids, stream)
+            inline, slots, pend, n = self._rows_of(seq_ids, stream)
             if inline is not None:
                 self._mask_inline(seq_ids, inline, scores, code, cols, ld, neg_inf, stream)
                 return scores
-            slots, pend, n = self._slots_fused(seq_ids, True)
             check(lib().bpd_dense_apply_mask_padded(
                 scores.data_ptr(), code, B, V, cols, ld, self._bits_ptr, self._W, self._S, self._pool_ptr, slots,
                 pend, n, float(neg_inf), self._err_ptr, stream))
@@ -510,14 +512,13 @@ class ConstraintBatch:
             B = len(seq_ids)
             ld = logits.stride(0) if B > 1 else self._V
             stream = _lib.stream_of(self.device)
-            inline = self._inline_rows(seq_ids, stream) if self._V else None
+            inline, slots, pend, n = self._rows_of(seq_ids, stream, _lib.MAX_INLINE_VALUES if self._V else 0)
             if inline is not None:
                 check(lib().bpd_soft_apply_inline(
                     logits.data_ptr(), code, B, self._V, ld, la.data_ptr(), int(la.shape[0]), self._pool_ptr,
                     inline[0], inline[2], inline[3].data_ptr(), float(alpha), None, stream))
                 self._launched_inline(seq_ids, inline)
                 return logits
-            slots, pend, n = self._slots_fused(seq_ids, True)
             check(lib().bpd_soft_apply_queued(
                 logits.data_ptr(), code, B, self._V, ld, la.data_ptr(), int(la.shape[0]), self._pool_ptr, slots,
                 pend, n, float(alpha), None, stream))
@@ -548,12 +549,11 @@ class ConstraintBatch:
             rows = (logits.data_ptr(), B, V, logits.stride(0) if B > 1 else V, self._S, acc.data_ptr(),
                     live.data_ptr(), eos, self._pool_ptr)
             rest = (C.byref(sc.c_struct()), int(k), float(alpha), ws.data_ptr(), ws_bytes, self._err_ptr, stream)
-            inline = self._inline_rows(seq_ids, stream, _lib.MAX_PRIOR_INLINE_VALUES)
+            inline, slots, pend, n = self._rows_of(seq_ids, stream, _lib.MAX_PRIOR_INLINE_VALUES)
             if inline is not None:
                 check(lib().bpd_soft_prior_inline(*rows, inline[0], inline[2], inline[3].data_ptr(), *rest))
                 self._launched_inline(seq_ids, inline)
                 return logits
-            slots, pend, n = self._slots_fused(seq_ids, True)
             check(lib().bpd_soft_prior_queued(*rows, slots, pend, n, *rest))
             if n:
                 self._launched()
