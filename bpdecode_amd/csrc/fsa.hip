@@ -5,8 +5,9 @@
 // A token's first 16 symbol classes are loaded once into registers and walked
 // from every row state of the block.  Verdicts become fill stores (logits) or
 // wave64 ballots (packed bits).  Tables that fit are walked in the absorbing
-// LDS form of walk.hpp (fsa_walk_kernel), larger ones through L2
-// (fsa_mask_kernel, kFsaRows rows and kFsaThreads * kFsaTok tokens a block).
+// LDS form of walk.hpp (fsa_walk_kernel), larger ones, and few rows of a large
+// one, through L2 (fsa_mask_kernel, kFsaRows rows and kFsaThreads * kFsaTok
+// tokens a block).
 
 #include <atomic>
 #include <cstdlib>
@@ -87,9 +88,10 @@ __device__ __forceinline__ bool walk_token(const FsaView& f, const int32_t* __re
 }
 
 // Mask over the staged walk table: a thread holds one token and walks it from
-// the block's rows (row_lo + rows_per_block of them), four at a time.  Bound
+// the block's rows (at most rows_per_block), four at a time.  Bound
 // by the walk's instructions and LDS reads.  The row states are read once per
-// block, into LDS, beside the table.
+// block, into LDS, beside the table.  Bits: packed allow bits, else the rejected
+// logits (element size E) are filled.
 // 826 states, V = 151,936, packed bits: 256 rows 150 us through L2, 67 here;
 // 826 rows 412 and 163; 71 states, 256 rows: 230 and 52.
 template <int E, bool Bits>
@@ -164,8 +166,8 @@ __global__ __launch_bounds__(1024) void fsa_walk_kernel(
   }
 }
 
-// The mask for tables too large to stage (Bits = false: fill the rejected
-// logits, element size E) or packed allow bits (Bits = true).  grid (ceil(V / (kFsaThreads kFsaTok)), ceil(rows / kFsaRows)).
+// The same through L2, for tables too large to stage and few rows of a large
+// one.  grid (ceil(V / (kFsaThreads kFsaTok)), ceil(rows / kFsaRows)).
 template <int E, bool Bits>
 __global__ __launch_bounds__(kFsaThreads) void fsa_mask_kernel(
     FsaView f, const int32_t* __restrict__ states, const int64_t* __restrict__ slots, int64_t rows,
@@ -173,8 +175,6 @@ __global__ __launch_bounds__(kFsaThreads) void fsa_mask_kernel(
     int64_t words, int32_t* __restrict__ err) {
   __shared__ int32_t rs[kFsaRows];
   const int tid = threadIdx.x;
-  const int32_t* tr = f.trans;
-  const uint8_t* lv = f.live;
   const int64_t r0 = int64_t(blockIdx.y) * kFsaRows;
   if (tid < kFsaRows) {
     const int64_t r = r0 + tid;
@@ -208,7 +208,7 @@ __global__ __launch_bounds__(kFsaThreads) void fsa_mask_kernel(
       const int32_t s = rs[r];
       if (s == kNoRow) break;  // rows past the batch come last
       bool ok = false;
-      if (on && s >= 0) ok = is_eos ? f.accept[s] != 0 : walk_token(f, tr, lv, s, pk, rest, len);
+      if (on && s >= 0) ok = is_eos ? f.accept[s] != 0 : walk_token(f, f.trans, f.live, s, pk, rest, len);
       if (Bits) {
         const uint64_t m = __ballot(ok);
         const int64_t tw = t - (tid & 63);  // first token of the wave, a multiple of 64

@@ -684,7 +684,8 @@ extern "C" int bpd_host_soft_apply(void* logits, int dtype, int64_t rows, int64_
 // whose tok_next columns are equal behave identically in every state, so a
 // round needs only logsumexp_{t in class} logpi_b(t) per class.  Classes are
 // built once per grammar on the host (bpd_host_soft_classes).  One call is
-// three kernels:
+// three launches, or two where the rounds launch also writes the output
+// (kFusedChunks):
 //   stats:  grid (G, rows), block g streams tokens [8192 g, 8192 (g+1)) of
 //           its row with their class ids and leaves the chunk's logsumexp
 //           and, per class, (max, sum exp(x - max)) of its members: a
@@ -693,7 +694,8 @@ extern "C" int bpd_host_soft_apply(void* logits, int dtype, int64_t rows, int64_
 //           pieces of <= 256 members instead (one wave per piece).
 //   rounds: one block per row merges the partials, runs the k-1 rounds with
 //           logZ, the class sums and the (class, next) pairs in LDS, and
-//           writes zcls[b, c] = logZ(next of class c from s_b) and lse[b].
+//           writes zcls[b, c] = logZ(next of class c from s_b) and lse[b]
+//           (or several blocks a row, each going on to its chunks' output).
 //   out:    one streaming pass, out = x - lse + alpha * zcls[b, class(t)].
 // The kernel boundaries order the cross-block hand-offs; an in-kernel
 // last-block hand-off needs agent-scope release fences, which write back the
@@ -794,7 +796,7 @@ constexpr int64_t kWideChunk = kPriorThreads * 4 * kWideLoads;  // 8192 tokens p
 
 struct PriorPlan {
   bool class_stats;  // class-atomic stats (else pieces)
-  bool wide;         // wave-shift stats over 16384-token chunks (class_stats only)
+  bool wide;         // wave-shift stats over kWideChunk tokens a block (class_stats only)
   int G;             // chunk blocks per row
   int Gp;            // piece blocks per row (pieces path)
 };
@@ -1059,7 +1061,7 @@ __global__ __launch_bounds__(kPriorThreads) void prior_stats_members_kernel(
 }
 
 // Wave-shift statistics, grid (G, rows): block g takes tokens
-// [16384 g, 16384 (g + 1)) of its row, 64 per thread (16 float4 groups in
+// [8192 g, 8192 (g + 1)) of its row, 32 per thread (eight float4 groups in
 // flight, each group coalesced), and the uint16 class map of the same tokens
 // (shared by every row, so it stays in L2).  Each wave shifts by its own
 // maximum M_w: the chunk logsumexp and, per class, sum exp(x - M_w) over the
