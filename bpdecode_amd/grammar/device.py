@@ -479,7 +479,9 @@ class CFGConstraintBatch:
     order.  From the first call on another stream (a capture among them) or
     the first look at the pool's tensors on, each reset is a launch of its
     own on the stream current at the call, so that replayed graphs and other
-    streams see it wherever the caller has ordered them after the call."""
+    streams see it wherever the caller has ordered them after the call.  That
+    first call on another stream waits on the host, once, for the resets that
+    it finds queued on the default stream."""
 
     def __init__(self, g: PdaTensors, capacity: int, device=None) -> None:
         self.g = g if device is None else g.to(device)
@@ -508,8 +510,8 @@ class CFGConstraintBatch:
 
     def _flush(self) -> None:
         """Enqueue the queued resets ahead of a use of the pool on the
-        current stream.  Off the default stream they go out there once more,
-        waited for, and nothing is queued any more."""
+        current stream.  Off the default stream they go out on the default
+        one, waited for on the host, and nothing is queued any more."""
         if not self._queueing:
             return
         direct = _lib.stream_of(self.device) != 0
